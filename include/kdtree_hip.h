@@ -164,8 +164,8 @@ int kd_counters(kd_ctx *ctx, int64_t out[5]);
 
 /* Launch-shape knobs of the kernels (no counterpart in the reference):
  * "leaf_predicated" 0/1 -- compute whole leaf batches with predication
- * instead of branching per body; "fp64_batched_walk" 0/1 -- run the FP64
- * path on the batched walk of the mixed paths; "lazy_dimension" 0/1 (default
+ * instead of branching per body; "fp64_batched_walk" 0/1 -- accepted
+ * and read back, but without effect: FP64 has one walk; "lazy_dimension" 0/1 (default
  * 1) -- let the build skip the sort and the device-wide partitions of a
  * dimension that the previous full build found could not be split at those
  * levels (a thin system's third dimension); every build checks that this

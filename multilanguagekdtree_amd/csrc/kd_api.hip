@@ -72,7 +72,8 @@ struct kd_ctx {
   int ev_used = 0;  // steps recorded in the current chunk
   double t_ms[3] = {0.0, 0.0, 0.0};
   int64_t t_steps = 0;
-  int traverse_variant = 0;  // bit 1: predicated leaf batches; bit 2: FP64 on the batched walk
+  int traverse_variant = 0;  // WALK_* bits
+  bool fp64_batched = false;  // a knob that changes nothing any more: FP64 has one walk
   // systems: one for a plain context, many for a batch
   Forest forest;
   std::vector<SysDesc> hsys;
@@ -427,14 +428,25 @@ int kd_get_params(const kd_ctx *c, kd_params *out) {
 
 int64_t kd_size(const kd_ctx *c) { return c ? c->n : -1; }
 
+// The upload check's result: *bad for a non-finite value, and the walk's
+// variant bit for masses of ordinary size.
+static int check_upload(kd_ctx *c, const StateDev &s, uint32_t n, int *bad) {
+  int flags[2] = {0, 0};
+  HIP_TRY(hipMemsetAsync(c->bad, 0, sizeof(flags), c->stream));
+  HIP_TRY(launch_sanitize(s, n, c->bad, c->stream));
+  HIP_TRY(hipMemcpyAsync(flags, c->bad, sizeof(flags), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  *bad = flags[0];
+  c->traverse_variant &= ~WALK_MASSES_IN_RANGE;
+  if (!flags[1]) c->traverse_variant |= WALK_MASSES_IN_RANGE;
+  return KD_OK;
+}
+
 static int upload_common(kd_ctx *c, int64_t n) {
   StateDev &s = c->st[c->cur];
   HIP_TRY(launch_iota(s.oid, (uint32_t)n, c->stream));
-  HIP_TRY(hipMemsetAsync(c->bad, 0, sizeof(int), c->stream));
-  HIP_TRY(launch_sanitize(s, (uint32_t)n, c->bad, c->stream));
-  int bad = 0;
-  HIP_TRY(hipMemcpyAsync(&bad, c->bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  int bad = 0, rc = check_upload(c, s, (uint32_t)n, &bad);
+  if (rc) return rc;
   if (bad) {
     c->has_state = false;
     return fail(KD_ERR_NONFINITE, "non-finite position, velocity or mass in upload");
@@ -702,11 +714,12 @@ int kd_counters(kd_ctx *c, int64_t out[5]) {
 int kd_set_tuning(kd_ctx *c, const char *key, int64_t value) {
   if (!c || !key) return fail(KD_ERR_ARG, "NULL argument");
   if (strcmp(key, "leaf_predicated") == 0) {
-    c->traverse_variant = value ? (c->traverse_variant | 2) : (c->traverse_variant & ~2);
+    c->traverse_variant &= ~WALK_PREDICATED;
+    if (value) c->traverse_variant |= WALK_PREDICATED;
     return KD_OK;
   }
   if (strcmp(key, "fp64_batched_walk") == 0) {
-    c->traverse_variant = value ? (c->traverse_variant | 4) : (c->traverse_variant & ~4);
+    c->fp64_batched = value != 0;
     return KD_OK;
   }
   if (strcmp(key, "lazy_dimension") == 0) {
@@ -729,9 +742,9 @@ int kd_set_tuning(kd_ctx *c, const char *key, int64_t value) {
 int kd_get_tuning(kd_ctx *c, const char *key, int64_t *value) {
   if (!c || !key || !value) return fail(KD_ERR_ARG, "NULL argument");
   if (strcmp(key, "leaf_predicated") == 0) {
-    *value = (c->traverse_variant & 2) ? 1 : 0;
+    *value = (c->traverse_variant & WALK_PREDICATED) ? 1 : 0;
   } else if (strcmp(key, "fp64_batched_walk") == 0) {
-    *value = (c->traverse_variant & 4) ? 1 : 0;
+    *value = c->fp64_batched ? 1 : 0;
   } else if (strcmp(key, "lazy_dimension") == 0) {
     *value = c->lazy_allowed && c->lazy_on ? 1 : 0;
   } else if (strcmp(key, "lazy_next") == 0) {
@@ -1209,7 +1222,8 @@ static void batch_from_padded(const kd_batch *b, const std::vector<double> &src,
 
 static int batch_traverse(kd_batch *b, const KickDrift *kick = nullptr) {
   kd_ctx *c = b->c;
-  return launch_traverse_forest(c->params.precision, c->params.count_interactions != 0, b->ws,
+  return launch_traverse_forest(c->params.precision, c->params.count_interactions != 0,
+                                c->traverse_variant, b->ws,
                                 c->tree, c->pos64, c->pos32, c->forest, b->tasks, b->ntasks,
                                 b->queue, b->cus, c->params.theta, c->params.leaf_size,
                                 c->acc[0], c->acc[1], c->acc[2], c->counters, c->stream,
@@ -1433,11 +1447,10 @@ extern "C" int kd_batch_upload(kd_batch *b, const double *x, const double *y, co
                            c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));  // stage is reused
   }
-  HIP_TRY(hipMemsetAsync(c->bad, 0, sizeof(int), c->stream));
-  HIP_TRY(launch_sanitize(s, total, c->bad, c->stream));
-  int bad = 0;
-  HIP_TRY(hipMemcpyAsync(&bad, c->bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  const int variant = c->traverse_variant;
+  int bad = 0, rc = check_upload(c, s, total, &bad);
+  if (rc) return rc;
+  if (c->traverse_variant != variant) drop_graphs(b);  // the captured walks embed it
   if (bad) {
     c->has_state = false;
     return fail(KD_ERR_NONFINITE, "non-finite position, velocity or mass in upload");

@@ -41,6 +41,22 @@ constexpr uint32_t FIX_SHORT = 16;
 
 constexpr int MAX_LEAF = 32;
 
+// The depth at which an FP64 walk's sum is cut into parts (kd_traverse.hip),
+// from the bodies and levels of the tree alone, so that a system's result does
+// not depend on what runs beside it; 0: one part.  A workgroup of 2^(d - 2)
+// wavefronts then walks 64 bodies.  It pays while the wavefronts alone leave
+// most of the GPU's 8192 slots empty: ring, FP64 walk in us, depth 0 / 4 / 5 /
+// 6: 155 / 69 / 57 / 61 at 1,000 bodies, 334 / 153 / 130 / 102 at 10,000, 406 /
+// 252 / 205 / 250 at 30,000, 541 / 448 / 605 / 1193 at 100,000, 584 / 636 / 884
+// / 1821 at 150,000 (every wavefront visits the nodes above the parts, and the
+// slowest part holds up the rest).  Every node above the depth is internal:
+// with L levels every node down to depth L - 3 is.
+__host__ __device__ inline int walk_depth(uint32_t n, int levels) {
+  int d = n <= 16384 ? 6 : n <= 65536 ? 5 : n <= 131072 ? 4 : 0;
+  if (d > levels - 2) d = levels - 2;
+  return d < 3 ? 0 : d;
+}
+
 // The block index a kernel should treat as its own so that each of the 8
 // XCDs runs one contiguous range of the grid: the dispatcher hands blocks to
 // the XCDs round robin (block b to XCD b mod 8), and neighbouring bodies
@@ -289,6 +305,9 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
                         const TreeDev &t, BuildBufs &b, double4 *pos64, float4 *pos32,
                         double theta, hipStream_t s, bool range_ready = false, int lazy = 3,
                         bool report = false, bool mid = true);
+// Bits of a walk's variant: predicated leaf batches; every body's mass lies
+// within the bounds of the FP64 walk's shorter arithmetic.
+constexpr int WALK_PREDICATED = 2, WALK_MASSES_IN_RANGE = 8;
 hipError_t launch_traverse(int precision, bool count, int variant, const TreeDev &t,
                            const double4 *pos64, const float4 *pos32, uint32_t n,
                            double theta, int leaf, double *ax, double *ay, double *az,
@@ -319,7 +338,7 @@ struct WalkShape {
   int threads = 256;
   int waves_per_cu = 0;
 };
-hipError_t launch_traverse_forest(int precision, bool count, const WalkShape &ws,
+hipError_t launch_traverse_forest(int precision, bool count, int variant, const WalkShape &ws,
                                   const TreeDev &t, const double4 *pos64, const float4 *pos32,
                                   const Forest &f, const uint2 *tasks, uint32_t ntasks,
                                   uint32_t *queue, int cus, double theta, int leaf, double *ax,

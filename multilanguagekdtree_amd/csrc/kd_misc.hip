@@ -69,7 +69,9 @@ __global__ void k_iota(uint32_t *__restrict__ v, uint32_t n) {
   if (i < n) v[i] = i;
 }
 
-// Device-side upload check: -0.0 -> +0.0 for positions, flags non-finite.
+// Device-side upload check: -0.0 -> +0.0 for positions; flags a non-finite
+// value in bad[0] and a mass whose size is neither 0 nor within
+// 2^-400..2^400 in bad[1] (the FP64 walk's shorter arithmetic needs that).
 __global__ void k_sanitize(double *x, double *y, double *z, const double *vx,
                            const double *vy, const double *vz, const double *m,
                            uint32_t n, int *bad) {
@@ -81,7 +83,9 @@ __global__ void k_sanitize(double *x, double *y, double *z, const double *vx,
   if (c == 0.0) z[i] = 0.0;
   if (!(isfinite(a) && isfinite(b) && isfinite(c) && isfinite(vx[i]) && isfinite(vy[i]) &&
         isfinite(vz[i]) && isfinite(m[i])))
-    *bad = 1;
+    bad[0] = 1;
+  const double w = fabs(m[i]);
+  if (w != 0.0 && !(w >= 0x1p-400 && w <= 0x1p400)) bad[1] = 1;
 }
 
 // FP64 direct sum (calc_pp_accel form, Sequential/RustVersion/src/

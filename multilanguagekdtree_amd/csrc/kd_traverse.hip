@@ -56,14 +56,6 @@ __device__ __forceinline__ Rec load_rec_at(const Rec *__restrict__ nodes_m1, uin
   return r;
 }
 
-// Advance past the subtree of h; returns 0 when the root is finished.
-__device__ __forceinline__ uint32_t heap_next(uint32_t h, int &depth) {
-  int t = __builtin_ctz(~h);
-  h >>= t;
-  depth -= t;
-  return h == 0 ? 0 : h + 1;
-}
-
 // ---------------------------------------------------------------------------
 // arithmetic policies
 // ---------------------------------------------------------------------------
@@ -72,6 +64,8 @@ struct F64 {
   static constexpr int CHUNK = 4;  // leaf bodies per batch of scalar loads
   static constexpr bool SELF_BY_INDEX = true;  // self pair dropped by a select
   static constexpr bool COMPACT = false;  // leaves are never split across lanes
+  static constexpr bool PARTS = true;     // the sum may be formed in parts (walk_parts)
+  static constexpr bool CHECKED = false;  // terms hold for every operand
   using Rec = NodeRec64;
   using Body = double4;
   using Self = double4;
@@ -116,6 +110,87 @@ struct F64 {
   }
   __device__ static void fold(Acc &) {}
   __device__ static double result(const Acc &a, int i) { return a.s[i]; }
+  __device__ static void clear(Acc &a) { a.s[0] = a.s[1] = a.s[2] = 0.0; }
+};
+
+// The F64 policy with shorter sequences for the square root and the quotient
+// of a term, for operands well inside the exponent range.  The compiler's own
+// cover every operand (scaling, special values): a pair term takes 47 vector
+// instructions with them and 33 so; the 1 M ring FP64 walk takes 2.41 ms
+// against 3.21.
+// Both results are still the correctly rounded ones, so terms and sums are
+// F64's bit for bit (4e9 random operands over 2^-300..2^300 against sqrt()
+// and the division: no bit differs).  From y0 = v_rsq_f64(d2), relative error
+// below 2^-24.1, the third-order iteration y = y0 (1 + e/2 + 3 e^2 / 8),
+// e = 1 - d2 y0^2, leaves y within about an ulp of d2^-1/2; the square root
+// g = d2 y and the quotient q = -m y^3 then each take one correction by their
+// exact residual (d2 - g^2, -m - q den: one fma each), after which the error
+// before the last rounding is some 2^-100.
+// Operands: m is 0 or within 2^-452..2^431 (the upload checks the bodies'
+// masses), d2 below 2^300 (the root's size bounds every distance) and above
+// 2^-300, which the walk only knows afterwards: the accumulator keeps the
+// smallest d2 (its high word, which orders positive doubles) and a wavefront
+// that met a smaller one walks again with F64.
+struct F64Short : F64 {
+  static constexpr bool CHECKED = true;
+  using Exact = F64;
+  struct Acc {
+    double s[3] = {0.0, 0.0, 0.0};
+    uint32_t least = 0x7ff00000u;  // high word of the smallest d2
+  };
+  static constexpr uint32_t LEAST = (1023u - 300u) << 20;
+  __device__ static bool in_range(const Acc &a) { return a.least > LEAST; }
+  // tree-wide: the root is internal and its extent small enough (every
+  // extent, and so every coordinate difference, is at most the root's size)
+  __device__ static bool usable(const NodeRec64 &root, uint32_t leaf) {
+    return root.count > leaf && root.size2 < 0x1p297;
+  }
+  // y = d2^-1/2 and g = sqrt(d2)
+  __device__ static void root_of(double d2, double &y, double &g) {
+#pragma clang fp contract(off)
+    const double y0 = __builtin_amdgcn_rsq(d2);
+    const double e = __builtin_fma(-(d2 * y0), y0, 1.0);
+    y = __builtin_fma(y0, __builtin_fma(e, 0.375, 0.5) * e, y0);
+    const double g1 = d2 * y;
+    g = __builtin_fma(__builtin_fma(-g1, g1, d2), 0.5 * y, g1);
+  }
+  // -m / den, where y^3 is 1 / den but for a few ulp
+  __device__ static double quotient(double m, double den, double y) {
+#pragma clang fp contract(off)
+    const double z = y * y * y;
+    const double q = -m * z;
+    return __builtin_fma(__builtin_fma(-den, q, -m), z, q);
+  }
+  __device__ static void m2p_sel(Acc &a, const Rec &r, const Diff &f, bool take) {
+#pragma clang fp contract(off)
+    if (!take) return;
+    double y, g;
+    root_of(f.d2, y, g);
+    const double magi = quotient(r.m, f.d2 * g, y);
+    a.least = min(a.least, (uint32_t)__double2hiint(f.d2));
+    a.s[0] += f.dx * magi;
+    a.s[1] += f.dy * magi;
+    a.s[2] += f.dz * magi;
+  }
+  __device__ static void p2p(Acc &a, const Self &p, const Body &q, bool self_pair) {
+#pragma clang fp contract(off)
+    const double dx = p.x - q.x;
+    const double dy = p.y - q.y;
+    const double dz = p.z - q.z;
+    double d2 = dx * dx + dy * dy + dz * dz;
+    // the self pair: its differences are 0, so any finite factor adds 0
+    d2 = __hiloint2double(self_pair ? 0x3ff00000 : __double2hiint(d2), __double2loint(d2));
+    double y, g;
+    root_of(d2, y, g);
+    const double magi = quotient(q.w, g * g * g, y);
+    a.least = min(a.least, (uint32_t)__double2hiint(d2));
+    a.s[0] += magi * dx;
+    a.s[1] += magi * dy;
+    a.s[2] += magi * dz;
+  }
+  __device__ static void fold(Acc &) {}
+  __device__ static double result(const Acc &a, int i) { return a.s[i]; }
+  __device__ static void clear(Acc &a) { a.s[0] = a.s[1] = a.s[2] = 0.0; }
 };
 
 // Blocked Kahan summation with the compensation carried in the partial:
@@ -146,6 +221,8 @@ struct F32 {
   static constexpr int CHUNK = 8;
   static constexpr bool SELF_BY_INDEX = false;
   static constexpr bool COMPACT = true;
+  static constexpr bool PARTS = false;
+  static constexpr bool CHECKED = false;
   using Rec = NodeRec32;
   using Body = float4;
   using Self = float4;  // x, y, z, e2
@@ -187,6 +264,7 @@ struct F32 {
     a.p[2] += g * dz;
   }
   __device__ static void fold(Acc &a) { kahan_fold(a); }
+  __device__ static void clear(Acc &a) { a = Acc(); }
   __device__ static double result(const Acc &a, int i) {
     return (double)a.s[i] + (double)a.p[i];
   }
@@ -196,6 +274,8 @@ struct D64 {
   static constexpr int CHUNK = 4;
   static constexpr bool SELF_BY_INDEX = true;
   static constexpr bool COMPACT = false;
+  static constexpr bool PARTS = false;
+  static constexpr bool CHECKED = false;
   using Rec = NodeRecD;
   using Body = double4;
   using Self = double4;
@@ -234,6 +314,7 @@ struct D64 {
     a.p[2] += g * dz;
   }
   __device__ static void fold(Acc &a) { kahan_fold(a); }
+  __device__ static void clear(Acc &a) { a = Acc(); }
   __device__ static double result(const Acc &a, int i) {
     return (double)a.s[i] + (double)a.p[i];
   }
@@ -251,6 +332,7 @@ struct WalkArgs {
   double *__restrict__ az;
   Counters cnt;
   KickDrift kd{};  // used by the walks that apply the kick-drift themselves
+  bool masses_in_range = false;  // every body's mass is within CHECKED policies' bounds
 };
 
 // A body's state, loaded when its wavefront starts so that the loads are
@@ -483,13 +565,215 @@ __device__ __forceinline__ float4 *walk_slots() {
   }
 }
 
+// Counts of one lane (COUNT kernels): node tests, accepted nodes, pairs, and
+// the wavefront's node and leaf visits.
+struct LaneCounts {
+  unsigned long long nt = 0, na = 0, np = 0, wv = 0, wl = 0;
+};
+
+// One internal node r at position h: the lanes in actm test it, the far-field
+// term is added when `mine` (wave-uniform), E takes the new acceptance level,
+// and the next position is returned.
+template <class P, bool COUNT>
+__device__ __forceinline__ uint32_t visit_inner(const typename P::Rec &r, uint32_t h, int lz,
+                                                uint64_t actm, bool active, bool mine,
+                                                double theta2, const typename P::Self &p, int &E,
+                                                typename P::Acc &acc, LaneCounts &c) {
+  constexpr int RSL = sizeof(typename P::Rec) == 32 ? 5 : 6;
+  // the test runs on every lane (no divergence); only active lanes use it
+  typename P::Diff f;
+  const bool ok = P::test(p, r, theta2, f);
+  // lane masks combined on the scalar unit, then used as lane conditions
+  const uint64_t okm = __builtin_amdgcn_ballot_w64(ok);
+  // the lanes that open the node, and from the same SCC the next node:
+  // the first child if any lane opens, else the skip (the compiler
+  // would test om against 0 a second time)
+  uint64_t om;
+  uint32_t hn;
+  asm("s_andn2_b64 %0, %2, %3\n\ts_cselect_b32 %1, %4, %5"
+      : "=&s"(om), "=s"(hn)
+      : "s"(actm), "s"(okm), "s"(2 * h), "s"(r.skip)
+      : "scc");
+  const bool take = __builtin_amdgcn_inverse_ballot_w64(actm & okm);
+  const bool open = __builtin_amdgcn_inverse_ballot_w64(om);
+  // wave-uniform: the far-field term is evaluated only when a lane takes it
+  if (mine && (actm & okm)) P::m2p_sel(acc, r, f, take);
+  // D = open ? unbounded : min(D, level): a taking lane had D >= level,
+  // a lane outside D < level
+  E = open ? -RSL : max(E, lz);
+  if (COUNT) {
+    c.nt += active ? 1 : 0;
+    c.na += take ? 1 : 0;
+  }
+  return hn;
+}
+
+// The walk from position h until it leaves for position `stop`.
+template <class P, bool COUNT, bool PRED>
+__device__ __forceinline__ void walk_nodes(const typename P::Rec *__restrict__ nodes_m1,
+                                           const typename P::Body *__restrict__ bodies,
+                                           uint32_t leaf, double theta2, uint32_t me,
+                                           const typename P::Self &p, int &E,
+                                           typename P::Acc &acc, float4 *__restrict__ slot,
+                                           uint32_t h, uint32_t stop, LaneCounts &c) {
+  do {
+    const typename P::Rec r = load_rec_at(nodes_m1, uni(h));
+    const int lz = __builtin_clz(h);  // 32 - level(h) - log2(RS)
+    // the lanes taking part, as a scalar mask (kept on the scalar unit) and
+    // as the lane's own condition
+    const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
+    const bool active = __builtin_amdgcn_inverse_ballot_w64(actm);
+    if (COUNT) ++c.wv;
+    if (r.count <= leaf) {
+      if (COUNT) ++c.wl;
+      bool split = false;
+      if constexpr (P::COMPACT) {
+        const uint32_t k = mask_count(actm);
+        if (k <= SPLIT_MAX) {
+          leaf_split<P, COUNT>(acc, p, bodies + r.start, r.count, r.start, me, actm, active, slot,
+                               c.np);
+          split = true;
+        }
+      }
+      if (!split)
+        for (uint32_t b = 0; b < r.count; b += P::CHUNK)
+          leaf_batch<P, P::CHUNK, COUNT, PRED>(acc, p, bodies + (r.start + b),
+                                               min((uint32_t)P::CHUNK, r.count - b),
+                                               r.start + b, me, active, c.np);
+      P::fold(acc);  // on every lane (a fold is valid at any point): no exec-mask change
+      h = r.skip;
+    } else {
+      h = visit_inner<P, COUNT>(r, h, lz, actm, active, true, theta2, p, E, acc, c);
+    }
+  } while (h != stop);
+}
+
+// The walk in parts: the nodes above level d are visited first to last, and
+// every node met at level d (lzd: the leading zeros of its position) begins
+// part i = 0, 1, ... of the sum.  own(i) (wave-uniform): whether this
+// wavefront adds part i; a part it does not own is passed over, which leaves
+// the lanes taking part in what follows as they would be (a subtree leaves a
+// lane that took part in it with D >= d).  begin(i): called before part i > 0
+// begins.  The far-field terms above level d belong to the part at hand.
+// Returns the number of parts (at least 1).  Every node above level d is
+// internal (walk_depth).
+template <class P, bool COUNT, bool PRED, class Own, class Begin>
+__device__ __forceinline__ uint32_t walk_parts(const typename P::Rec *__restrict__ nodes_m1,
+                                               const typename P::Body *__restrict__ bodies,
+                                               uint32_t leaf, double theta2, uint32_t me,
+                                               const typename P::Self &p, int &E,
+                                               typename P::Acc &acc, float4 *__restrict__ slot,
+                                               int lzd, LaneCounts &c, Own own, Begin begin) {
+  constexpr uint32_t RS = sizeof(typename P::Rec);
+  uint32_t h = RS, parts = 0;
+  bool mine = own(0);
+  do {
+    const int lz = __builtin_clz(h);
+    if (lz == lzd) {
+      if (parts > 0) begin(parts);
+      mine = own(parts);
+      ++parts;
+      // the node after this subtree (position 0: none)
+      uint32_t x = h / RS;
+      x >>= __builtin_ctz(~x);
+      const uint32_t next = x == 0 ? 0 : (x + 1) * RS;
+      if (mine) walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, h, next, c);
+      h = next;
+    } else {
+      const typename P::Rec r = load_rec_at(nodes_m1, uni(h));
+      const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
+      const bool active = __builtin_amdgcn_inverse_ballot_w64(actm);
+      if (COUNT) ++c.wv;
+      h = visit_inner<P, COUNT>(r, h, lz, actm, active, mine, theta2, p, E, acc, c);
+    }
+  } while (h != 0);
+  return parts > 0 ? parts : 1;
+}
+
+// What a wavefront does with its bodies' accelerations (x, y, z): the
+// kick-drift, or the acceleration arrays.
+template <bool KD, class A>
+__device__ __forceinline__ void walk_finish(const A &a, const BodyState &bs, uint32_t wbase,
+                                            uint32_t me, bool valid, double x, double y,
+                                            double z) {
+  if (KD) {
+    uint64_t lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0ull, 0ull, 0ull};
+    if (valid) kick_drift_one(a.kd, me, bs, x, y, z, lo, hi);
+    if (a.kd.wave_range)
+      wave_range_store(a.kd.wave_range + 6 * (size_t)(wbase >> 6), lo, hi, me & 63);
+  } else if (valid) {
+    a.ax[me] = x;
+    a.ay[me] = y;
+    a.az[me] = z;
+  }
+}
+
+// The position is the byte offset of the current record, off = h RS (the
+// records' skip pointers are stored the same way), so no multiply is
+// needed per visit.  The lane's acceptance level D (root 1; unbounded
+// while it keeps opening) is kept as E = 32 - D - log2(RS) and compared
+// with clz(off) = 32 - level(h) - log2(RS), which saves forming the level:
+// E = 32 - log2(RS) keeps a lane out of every node, E = -log2(RS) lets it
+// into every node.
+template <class P>
+__device__ __forceinline__ int walk_start(bool valid) {
+  constexpr uint32_t RS = sizeof(typename P::Rec);
+  static_assert(RS == 32 || RS == 64, "records of 32 or 64 bytes");
+  constexpr int RSL = RS == 32 ? 5 : 6;
+  return valid ? -RSL : 32 - RSL;
+}
+// clz(off) of the nodes at depth d (root 0)
+template <class P>
+__device__ __forceinline__ int depth_lz(int d) {
+  return 31 - (sizeof(typename P::Rec) == 32 ? 5 : 6) - d;
+}
+
+// The sum of a wavefront's bodies: in one part, or (PARTS) in the parts of
+// depth d, added in order (the sum that k_walk_split forms with several
+// wavefronts).  Returns whether it holds (CHECKED policies: every lane's
+// operands were in range).
+template <class P, bool COUNT, bool PRED, bool PARTS>
+__device__ __forceinline__ bool walk_sum(const typename P::Rec *__restrict__ nodes_m1,
+                                         const typename P::Body *__restrict__ bodies,
+                                         uint32_t leaf, double theta2, uint32_t me, bool valid,
+                                         const typename P::Self &p, float4 *__restrict__ slot,
+                                         int d, LaneCounts &c, double sum[3]) {
+  typename P::Acc acc;
+  int E = walk_start<P>(valid);
+  if constexpr (PARTS) {
+    sum[0] = sum[1] = sum[2] = 0.0;
+    walk_parts<P, COUNT, PRED>(
+        nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, depth_lz<P>(d), c,
+        [](uint32_t) { return true; },
+        [&](uint32_t) {
+          P::fold(acc);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) sum[q] += P::result(acc, q);
+          P::clear(acc);
+        });
+    P::fold(acc);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sum[q] += P::result(acc, q);
+  } else {
+    walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot,
+                               (uint32_t)sizeof(typename P::Rec), 0u, c);
+    P::fold(acc);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sum[q] = P::result(acc, q);
+  }
+  if constexpr (P::CHECKED)
+    return __builtin_amdgcn_ballot_w64(!P::in_range(acc)) == 0;
+  else
+    return true;
+}
+
 // The walk of one wavefront: bodies [wbase, wbase + 64) of a tree whose
 // records start one before nodes_m1[1] and whose bodies start at bodies[0].
-template <class P, bool COUNT, bool PRED, bool KD = false>
+template <class P, bool COUNT, bool PRED, bool KD = false, bool PARTS = false>
 __device__ __forceinline__ void walk_wave(const typename P::Rec *__restrict__ nodes_m1,
                                           const typename P::Body *__restrict__ bodies,
                                           const WalkArgs<P> &a, uint32_t wbase_in,
-                                          float4 *__restrict__ slot) {
+                                          float4 *__restrict__ slot, int d = 0) {
   // wave-uniform by construction; readfirstlane lets the compiler know it
   const uint32_t wbase = uni(wbase_in);
   const uint32_t lane = threadIdx.x & 63;
@@ -498,97 +782,31 @@ __device__ __forceinline__ void walk_wave(const typename P::Rec *__restrict__ no
   const typename P::Self p = P::self(bodies[valid ? me : wbase]);
   BodyState bs{};
   if (KD) bs = body_state(a.kd, valid ? me : wbase);
-  typename P::Acc acc;
-  // The position is the byte offset of the current record, off = h RS (the
-  // records' skip pointers are stored the same way), so no multiply is
-  // needed per visit.  The lane's acceptance level D (root 1; unbounded
-  // while it keeps opening) is kept as F = 32 - D - log2(RS) and compared
-  // with clz(off) = 32 - level(h) - log2(RS), which saves forming the level:
-  // F = 32 - log2(RS) keeps a lane out of every node, F = -log2(RS) lets it
-  // into every node.
-  constexpr uint32_t RS = sizeof(typename P::Rec);
-  static_assert(RS == 32 || RS == 64, "records of 32 or 64 bytes");
-  constexpr int RSL = RS == 32 ? 5 : 6;
-  int E = valid ? -RSL : 32 - RSL;
-  unsigned long long nt = 0, na = 0, np = 0, wv = 0, wl = 0;
-  uint32_t h = RS;  // the root, heap index 1
-  do {
-    const typename P::Rec r = load_rec_at(nodes_m1, uni(h));
-    const int lz = __builtin_clz(h);  // 32 - level(h) - log2(RS)
-    // the lanes taking part, as a scalar mask (kept on the scalar unit) and
-    // as the lane's own condition
-    const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
-    const bool active = __builtin_amdgcn_inverse_ballot_w64(actm);
-    if (COUNT) ++wv;
-    if (r.count <= a.leaf) {
-      if (COUNT) ++wl;
-      bool split = false;
-      if constexpr (P::COMPACT) {
-        const uint32_t k = mask_count(actm);
-        if (k <= SPLIT_MAX) {
-          leaf_split<P, COUNT>(acc, p, bodies + r.start, r.count, r.start, me, actm, active, slot,
-                               np);
-          split = true;
-        }
-      }
-      if (!split)
-        for (uint32_t b = 0; b < r.count; b += P::CHUNK)
-          leaf_batch<P, P::CHUNK, COUNT, PRED>(acc, p, bodies + (r.start + b),
-                                               min((uint32_t)P::CHUNK, r.count - b),
-                                               r.start + b, me, active, np);
-      P::fold(acc);  // on every lane (a fold is valid at any point): no exec-mask change
-      h = r.skip;
-    } else {
-      // the test runs on every lane (no divergence); only active lanes use it
-      typename P::Diff f;
-      const bool ok = P::test(p, r, a.theta2, f);
-      // lane masks combined on the scalar unit, then used as lane conditions
-      const uint64_t okm = __builtin_amdgcn_ballot_w64(ok);
-      // the lanes that open the node, and from the same SCC the next node:
-      // the first child if any lane opens, else the skip (the compiler
-      // would test om against 0 a second time)
-      uint64_t om;
-      uint32_t hn;
-      asm("s_andn2_b64 %0, %2, %3\n\ts_cselect_b32 %1, %4, %5"
-          : "=&s"(om), "=s"(hn)
-          : "s"(actm), "s"(okm), "s"(2 * h), "s"(r.skip)
-          : "scc");
-      const bool take = __builtin_amdgcn_inverse_ballot_w64(actm & okm);
-      const bool open = __builtin_amdgcn_inverse_ballot_w64(om);
-      // wave-uniform: the far-field term is evaluated only when a lane takes it
-      if (actm & okm) P::m2p_sel(acc, r, f, take);
-      // D = open ? unbounded : min(D, level): a taking lane had D >= level,
-      // a lane outside D < level
-      E = open ? -RSL : max(E, lz);
-      if (COUNT) {
-        nt += active ? 1 : 0;
-        na += take ? 1 : 0;
-      }
-      h = hn;
-    }
-  } while (h != 0);
-  P::fold(acc);
-  if (KD) {
-    uint64_t lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0ull, 0ull, 0ull};
-    if (valid)
-      kick_drift_one(a.kd, me, bs, P::result(acc, 0), P::result(acc, 1), P::result(acc, 2), lo,
-                     hi);
-    if (a.kd.wave_range) wave_range_store(a.kd.wave_range + 6 * (size_t)(wbase >> 6), lo, hi, lane);
-  } else if (valid) {
-    a.ax[me] = P::result(acc, 0);
-    a.ay[me] = P::result(acc, 1);
-    a.az[me] = P::result(acc, 2);
+  LaneCounts c;
+  double sum[3];
+  if constexpr (P::CHECKED) {
+    bool done = a.masses_in_range && P::usable(nodes_m1[1], a.leaf);
+    if (done)
+      done = walk_sum<P, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p,
+                                             slot, d, c, sum);
+    if (!done)
+      walk_sum<typename P::Exact, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me,
+                                                      valid, p, slot, d, c, sum);
+  } else {
+    walk_sum<P, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p, slot, d, c,
+                                    sum);
   }
+  walk_finish<KD>(a, bs, wbase, me, valid, sum[0], sum[1], sum[2]);
   if (COUNT) {
-    nt = wave_sum_u64(nt);
-    na = wave_sum_u64(na);
-    np = wave_sum_u64(np);
+    c.nt = wave_sum_u64(c.nt);
+    c.na = wave_sum_u64(c.na);
+    c.np = wave_sum_u64(c.np);
     if (lane == 0) {
-      atomicAdd(&a.cnt.c[0], nt);
-      atomicAdd(&a.cnt.c[1], na);
-      atomicAdd(&a.cnt.c[2], np);
-      atomicAdd(&a.cnt.c[3], wv);
-      atomicAdd(&a.cnt.c[4], wl);
+      atomicAdd(&a.cnt.c[0], c.nt);
+      atomicAdd(&a.cnt.c[1], c.na);
+      atomicAdd(&a.cnt.c[2], c.np);
+      atomicAdd(&a.cnt.c[3], c.wv);
+      atomicAdd(&a.cnt.c[4], c.wl);
     }
   }
 }
@@ -619,13 +837,81 @@ __device__ __forceinline__ uint32_t walk_block() {
   const uint32_t t = nb - full, q = t / 8u, r = t % 8u, it = (blockIdx.x - full) / 8u;
   return full + x * q + (x < r ? x : r) + it;
 }
-template <class P, bool COUNT, bool PRED, bool KD = false>
+template <class P, bool COUNT, bool PRED, bool KD = false, bool PARTS = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KD_WALK_WAVES))) void k_walk(
     const typename P::Rec *__restrict__ nodes_m1, const typename P::Body *__restrict__ bodies,
-    WalkArgs<P> a) {
+    WalkArgs<P> a, int d) {
   const uint32_t wbase = (walk_block() * blockDim.x + threadIdx.x) & ~63u;
   if (wbase >= a.n) return;
-  walk_wave<P, COUNT, PRED, KD>(nodes_m1, bodies, a, wbase, walk_slots<P, 256>());
+  walk_wave<P, COUNT, PRED, KD, PARTS>(nodes_m1, bodies, a, wbase, walk_slots<P, 256>(), d);
+}
+
+// The walk of one wavefront's 64 bodies by the S wavefronts of a workgroup,
+// for systems whose wavefronts alone leave the GPU waiting on serial chains
+// of node visits (walk_depth: where, and what it measured).  Part i of the sum (walk_parts, depth log2(S) + 2: at most
+// 4 parts a wavefront) is wavefront i mod S's; every wavefront visits the
+// nodes above the parts, and the parts are added in order at the end, so the
+// result is walk_wave's with PARTS, bit for bit.
+template <class P, bool KD, int S>
+__global__ __launch_bounds__(64 * S) void k_walk_split(
+    const typename P::Rec *__restrict__ nodes_m1, const typename P::Body *__restrict__ bodies,
+    WalkArgs<P> a) {
+  static_assert(P::PARTS && !P::COMPACT, "a policy whose sums may be cut into parts");
+  constexpr int D = S == 2 ? 3 : S == 4 ? 4 : S == 8 ? 5 : 6;
+  static_assert((1 << D) == 4 * S, "four parts a wavefront");
+  __shared__ double tot[3][64];
+  const uint32_t wbase = xcd_block() * 64u;
+  const uint32_t w = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint32_t me = wbase + lane;
+  const bool valid = me < a.n;
+  const typename P::Self p = P::self(bodies[valid ? me : wbase]);
+  BodyState bs{};
+  if (KD && w == 0) bs = body_state(a.kd, valid ? me : wbase);
+  double part[4][3];
+  uint32_t parts = 0;
+  auto own = [&](uint32_t i) { return (i & (S - 1u)) == w; };
+  auto walk = [&](auto policy) {
+    using Q = decltype(policy);
+    typename Q::Acc acc;
+    LaneCounts c;
+    int E = walk_start<Q>(valid);
+    uint32_t k = 0;  // parts of this wavefront that are done
+    auto keep = [&]() {
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q)
+        if (q == k)  // wave-uniform
+          for (int x = 0; x < 3; ++x) part[q][x] = Q::result(acc, x);
+      Q::clear(acc);
+      ++k;
+    };
+    parts = walk_parts<Q, false, false>(nodes_m1, bodies, a.leaf, a.theta2, me, p, E, acc, nullptr,
+                                        depth_lz<Q>(D), c, own, [&](uint32_t i) {
+                                          if (own(i - 1)) keep();
+                                        });
+    if (own(parts - 1)) keep();
+    if constexpr (Q::CHECKED)
+      return !__syncthreads_or(!Q::in_range(acc));
+    else
+      return true;
+  };
+  if constexpr (P::CHECKED) {
+    bool done = a.masses_in_range && P::usable(nodes_m1[1], a.leaf);
+    if (done) done = walk(P());
+    if (!done) walk(typename P::Exact());
+  } else {
+    walk(P());
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q) {
+    for (uint32_t v = 0; v < S && q * S + v < parts; ++v) {
+      if (v == w)
+        for (int x = 0; x < 3; ++x)
+          tot[x][lane] = (q + v == 0 ? 0.0 : tot[x][lane]) + part[q][x];
+      __syncthreads();
+    }
+  }
+  if (w == 0)
+    walk_finish<KD>(a, bs, wbase, me, valid, tot[0][lane], tot[1][lane], tot[2][lane]);
 }
 
 // Forest walk: a task is one wavefront of one system (x: system, y: first
@@ -674,8 +960,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
       st.vz += S.body_off;
       if (b.kd.wave_range) b.kd.wave_range += 6 * ((size_t)t - (task.y >> 6));
     }
-    walk_wave<P, COUNT, false, KD>(nodes + S.node_off - 1, bodies + S.body_off, b, task.y,
-                                   walk_slots<P, NT>());
+    const int d = P::PARTS ? walk_depth(S.n, (int)S.levels) : 0;
+    walk_wave<P, COUNT, false, KD, P::PARTS>(nodes + S.node_off - 1, bodies + S.body_off, b, task.y,
+                                         walk_slots<P, NT>(), d);
     if (!PERSIST) return;
   }
 }
@@ -684,173 +971,85 @@ __global__ void k_queue_reset(uint32_t *queue) {
   if (threadIdx.x < 8) queue[threadIdx.x] = 0u;
 }
 
-// The plain FP64 path keeps a simpler loop: it is VALU-bound (FP64 sqrt and
-// divide dominate), and this form issues fewer vector instructions per visit
-// than the batched walk above: leaf bodies are read one at a time under the
-// active-lane mask and the self pair is skipped by branch.
-template <bool COUNT, bool KD = false>
-__global__ __launch_bounds__(256) void k_walk_f64(const NodeRec64 *__restrict__ nodes,
-                                                  const double4 *__restrict__ pos,
-                                                  WalkArgs<F64> a) {
-#pragma clang fp contract(off)
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wbase = (xcd_block() * blockDim.x + threadIdx.x) & ~63u;
-  if (wbase >= a.n) return;
-  const uint32_t me = wbase + lane;
-  const bool valid = me < a.n;
-  const double4 p = valid ? pos[me] : make_double4(0.0, 0.0, 0.0, 0.0);
-  BodyState bs{};
-  if (KD) bs = body_state(a.kd, valid ? me : wbase);
-  double sx = 0.0, sy = 0.0, sz = 0.0;
-  int D = valid ? 0x7fffffff : -1;
-  unsigned long long nt = 0, na = 0, np = 0, wv = 0, wl = 0;
-  uint32_t h = 1;
-  int depth = 0;
-  while (h != 0) {
-    const NodeRec64 r = nodes[uni(h) - 1];
-    const bool active = depth <= D;
-    if (COUNT) ++wv;
-    if (r.count <= a.leaf) {
-      if (COUNT) ++wl;
-      if (active) {
-        for (uint32_t jj = 0; jj < r.count; ++jj) {
-          const uint32_t j = r.start + jj;
-          const double4 q = pos[j];
-          if (j != me) {
-            double dx = p.x - q.x;
-            double dy = p.y - q.y;
-            double dz = p.z - q.z;
-            double dp2 = dx * dx + dy * dy + dz * dz;
-            double dist = sqrt(dp2);
-            double magi = -q.w / (dist * dist * dist);
-            sx += magi * dx;
-            sy += magi * dy;
-            sz += magi * dz;
-            if (COUNT) ++np;
-          }
-        }
-      }
-      h = heap_next(h, depth);
-      continue;
-    }
-    bool open = false;
-    if (active) {
-      double dx = p.x - r.cx;
-      double dy = p.y - r.cy;
-      double dz = p.z - r.cz;
-      double d2 = dx * dx + dy * dy + dz * dz;
-      if (COUNT) ++nt;
-      if (r.size2 < a.theta2 * d2) {
-        double dist = sqrt(d2);
-        double magi = -r.m / (d2 * dist);
-        sx += dx * magi;
-        sy += dy * magi;
-        sz += dz * magi;
-        D = depth;
-        if (COUNT) ++na;
-      } else {
-        D = 0x7fffffff;
-        open = true;
-      }
-    }
-    if (__any(open)) {
-      h = 2 * h;
-      ++depth;
-    } else {
-      h = heap_next(h, depth);
-    }
-  }
-  if (KD) {
-    uint64_t lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0ull, 0ull, 0ull};
-    if (valid) kick_drift_one(a.kd, me, bs, sx, sy, sz, lo, hi);
-    if (a.kd.wave_range) wave_range_store(a.kd.wave_range + 6 * (size_t)(wbase >> 6), lo, hi, lane);
-  } else if (valid) {
-    a.ax[me] = sx;
-    a.ay[me] = sy;
-    a.az[me] = sz;
-  }
-  if (COUNT) {
-    nt = wave_sum_u64(nt);
-    na = wave_sum_u64(na);
-    np = wave_sum_u64(np);
-    if (lane == 0) {
-      atomicAdd(&a.cnt.c[0], nt);
-      atomicAdd(&a.cnt.c[1], na);
-      atomicAdd(&a.cnt.c[2], np);
-      atomicAdd(&a.cnt.c[3], wv);
-      atomicAdd(&a.cnt.c[4], wl);
-    }
+template <class P, bool KD, bool PARTS>
+static void launch_whole(const WalkArgs<P> &a, bool count, bool pred, int d, hipStream_t s) {
+  const unsigned blocks = (a.n + 255) / 256;
+  if (count) {
+    if (pred)
+      k_walk<P, true, true, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+    else
+      k_walk<P, true, false, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+  } else {
+    if (pred)
+      k_walk<P, false, true, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+    else
+      k_walk<P, false, false, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
   }
 }
 
-template <class P>
-static void launch_policy(const WalkArgs<P> &a, bool count, int variant, hipStream_t s,
-                          bool kick = false) {
-  const unsigned blocks = (a.n + 255) / 256;
-  const bool pred = (variant & 2) != 0;
-  if (kick) {
-    if (pred)
-      k_walk<P, false, true, true><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+// FP64: the short sequences unless interactions are counted or leaf batches
+// predicated (padding bodies of a batch need a select of their own).
+template <bool KD>
+static void launch_f64(const WalkArgs<F64Short> &a, bool count, bool pred, hipStream_t s) {
+  const int d = walk_depth(a.n, make_shape(a.n, (int)a.leaf).levels);
+  const unsigned groups = (a.n + 63) / 64;
+  if (count || pred) {
+    const WalkArgs<F64> e{a.nodes, a.bodies, a.n, a.leaf, a.theta2, a.ax, a.ay, a.az, a.cnt, a.kd};
+    if (d == 0)
+      launch_whole<F64, KD, false>(e, count, pred, d, s);
     else
-      k_walk<P, false, false, true><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
-  } else if (count) {
-    if (pred)
-      k_walk<P, true, true><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
-    else
-      k_walk<P, true, false><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+      launch_whole<F64, KD, true>(e, count, pred, d, s);
+  } else if (d == 0) {
+    k_walk<F64Short, false, false, KD, false>
+        <<<(a.n + 255) / 256, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+  } else if (d == 3) {
+    k_walk_split<F64Short, KD, 2><<<groups, 128, 0, s>>>(a.nodes - 1, a.bodies, a);
+  } else if (d == 4) {
+    k_walk_split<F64Short, KD, 4><<<groups, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+  } else if (d == 5) {
+    k_walk_split<F64Short, KD, 8><<<groups, 512, 0, s>>>(a.nodes - 1, a.bodies, a);
   } else {
-    if (pred)
-      k_walk<P, false, true><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
-    else
-      k_walk<P, false, false><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+    k_walk_split<F64Short, KD, 16><<<groups, 1024, 0, s>>>(a.nodes - 1, a.bodies, a);
   }
+}
+
+template <bool KD>
+static hipError_t launch_walk(int precision, bool count, int variant, const TreeDev &t,
+                              const double4 *pos64, const float4 *pos32, uint32_t n, double theta,
+                              int leaf, double *ax, double *ay, double *az, Counters c,
+                              const KickDrift &kd, hipStream_t s) {
+  const double theta2 = theta * theta;
+  const bool pred = (variant & WALK_PREDICATED) != 0;
+  const bool masses = (variant & WALK_MASSES_IN_RANGE) != 0;
+  if (precision == 0) {
+    launch_f64<KD>(WalkArgs<F64Short>{t.rec64, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd,
+                                      masses},
+                   count, pred, s);
+  } else if (precision == 1) {
+    launch_whole<F32, KD, false>(
+        WalkArgs<F32>{t.rec32, pos32, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred,
+        0, s);
+  } else {
+    launch_whole<D64, KD, false>(
+        WalkArgs<D64>{t.recd, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred, 0,
+        s);
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_traverse(int precision, bool count, int variant, const TreeDev &t,
                            const double4 *pos64, const float4 *pos32, uint32_t n,
                            double theta, int leaf, double *ax, double *ay, double *az,
                            unsigned long long *counters, hipStream_t s) {
-  Counters c{counters};
-  const double theta2 = theta * theta;
-  if (precision == 0) {
-    WalkArgs<F64> a{t.rec64, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c};
-    const unsigned blocks = (n + 255) / 256;
-    if (variant & 4) {
-      launch_policy(a, count, variant, s);
-    } else if (count) {
-      k_walk_f64<true><<<blocks, 256, 0, s>>>(a.nodes, a.bodies, a);
-    } else {
-      k_walk_f64<false><<<blocks, 256, 0, s>>>(a.nodes, a.bodies, a);
-    }
-  } else if (precision == 1) {
-    WalkArgs<F32> a{t.rec32, pos32, n, (uint32_t)leaf, theta2, ax, ay, az, c};
-    launch_policy(a, count, variant, s);
-  } else {
-    WalkArgs<D64> a{t.recd, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c};
-    launch_policy(a, count, variant, s);
-  }
-  return hipGetLastError();
+  return launch_walk<false>(precision, count, variant, t, pos64, pos32, n, theta, leaf, ax, ay, az,
+                            Counters{counters}, KickDrift{}, s);
 }
 
 hipError_t launch_traverse_kick(int precision, int variant, const TreeDev &t, const double4 *pos64,
                                 const float4 *pos32, uint32_t n, double theta, int leaf,
                                 const KickDrift &kd, hipStream_t s) {
-  Counters c{nullptr};
-  const double theta2 = theta * theta;
-  if (precision == 0) {
-    WalkArgs<F64> a{t.rec64, pos64, n, (uint32_t)leaf, theta2, nullptr, nullptr, nullptr, c, kd};
-    if (variant & 4)
-      launch_policy(a, false, variant, s, true);
-    else
-      k_walk_f64<false, true><<<(n + 255) / 256, 256, 0, s>>>(a.nodes, a.bodies, a);
-  } else if (precision == 1) {
-    WalkArgs<F32> a{t.rec32, pos32, n, (uint32_t)leaf, theta2, nullptr, nullptr, nullptr, c, kd};
-    launch_policy(a, false, variant, s, true);
-  } else {
-    WalkArgs<D64> a{t.recd, pos64, n, (uint32_t)leaf, theta2, nullptr, nullptr, nullptr, c, kd};
-    launch_policy(a, false, variant, s, true);
-  }
-  return hipGetLastError();
+  return launch_walk<true>(precision, false, variant, t, pos64, pos32, n, theta, leaf, nullptr,
+                           nullptr, nullptr, Counters{nullptr}, kd, s);
 }
 
 template <class P, bool COUNT, bool PERSIST, bool KD>
@@ -908,7 +1107,7 @@ static void launch_forest(const WalkArgs<P> &a, bool count, bool kick, const Wal
   }
 }
 
-hipError_t launch_traverse_forest(int precision, bool count, const WalkShape &ws,
+hipError_t launch_traverse_forest(int precision, bool count, int variant, const WalkShape &ws,
                                   const TreeDev &t, const double4 *pos64, const float4 *pos32,
                                   const Forest &f, const uint2 *tasks, uint32_t ntasks,
                                   uint32_t *queue, int cus, double theta, int leaf, double *ax,
@@ -921,8 +1120,14 @@ hipError_t launch_traverse_forest(int precision, bool count, const WalkShape &ws
   const KickDrift kd = kick ? *kick : KickDrift{};
   const bool k = kick != nullptr;
   if (precision == 0) {
-    WalkArgs<F64> a{t.rec64, pos64, 0, (uint32_t)leaf, theta2, ax, ay, az, c, kd};
-    launch_forest(a, count && !k, k, ws, f.sys, tasks, ntasks, queue, cus, s);
+    if (count && !k) {
+      WalkArgs<F64> a{t.rec64, pos64, 0, (uint32_t)leaf, theta2, ax, ay, az, c, kd};
+      launch_forest(a, true, k, ws, f.sys, tasks, ntasks, queue, cus, s);
+    } else {
+      WalkArgs<F64Short> a{t.rec64, pos64, 0, (uint32_t)leaf, theta2, ax, ay, az, c, kd,
+                           (variant & WALK_MASSES_IN_RANGE) != 0};
+      launch_forest(a, false, k, ws, f.sys, tasks, ntasks, queue, cus, s);
+    }
   } else if (precision == 1) {
     WalkArgs<F32> a{t.rec32, pos32, 0, (uint32_t)leaf, theta2, ax, ay, az, c, kd};
     launch_forest(a, count && !k, k, ws, f.sys, tasks, ntasks, queue, cus, s);

@@ -1,0 +1,61 @@
+"""The FP64 walk's forms: sums cut into parts that the wavefronts of a workgroup
+share (sizes around each change of depth, and leaf sizes whose trees are too
+shallow for it), and the shorter square root and quotient of a term.  The
+predicated walk runs the compiler's own square root and division with one
+wavefront for 64 bodies and forms the same sums, so every form must equal it
+bit for bit."""
+import numpy as np
+import pytest
+
+from helpers import accel_errors
+from multilanguagekdtree_amd import kdtree as K
+
+pytestmark = pytest.mark.gpu
+
+
+def accel(b, predicated, leaf=7, theta=0.3):
+    with K.Simulation(len(b["x"]), theta=theta, leaf_size=leaf) as s:
+        s.set_tuning("leaf_predicated", predicated)
+        s.upload(b)
+        return s.accel()
+
+
+def cloud(n, seed):
+    rng = np.random.default_rng(seed)
+    p = rng.normal(size=(3, n))
+    return dict(zip(K.FIELDS, (*p, *np.zeros((3, n)), rng.uniform(0.5, 2.0, n) / n)))
+
+
+@pytest.mark.parametrize("n,leaf", [
+    (5, 7), (8, 7), (29, 7), (60, 7), (113, 7), (500, 32), (700, 32), (4097, 2), (16384, 7),
+    (16385, 7), (65536, 8), (65537, 7), (131072, 7), (131073, 7)])
+def test_forms_agree(n, leaf):
+    for b in (K.ring(n, seed=n), cloud(n, n)):
+        np.testing.assert_array_equal(accel(b, 0, leaf), accel(b, 1, leaf))
+
+
+@pytest.mark.parametrize("n", [200, 3000, 70000, 140000])
+@pytest.mark.parametrize("px,pm", [(-200, 0), (-140, 0), (140, 0), (200, 0), (0, -450), (0, 430)])
+def test_scaled_systems(n, px, pm):
+    # positions times 2^px and masses times 2^pm: every operation of the
+    # reference arithmetic scales exactly, also where the short sequences do
+    # not hold and the walk falls back
+    b = cloud(n, 7)
+    s = {f: v * 2.0 ** (px if f in "xyz" else pm if f == "m" else 0) for f, v in b.items()}
+    a = accel(s, 0)
+    np.testing.assert_array_equal(a, accel(s, 1))
+    np.testing.assert_array_equal(a * 2.0 ** (px - pm) * 2.0 ** px, accel(b, 0))
+
+
+def test_uneven_masses_and_close_pairs(orc):
+    # a massless body, masses over 600 orders of two, and pairs 2^-160 apart
+    # near the origin (their d2 is below the short sequences' range)
+    b = cloud(2000, 11)
+    for m in (1.0, 2.0 ** -300, 2.0 ** -420):
+        b["m"][3], b["m"][4] = 0.0, m
+        for f in "xyz":
+            b[f][10], b[f][11] = 0.0, 2.0 ** -160
+        a = accel(b, 0)
+        np.testing.assert_array_equal(a, accel(b, 1))
+        ref, absref, _ = orc.accel(b, want_abs=True)
+        assert accel_errors(a, ref, absref)[1].max() <= 1e-12
