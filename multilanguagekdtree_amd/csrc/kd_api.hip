@@ -539,8 +539,11 @@ static int build_impl(kd_ctx *c, bool range_ready = false) {
                        c->pos64, c->pos32, c->params.theta, c->stream, range_ready, lazy,
                        report, mid));
   if (report) {
-    HIP_TRY(hipEventSynchronize(c->b.ev_viol));
-    uint32_t unsafe = *c->b.viol_host;
+    // a system of one segment has no device-wide split, so any dimension may
+    // be skipped there
+    const bool whole = one_segment(c->forest);
+    if (!whole) HIP_TRY(hipEventSynchronize(c->b.ev_viol));
+    uint32_t unsafe = whole ? 0u : *c->b.viol_host;
     bool full = lazy == 3;  // a full build reports every dimension
     if (lazy < 3) {
       ++c->lazy_builds;
@@ -671,11 +674,12 @@ int kd_step(kd_ctx *c, int64_t steps) {
       // the walk advances each body as it finishes it; the next build's
       // range comes from the wavefronts' ranges
       const uint32_t n = (uint32_t)c->n;
-      const KickDrift kd{c->st[c->cur], c->params.dt, c->bad, more ? c->wave_range : nullptr};
+      const bool range = more && !one_segment(c->forest);
+      const KickDrift kd{c->st[c->cur], c->params.dt, c->bad, range ? c->wave_range : nullptr};
       HIP_TRY(launch_traverse_kick(c->params.precision, c->traverse_variant, c->tree, c->pos64,
                                    c->pos32, n, c->params.theta, c->params.leaf_size, kd,
                                    c->stream));
-      if (more) HIP_TRY(launch_range_from_waves(c->wave_range, (n + 63) / 64, c->b.range, c->stream));
+      if (range) HIP_TRY(launch_range_from_waves(c->wave_range, (n + 63) / 64, c->b.range, c->stream));
       if ((rc = record(c, 2))) return rc;
     } else {
       if ((rc = traverse_impl(c))) return rc;

@@ -62,66 +62,29 @@ __device__ __forceinline__ T block_excl_sum(T v, T *sh, T &total) {
   return before + x - v;
 }
 
-// Segmented inclusive-scan element: value and "segment starts here" flag.
-struct SegV {
-  uint64_t v;
-  uint32_t h;
-};
-__device__ __forceinline__ SegV seg_combine(SegV a, SegV b) {
-  SegV r;
-  r.v = b.h ? b.v : a.v + b.v;
-  r.h = a.h | b.h;
-  return r;
+// v from the lane that the DPP control CTRL names, 0 where that lane is
+// outside the row or the row is not in ROWS.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
 }
 
-// Exclusive segmented carry for each thread: combination of all earlier
-// threads' aggregates.  shv/shh need NT/64 entries.  One barrier: every
-// wavefront combines the per-wavefront totals itself, so the caller must
-// pass a barrier between two calls before shv/shh are written again.
-template <int NT>
-__device__ __forceinline__ SegV block_seg_carry(SegV agg, uint64_t *shv,
-                                                uint32_t *shh) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  SegV x = agg;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    SegV y;
-    y.v = __shfl_up(x.v, o, 64);
-    y.h = __shfl_up(x.h, o, 64);
-    if (lane >= o) x = seg_combine(y, x);
-  }
-  if (lane == 63) {
-    shv[w] = x.v;
-    shh[w] = x.h;
-  }
-  __syncthreads();
-  SegV t;
-  t.v = lane < NT / 64 ? shv[lane] : 0;
-  t.h = lane < NT / 64 ? shh[lane] : 0;
-#pragma unroll
-  for (int o = 1; o < NT / 64; o <<= 1) {
-    SegV y;
-    y.v = __shfl_up(t.v, o, 64);
-    y.h = __shfl_up(t.h, o, 64);
-    if (lane >= o) t = seg_combine(y, t);
-  }
-  // exclusive within the wave
-  SegV prev;
-  prev.v = __shfl_up(x.v, 1, 64);
-  prev.h = __shfl_up(x.h, 1, 64);
-  if (lane == 0) {
-    prev.v = 0;
-    prev.h = 0;
-  }
-  // the combination of the totals of wavefronts 0 .. w-1
-  SegV carry;
-  carry.v = __shfl(t.v, w > 0 ? w - 1 : 0, 64);
-  carry.h = __shfl(t.h, w > 0 ? w - 1 : 0, 64);
-  if (w == 0) {
-    carry.v = 0;
-    carry.h = 0;
-  }
-  return lane == 0 ? carry : seg_combine(carry, prev);
+// Inclusive sums over lanes 0..31 and, apart from them, 32..63 (FULL: over
+// all 64): four shifts within rows of 16, then the row totals broadcast.
+template <bool FULL>
+__device__ __forceinline__ uint32_t lane_scan(uint32_t v) {
+  v += dpp_u32<0x111, 0xF>(v);
+  v += dpp_u32<0x112, 0xF>(v);
+  v += dpp_u32<0x114, 0xF>(v);
+  v += dpp_u32<0x118, 0xF>(v);
+  v += dpp_u32<0x142, 0xA>(v);
+  if (FULL) v += dpp_u32<0x143, 0xC>(v);
+  return v;
+}
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 // ---------------------------------------------------------------------------
@@ -1003,6 +966,7 @@ struct SubArgs {
   int leaf;
   double theta2;
   int lazy;  // a dimension whose list the device-wide levels did not keep (3: none)
+  bool sort_all;  // no list was sorted (one segment is the whole system)
   // (system, segment) of every workgroup in a forest (nullptr: a single
   // system, workgroup k takes segment k)
   const uint2 *tasks;
@@ -1090,66 +1054,26 @@ __device__ void write_internal_rec(const TreeDev &t, uint32_t h, uint32_t start,
   if (t.recs & REC_D) t.recd[h] = dd;
 }
 
-// Body range [s, s + cnt) of node c at depth lam below a segment of n0
-// bodies (every split at floor(count / 2)); false if an ancestor is a leaf,
-// so that the node does not exist.
-__device__ __forceinline__ bool sub_node(uint32_t c, int lam, uint32_t n0, int leaf,
-                                         uint32_t &s, uint32_t &cnt) {
-  s = 0;
-  cnt = n0;
-  for (int b = lam - 1; b >= 0; --b) {
-    if (cnt <= (uint32_t)leaf) return false;
-    const uint32_t half = cnt >> 1;
-    if ((c >> b) & 1u) {
-      s += half;
-      cnt -= half;
-    } else {
-      cnt = half;
-    }
-  }
-  return true;
-}
-
-// The lazy dimension's order inside a segment: the order of the presorted
-// lists, (coordinate, working id).  Sorted by a bitonic network in the form
-// whose comparators all sort upward: the merge of two sorted blocks into one
-// of `size` positions first compares mirror positions x and x ^ (size - 1),
-// then x and x + stride for strides size/4 .. 1.  Positions at or past n0
-// act as +inf: they are never read or written, and every comparator whose
-// upper position is one of them is skipped.  A pass runs up to LZ_G
-// consecutive stages of one merge in registers, 2^g positions a thread, so
-// the values cross LDS once per LZ_G stages, not once per stage.  At 10 M
-// ring bodies (segments of ~1220) a build takes 3.07 ms with 2 stages a pass
-// on 32-bit values (3.09 ms with 3 stages, half the threads idle; 3.17 ms on
-// 64-bit keys; 3.45 ms for one LDS round trip per stage over every position
-// of the padded block).
-#ifndef KD_LZ_G
-#define KD_LZ_G 2
-#endif
-constexpr int LZ_G = KD_LZ_G;
-
-// The values the network sorts, in two forms.  Packed: a 21-bit fixed-point
-// key of the coordinate over the segment's own range and the 11-bit local
-// index in one word (4 bytes a value, one compare a comparator); bodies whose
-// keys collide are put in exact order afterwards.  Wide: the 64-bit ordered
-// key of the coordinate and the local index, equal keys by working id (exact
-// by itself; the form a segment falls back to when keys collide in runs
-// longer than LZ_RUN).
-struct LzPacked {
-  uint32_t *k;
-  using V = uint32_t;
-  __device__ V get(uint32_t p) const { return k[p]; }
-  __device__ void put(uint32_t p, V v) const { k[p] = v; }
-  __device__ void order(V &a, V &b) const {
-    const V lo = a < b ? a : b, hi = a < b ? b : a;
-    a = lo;
-    b = hi;
-  }
-};
+// A dimension's order inside a segment, for a dimension whose list the
+// device-wide steps did not keep.  The order of equal coordinates is free:
+// a split takes the key at the median, and a run of equal keys there is put
+// in order of the original indices first.  The values sorted are a 21-bit
+// fixed-point key of the coordinate over the segment's own range with the
+// 11-bit local index below it, by a radix sort in LDS; bodies whose keys
+// collide are put in exact order afterwards, and a segment with a run of more
+// than LZ_RUN colliding keys of unequal coordinates falls back to a bitonic
+// network on 64-bit ordered keys.
+//
+// The network is in the form whose comparators all sort upward: the merge of
+// two sorted blocks into one of `size` positions first compares mirror
+// positions x and x ^ (size - 1), then x and x + stride for strides size/4 ..
+// 1.  Positions at or past n0 act as +inf: they are never read or written,
+// and every comparator whose upper position is one of them is skipped.  A
+// pass runs 2 consecutive stages of one merge in registers, 4 positions a
+// thread.
 struct LzWide {
   uint64_t *k;
   uint16_t *l;
-  const uint32_t *ids;
   struct V {
     uint64_t k;
     uint16_t l;
@@ -1160,7 +1084,7 @@ struct LzWide {
     l[p] = v.l;
   }
   __device__ void order(V &a, V &b) const {
-    if (a.k > b.k || (a.k == b.k && ids[a.l] > ids[b.l])) {
+    if (a.k > b.k) {
       const V t = a;
       a = b;
       b = t;
@@ -1169,6 +1093,77 @@ struct LzWide {
 };
 constexpr uint32_t LZ_KEY_BITS = 21, LZ_KEY_MAX = (1u << LZ_KEY_BITS) - 1, LZ_RUN = 16;
 static_assert(SUB_MAX <= (1 << (32 - LZ_KEY_BITS)), "local indices fill the packed low bits");
+
+// Radix sort of the n0 <= SUB_MAX words in v by their top 21 bits, three
+// stable passes of 7 bits (v -> w -> v -> w: the result is in w).  Each
+// wavefront ranks a run of consecutive positions, 64 at a time: the lanes
+// with the same digit are found by one ballot per digit bit, and the lane
+// that comes first of them advances the wavefront's count of the digit.  The
+// counts of all wavefronts are then scanned in (digit, wavefront) order.
+// cnt: NT / 64 x 128 words, sh: NT / 64 words.  At segments of ~1220 bodies
+// this takes 5 us against 15 for the bitonic network it replaced (33 passes).
+template <int NT>
+__device__ void lz_radix(uint32_t *v, uint32_t *w, uint32_t n0, uint32_t *cnt, uint32_t *sh,
+                         int tid) {
+  constexpr int NW = NT / 64, IT = SUB_MAX / NT, DB = 7, ND = 1 << DB;
+  static_assert(NW * ND == 2 * NT, "two counters a thread");
+  const uint32_t wv = tid >> 6, lane = tid & 63;
+  const uint32_t per = (n0 + NT - 1) / NT;  // rounds of 64 positions a wavefront
+  const uint32_t base = wv * per * 64;
+  for (int pass = 0; pass < 3; ++pass) {
+    const int shift = 32 - LZ_KEY_BITS + DB * pass;
+    uint32_t *my = cnt + wv * ND;
+    for (uint32_t q = lane; q < (uint32_t)ND; q += 64) my[q] = 0;
+    wave_sync();
+    uint32_t x[IT], r[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t i = base + it * 64 + lane;
+      x[it] = (uint32_t)it < per && i < n0 ? v[i] : 0u;
+    }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      if ((uint32_t)it >= per || base + it * 64 >= n0) break;  // wave-uniform
+      const bool use = base + it * 64 + lane < n0;
+      const uint32_t d = (x[it] >> shift) & (ND - 1);
+      uint64_t same = __builtin_amdgcn_ballot_w64(use);
+#pragma unroll
+      for (int b = 0; b < DB; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(bit);
+        same &= bit ? m : ~m;
+      }
+      const uint32_t below = lanes_below(same);
+      const uint32_t before = use ? my[d] : 0u;
+      r[it] = before + below;
+      wave_sync();
+      if (use && below == 0) my[d] = before + (uint32_t)__builtin_popcountll(same);
+      wave_sync();
+    }
+    __syncthreads();
+    // exclusive scan over (digit, wavefront): thread t holds digit t / 4,
+    // wavefronts 2 (t mod 4) and the next
+    const uint32_t dg = tid / (NW / 2), w0 = 2 * (tid % (NW / 2));
+    const uint32_t c0 = cnt[w0 * ND + dg], c1 = cnt[(w0 + 1) * ND + dg];
+    const uint32_t inc = lane_scan<true>(c0 + c1);
+    if (lane == 63) sh[wv] = inc;
+    __syncthreads();
+    uint32_t off = inc - c0 - c1;
+    for (uint32_t q = 0; q < (uint32_t)NW; ++q) off += q < wv ? sh[q] : 0u;
+    cnt[w0 * ND + dg] = off;
+    cnt[(w0 + 1) * ND + dg] = off + c0;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      if ((uint32_t)it >= per || base + it * 64 + lane >= n0) break;
+      w[my[(x[it] >> shift) & (ND - 1)] + r[it]] = x[it];
+    }
+    __syncthreads();
+    uint32_t *t = v;
+    v = w;
+    w = t;
+  }
+}
 
 // Merges of sizes 2 .. 2^G over runs of 2^G consecutive positions.
 template <int NT, int G, class Pol>
@@ -1255,7 +1250,7 @@ __device__ __forceinline__ void lz_pass(const Pol &pol, uint32_t n0, uint32_t M,
 template <int NT, int G, class Pol>
 __device__ void lz_sort(const Pol &pol, uint32_t n0, int tid) {
   static_assert((SUB_MAX >> G) <= NT, "one set of positions a thread");
-  static_assert(G >= 2 && G <= 3, "passes of 2 or 3 stages");
+  static_assert(G == 2, "passes of 2 stages");
   constexpr int WL = 6 + G;
   int lm = G;
   while ((1u << lm) < n0) ++lm;
@@ -1279,21 +1274,20 @@ __device__ void lz_sort(const Pol &pol, uint32_t n0, int tid) {
       } else {
         // the last ls + 1 < G stages: strides 2^ls .. 1
         sync(G - 1);
-        if (G - 1 - ls == 1) lz_pass<NT, G, false, 1>(pol, n0, M, size, G - 1, tid);
-        else lz_pass<NT, G, false, (G >= 3 ? 2 : 1)>(pol, n0, M, size, G - 1, tid);
+        lz_pass<NT, G, false, 1>(pol, n0, M, size, G - 1, tid);
       }
     }
   }
   __syncthreads();
 }
 
-// The lazy dimension's order of a segment: local indices into iz.  buf: 8
-// SUB_MAX bytes of LDS; shd: 2 NT / 64 doubles; flagp: one word.  The packed
-// form first; a run of more than LZ_RUN colliding keys (a segment whose
-// coordinates are all equal, or nearly) sends the segment to the wide form.
-template <int NT>
-__device__ void lz_order(unsigned char *buf, uint16_t *iz, const uint32_t *ids, const double *zc,
-                         uint32_t n0, int tid, double *shd, uint32_t *flagp) {
+// A dimension's order of a segment: local indices into iz (its 2 SUB_MAX
+// bytes also hold the sort's counts before that).  buf: 8 SUB_MAX bytes of
+// LDS; shd: 2 NT / 64 doubles; flagp: two words.  zc(i): local index i's
+// coordinate.
+template <int NT, class Coord>
+__device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint32_t n0, int tid,
+                         double *shd, uint32_t *flagp) {
   constexpr int IT = SUB_MAX / NT;
   constexpr int NW = NT / 64;
   double z[IT];
@@ -1301,7 +1295,7 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const uint32_t *ids, 
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
     const uint32_t i = tid + q * NT;
-    z[q] = i < n0 ? zc[ids[i]] : 0.0;
+    z[q] = i < n0 ? zc(i) : 0.0;
     if (i < n0) {
       lo = fmin(lo, z[q]);
       hi = fmax(hi, z[q]);
@@ -1316,73 +1310,84 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const uint32_t *ids, 
     shd[tid >> 6] = lo;
     shd[NW + (tid >> 6)] = hi;
   }
-  if (tid == 0) *flagp = 0;
+  if (tid < 2) flagp[tid] = 0;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
     lo = fmin(lo, shd[w]);
     hi = fmax(hi, shd[NW + w]);
   }
-  // all coordinates equal (a planar system) leaves the order to the working
-  // ids, which the wide form gives directly
-  if (hi > lo) {
-    // a monotone map of the coordinate, so distinct keys are in coordinate
-    // order and only equal keys need the exact comparison
-    const double scale = (double)LZ_KEY_MAX / (hi - lo);
-    uint32_t *kp = reinterpret_cast<uint32_t *>(buf);
+  if (!(hi > lo)) {  // all coordinates equal (a planar system): any order
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       const uint32_t i = tid + q * NT;
-      if (i < n0) {
-        const uint32_t key = (uint32_t)fmin(fmax((z[q] - lo) * scale, 0.0), (double)LZ_KEY_MAX);
-        kp[i] = (key << (32 - LZ_KEY_BITS)) | i;
-      }
+      if (i < n0) iz[i] = (uint16_t)i;
     }
     __syncthreads();
-    lz_sort<NT, LZ_G>(LzPacked{kp}, n0, tid);
-    constexpr uint32_t IMASK = (1u << (32 - LZ_KEY_BITS)) - 1;
+    return;
+  }
+  // a monotone map of the coordinate, so distinct keys are in coordinate
+  // order and only equal keys need the exact comparison
+  const double scale = (double)LZ_KEY_MAX / (hi - lo);
+  uint32_t *kv = reinterpret_cast<uint32_t *>(buf), *kp = kv + SUB_MAX;
 #pragma unroll
-    for (int q = 0; q < IT; ++q) {
-      const uint32_t i = tid + q * NT;
-      if (i < n0) iz[i] = (uint16_t)(kp[i] & IMASK);
+  for (int q = 0; q < IT; ++q) {
+    const uint32_t i = tid + q * NT;
+    if (i < n0) {
+      const uint32_t key = (uint32_t)fmin(fmax((z[q] - lo) * scale, 0.0), (double)LZ_KEY_MAX);
+      kv[i] = (key << (32 - LZ_KEY_BITS)) | i;
     }
-    __syncthreads();
-    // runs of equal keys, each ordered by the thread at its start by
-    // (coordinate, working id)
+  }
+  __syncthreads();  // and shd, reused by the sort, has been read
+  lz_radix<NT>(kv, kp, n0, reinterpret_cast<uint32_t *>(iz), reinterpret_cast<uint32_t *>(shd),
+               tid);
+  constexpr uint32_t IMASK = (1u << (32 - LZ_KEY_BITS)) - 1;
 #pragma unroll
-    for (int q = 0; q < IT; ++q) {
-      const uint32_t i = tid + q * NT;
-      if (i + 1 >= n0) continue;
-      const uint32_t key = kp[i] >> (32 - LZ_KEY_BITS);
-      if ((kp[i + 1] >> (32 - LZ_KEY_BITS)) != key) continue;
-      if (i > 0 && (kp[i - 1] >> (32 - LZ_KEY_BITS)) == key) continue;
-      uint32_t j = i + 1;
-      while (j < n0 && j - i <= LZ_RUN && (kp[j] >> (32 - LZ_KEY_BITS)) == key) ++j;
-      if (j - i > LZ_RUN) {
-        *flagp = 1;
-        continue;
-      }
-      for (uint32_t x = i + 1; x < j; ++x) {
-        const uint16_t v = iz[x];
-        const uint32_t idv = ids[v];
-        const double zv = zc[idv];
-        uint32_t y = x;
-        while (y > i) {
-          const uint16_t u = iz[y - 1];
-          const uint32_t idu = ids[u];
-          const double zu = zc[idu];
-          if (zu < zv || (zu == zv && idu < idv)) break;
-          iz[y] = u;
-          --y;
-        }
-        iz[y] = v;
-      }
-    }
-  } else if (tid == 0) {
-    *flagp = 1;
+  for (int q = 0; q < IT; ++q) {
+    const uint32_t i = tid + q * NT;
+    if (i < n0) iz[i] = (uint16_t)(kp[i] & IMASK);
   }
   __syncthreads();
-  if (*flagp) {
+  // runs of equal keys with unequal coordinates, each ordered by the thread
+  // at its start (flagp[0]: such a pair exists, flagp[1]: a long run exists)
+#pragma unroll
+  for (int q = 0; q < IT; ++q) {
+    const uint32_t i = tid + q * NT;
+    if (i + 1 >= n0) continue;
+    const uint32_t a = kp[i], b = kp[i + 1];
+    if ((a ^ b) >> (32 - LZ_KEY_BITS)) continue;
+    if (zc(a & IMASK) != zc(b & IMASK)) flagp[0] = 1;
+  }
+  __syncthreads();
+  if (!flagp[0]) return;
+#pragma unroll
+  for (int q = 0; q < IT; ++q) {
+    const uint32_t i = tid + q * NT;
+    if (i + 1 >= n0) continue;
+    const uint32_t key = kp[i] >> (32 - LZ_KEY_BITS);
+    if ((kp[i + 1] >> (32 - LZ_KEY_BITS)) != key) continue;
+    if (i > 0 && (kp[i - 1] >> (32 - LZ_KEY_BITS)) == key) continue;
+    uint32_t j = i + 1;
+    while (j < n0 && j - i <= LZ_RUN && (kp[j] >> (32 - LZ_KEY_BITS)) == key) ++j;
+    if (j - i > LZ_RUN) {
+      flagp[1] = 1;
+      continue;
+    }
+    for (uint32_t x = i + 1; x < j; ++x) {
+      const uint16_t v = iz[x];
+      const double zv = zc(v);
+      uint32_t y = x;
+      while (y > i) {
+        const uint16_t u = iz[y - 1];
+        if (zc(u) <= zv) break;
+        iz[y] = u;
+        --y;
+      }
+      iz[y] = v;
+    }
+  }
+  __syncthreads();
+  if (flagp[1]) {
     uint64_t *kz = reinterpret_cast<uint64_t *>(buf);
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
@@ -1393,36 +1398,54 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const uint32_t *ids, 
       }
     }
     __syncthreads();
-    lz_sort<NT, 2>(LzWide{kz, iz, ids}, n0, tid);
+    lz_sort<NT, 2>(LzWide{kz, iz}, n0, tid);
   }
 }
 
-// At most 64 VGPRs, so that four workgroups (the LDS limit) fit on a CU
-// rather than three: the build takes 3.27 ms against 3.54 ms at 10 M bodies.
+// The subtree builder: one workgroup finishes a segment of <= SUB_MAX bodies.
+// What bounds it is latency: a level is a chain of LDS round trips between
+// four barriers.  So the lefts before a position are counted by ballots (one
+// 64-bit word of flags a list and wavefront) and a scan of the words' counts
+// in DPP, where a segmented scan of per-thread sums took three shuffles a
+// step, and a list needs no case for the dimension that is split (it is
+// partitioned already, and the counts say so).
+//   FEW: a grid of at most one workgroup a CU (up to ~500,000 bodies), where
+// LDS is not short: the segment's coordinates are kept there (48 KB), so the
+// splits and the state do not wait on global memory.  Otherwise four
+// workgroups share a CU (37 KB and at most 64 VGPRs each).
+//   a.sort_all (FEW, a single segment): no lists were sorted; each dimension
+// is ordered here.
+// Builds in us, against the segmented scan and the bitonic sort: 147 -> 61 at
+// 1,000 ring bodies (with 14 launches less), 217 -> 178 at 5,000, 341 -> 305 at
+// 100,000, 2884 -> 2757 at 10 M.
 #ifndef KD_SUB_WAVES
 #define KD_SUB_WAVES 8
 #endif
-__global__ __launch_bounds__(SUB_THREADS) __attribute__((amdgpu_waves_per_eu(KD_SUB_WAVES))) void
-k_subtree(SubArgs a) {
+template <bool FEW>
+__global__ __launch_bounds__(SUB_THREADS)
+    __attribute__((amdgpu_waves_per_eu(FEW ? 2 : KD_SUB_WAVES))) void k_subtree(SubArgs a) {
 #pragma clang fp contract(off)
-  constexpr int NT = SUB_THREADS, IT = SUB_ITEMS;
+  constexpr int NT = SUB_THREADS, IT = SUB_ITEMS, NWORD = SUB_MAX / 64;
+  static_assert(NWORD == 32, "the words of a list are scanned by half a wavefront");
   // one LDS buffer: ids (working id of every local index), lst (the three
-  // sorted lists of local indices, double-buffered), flag, sdarr; once the
-  // bodies are placed, the node moments reuse it as staging and node sums
-  __shared__ __align__(16) unsigned char smem[18 * SUB_MAX];
+  // sorted lists of local indices, double-buffered), flag, sdarr; FEW: the
+  // coordinates.  Once the bodies are placed, the node moments reuse it all
+  // as staging and node sums.
+  constexpr uint32_t SMEM = (FEW ? 42 : 18) * SUB_MAX;
+  __shared__ __align__(16) unsigned char smem[SMEM];
   uint32_t *ids = reinterpret_cast<uint32_t *>(smem);
   uint16_t(*lst)[3][SUB_MAX] = reinterpret_cast<uint16_t(*)[3][SUB_MAX]>(smem + 4 * SUB_MAX);
   uint8_t *flag = smem + 16 * SUB_MAX;
   uint8_t *sdarr = smem + 17 * SUB_MAX;
-  __shared__ uint64_t shv[NT / 64];
-
-  __shared__ uint32_t shh[NT / 64];
+  double(*sc)[SUB_MAX] = reinterpret_cast<double(*)[SUB_MAX]>(smem + 18 * SUB_MAX);  // FEW
+  __shared__ uint64_t words[3][NWORD];  // per list, the left flags of 64 positions
+  __shared__ uint8_t inner[SUB_MAX];    // subtree heap slots that split
   // per level (by parity): some segment of the level splits, so bodies are
   // still alive below it
   __shared__ uint32_t splits[2];
-  // the lazy dimension's sort: block range of the coordinate, fallback flag
+  // a dimension's sort: block range of the coordinate, flags
   __shared__ double shd[2 * NT / 64];
-  __shared__ uint32_t lzflag;
+  __shared__ uint32_t lzflag[2];
 
   const uint2 task = a.tasks ? a.tasks[blockIdx.x] : make_uint2(0u, blockIdx.x);
   const SysDesc S = a.sys[task.x];
@@ -1444,34 +1467,59 @@ k_subtree(SubArgs a) {
   if (n0 == 0) return;
   const int leaf = a.leaf;
   const int tid = threadIdx.x;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   if (tid < 2) splits[tid] = 0;
+  for (uint32_t i = tid; i < SUB_MAX; i += NT) inner[i] = 0;
+  auto coord = [&](int d, uint32_t i) { return FEW ? sc[d][i] : a.P.c[d][ids[i]]; };
 
-  for (uint32_t i = tid; i < n0; i += NT) {
-    uint32_t id = L0[sl + i];
-    ids[i] = id;
-    lst[0][g0][i] = (uint16_t)i;
-    a.loc[id] = i;
+  if (FEW && a.sort_all) {
+    for (uint32_t i = tid; i < n0; i += NT) {
+      ids[i] = i;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) sc[d][i] = a.P.c[d][i];
+    }
+    __syncthreads();
+    for (int d = 0; d < 3; ++d)
+      lz_order<NT>(smem + 10 * SUB_MAX, lst[0][d], [&](uint32_t i) { return sc[d][i]; }, n0, tid,
+                   shd, lzflag);
+  } else {
+    for (uint32_t i = tid; i < n0; i += NT) {
+      uint32_t id = L0[sl + i];
+      ids[i] = id;
+      lst[0][g0][i] = (uint16_t)i;
+      a.loc[id] = i;
+      if (FEW) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) sc[d][i] = a.P.c[d][id];
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (uint32_t i = tid; i < n0; i += NT) {
+      lst[0][g1][i] = (uint16_t)a.loc[L1[sl + i]];
+      if (lz == 3) lst[0][2][i] = (uint16_t)a.loc[L2[sl + i]];
+    }
+    __syncthreads();
+    if (lz < 3) {
+      // the lazy dimension's order; the keys use the LDS of the second list
+      // buffer, flags and sdarr (not live yet), the local indices end in
+      // lst[0][lz]
+      static_assert(18 * SUB_MAX - 10 * SUB_MAX >= 8 * SUB_MAX,
+                    "the sort's keys need 8 SUB_MAX bytes");
+      static_assert(2 * SUB_MAX >= NT / 64 * 128 * 4, "the sort's counts fit a list");
+      const double *zc = a.P.c[lz];
+      lz_order<NT>(smem + 10 * SUB_MAX, lst[0][lz],
+                   [&](uint32_t i) { return FEW ? sc[lz][i] : zc[ids[i]]; }, n0, tid, shd, lzflag);
+    }
   }
-  __threadfence_block();
   __syncthreads();
-  for (uint32_t i = tid; i < n0; i += NT) {
-    lst[0][g1][i] = (uint16_t)a.loc[L1[sl + i]];
-    if (lz == 3) lst[0][2][i] = (uint16_t)a.loc[L2[sl + i]];
-  }
-  __syncthreads();
-  if (lz < 3) {
-    // the lazy dimension's order; the keys use the LDS of the second list
-    // buffer, flags and sdarr (not live yet), the local indices end in
-    // lst[0][lz]
-    static_assert(18 * SUB_MAX - 10 * SUB_MAX >= 8 * SUB_MAX, "lazy-sort keys need 8 SUB_MAX bytes");
-    lz_order<NT>(smem + 10 * SUB_MAX, lst[0][lz], ids, a.P.c[lz], n0, tid, shd, &lzflag);
-  }
 
+  // positions j = it NT + tid: a wavefront holds 64 consecutive ones
   uint32_t st[IT], ct[IT], cc[IT], hl[IT];
   bool alive[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    uint32_t j = tid * IT + it;
+    uint32_t j = it * NT + tid;
     alive[it] = j < n0;
     st[it] = 0;
     ct[it] = n0;
@@ -1480,28 +1528,37 @@ k_subtree(SubArgs a) {
   }
   int cur = 0;
   int lam_end = 0;
+  // the first segment a thread decides at a level, loaded a level ahead
+  uint32_t next_s = tid == 0 ? s0l : 0u, next_c = tid == 0 ? n0 : 0u;
   for (int lam = 0;; ++lam) {
     const uint32_t hbase = (1u << (level + lam)) - 1 + (k << lam);
+    const uint32_t this_s = next_s, this_c = next_c;
+    {
+      const uint32_t hn = (1u << (level + lam + 1)) - 1 + (k << (lam + 1)) + tid;
+      const bool there = (uint32_t)tid < (2u << lam) && hn < S.slots;
+      next_s = there ? t.seg_start[hn] : 0u;
+      next_c = there ? t.seg_count[hn] : 0u;
+    }
     // one thread per segment of this level: split decision or leaf mark
     for (uint32_t c = tid; c < (1u << lam); c += NT) {
-      uint32_t sgs, sgc;
-      if (!sub_node(c, lam, n0, leaf, sgs, sgc)) continue;  // an ancestor is a leaf
       const uint32_t h = hbase + c;
+      const uint32_t sgc = c == (uint32_t)tid ? this_c : t.seg_count[h];
+      if (sgc == 0) continue;  // an ancestor is a leaf
+      const uint32_t sgs = (c == (uint32_t)tid ? this_s : t.seg_start[h]) - s0l;
       if (sgc <= (uint32_t)leaf) {
         sdarr[sgs] = 0xFF;  // leaf: its bodies are finished at this level
       } else {
         // the ends and the two middle keys of every dimension as one batch of
         // independent loads (one round trip; the dimension index is a
         // constant in each load, so no pointer is fetched at run time)
-        const uint32_t mid = sgs + sgc / 2;
+        const uint32_t mid = sgs + sgc / 2, end = sgs + sgc - 1;
         const uint16_t *l0 = lst[cur][0], *l1 = lst[cur][1], *l2 = lst[cur][2];
-        const double *c0 = a.P.c[0], *c1 = a.P.c[1], *c2 = a.P.c[2];
-        const double e0 = c0[ids[l0[sgs + sgc - 1]]] - c0[ids[l0[sgs]]];
-        const double e1 = c1[ids[l1[sgs + sgc - 1]]] - c1[ids[l1[sgs]]];
-        const double e2 = c2[ids[l2[sgs + sgc - 1]]] - c2[ids[l2[sgs]]];
-        const double m0 = c0[ids[l0[mid]]], p0 = c0[ids[l0[mid - 1]]];
-        const double m1 = c1[ids[l1[mid]]], p1 = c1[ids[l1[mid - 1]]];
-        const double m2 = c2[ids[l2[mid]]], p2 = c2[ids[l2[mid - 1]]];
+        const double e0 = coord(0, l0[end]) - coord(0, l0[sgs]);
+        const double e1 = coord(1, l1[end]) - coord(1, l1[sgs]);
+        const double e2 = coord(2, l2[end]) - coord(2, l2[sgs]);
+        const double m0 = coord(0, l0[mid]), p0 = coord(0, l0[mid - 1]);
+        const double m1 = coord(1, l1[mid]), p1 = coord(1, l1[mid - 1]);
+        const double m2 = coord(2, l2[mid]), p2 = coord(2, l2[mid - 1]);
         // argmax with ties to the lower dimension, by selects
         const bool s1 = e1 > e0;
         const double b01 = s1 ? e1 : e0;
@@ -1511,9 +1568,9 @@ k_subtree(SubArgs a) {
         const double kv = s2 ? m2 : (s1 ? m1 : m0);
         const double kprev = s2 ? p2 : (s1 ? p1 : p0);
         uint16_t *ls = lst[cur][sd];
-        const double *key = a.P.c[sd];
         if (kprev == kv) {
           // equal keys straddle the median: order the run by original index
+          const double *key = a.P.c[sd];
           uint32_t r0 = mid, r1 = mid + 1;
           while (r0 > sgs && key[ids[ls[r0 - 1]]] == kv) --r0;
           while (r1 < sgs + sgc && key[ids[ls[r1]]] == kv) ++r1;
@@ -1532,78 +1589,78 @@ k_subtree(SubArgs a) {
         t.split_val[h] = kv;
         t.size[h] = best;
         sdarr[sgs] = (uint8_t)sd;
+        inner[(1u << lam) - 1 + c] = 1;
         splits[lam & 1] = 1;
       }
     }
     __syncthreads();
+    lam_end = lam;
+    uint32_t sd[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      if (alive[it] && sdarr[st[it]] == 0xFF) {
+      sd[it] = alive[it] ? sdarr[st[it]] : 0xFFu;
+      if (alive[it] && sd[it] == 0xFF) {
         alive[it] = false;
         hl[it] = hbase + cc[it];  // heap slot of the leaf this body ends in
       }
     }
-    lam_end = lam;
     // a body is still alive iff its segment splits at this level
     if (!splits[lam & 1]) break;
     // the other parity's flag was last read at the previous level, before
     // the barrier above; the next level sets it after later barriers
     if (tid == 0) splits[(lam + 1) & 1] = 0;
 
-    // flags from the split-dim list
+    // left flags, from the split dimension's list
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      if (!alive[it]) continue;
-      uint32_t j = tid * IT + it;
-      int sd = sdarr[st[it]];
-      uint32_t mid = st[it] + ct[it] / 2;
-      flag[lst[cur][sd][j]] = j < mid ? 1 : 0;
+      const uint32_t j = it * NT + tid;
+      if (alive[it]) flag[lst[cur][sd[it]][j]] = j < st[it] + ct[it] / 2 ? 1 : 0;
     }
     __syncthreads();
-
-    // segmented exclusive scan of the left flags, three lists packed
-    uint64_t v[IT];
-    uint32_t hd[IT];
-    SegV agg;
-    agg.v = 0;
-    agg.h = 0;
+    // every list's flags in list order, a word per 64 positions
+    uint32_t x[IT][3];
+    uint64_t b[IT][3];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      uint32_t j = tid * IT + it;
-      v[it] = 0;
-      hd[it] = 1;
-      if (alive[it]) {
-        int sd = sdarr[st[it]];
+      const uint32_t j = it * NT + tid;
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-          if (d != sd) v[it] += (uint64_t)flag[lst[cur][d][j]] << (16 * d);
-        hd[it] = (j == st[it]) ? 1u : 0u;
-      }
-      SegV e;
-      e.v = v[it];
-      e.h = hd[it];
-      agg = seg_combine(agg, e);
+      for (int d = 0; d < 3; ++d) x[it][d] = j < n0 ? lst[cur][d][j] : 0u;
     }
-    SegV carry = block_seg_carry<NT>(agg, shv, shh);
-    uint64_t run = carry.v;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      uint32_t j = tid * IT + it;
-      if (hd[it]) run = 0;
-      uint64_t ex = run;  // lefts before j in its segment, per list
-      run += v[it];
-      if (j >= n0) continue;
-      int sd = alive[it] ? sdarr[st[it]] : -1;
-      uint32_t mid = st[it] + ct[it] / 2;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        uint16_t x = lst[cur][d][j];
-        uint32_t dst = j;
-        if (alive[it] && d != sd) {
-          uint32_t e = (uint32_t)((ex >> (16 * d)) & 0xFFFFu);
-          dst = flag[x] ? st[it] + e : mid + (j - st[it] - e);
-        }
-        lst[cur ^ 1][d][dst] = x;
+        b[it][d] = __builtin_amdgcn_ballot_w64(alive[it] && flag[x[it][d]] != 0);
+        if (lane == 0) words[d][it * (NT / 64) + wv] = b[it][d];
+      }
+    }
+    __syncthreads();
+    // lefts before every word: lists 0 (low half) and 1, then list 2
+    const uint32_t q = lane & (NWORD - 1);
+    const uint32_t p01 = (uint32_t)__builtin_popcountll(words[0][q]) |
+                         ((uint32_t)__builtin_popcountll(words[1][q]) << 16);
+    const uint32_t p2 = (uint32_t)__builtin_popcountll(words[2][q]);
+    const uint32_t e01 = lane_scan<false>(p01) - p01, e2 = lane_scan<false>(p2) - p2;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t j = it * NT + tid, w = it * (NT / 64) + wv;
+      // lefts before the segment: the same in every list, read in list 0
+      // (on every lane: the scan's lanes must be active to be read)
+      const uint32_t sw = st[it] >> 6;
+      const uint32_t lb = (__shfl(e01, sw, 64) & 0xFFFFu) +
+                          (uint32_t)__builtin_popcountll(words[0][sw] &
+                                                         ((1ull << (st[it] & 63u)) - 1u));
+      const uint32_t f01 = (uint32_t)__builtin_amdgcn_readlane((int)e01, (int)w);
+      const uint32_t f2 = (uint32_t)__builtin_amdgcn_readlane((int)e2, (int)w);
+      if (j >= n0) continue;
+      const uint32_t mid = st[it] + ct[it] / 2;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const uint32_t pre = d == 0 ? f01 & 0xFFFFu : d == 1 ? f01 >> 16 : f2;
+        const uint32_t e = pre + lanes_below(b[it][d]) - lb;  // lefts before j in its segment
+        const bool left = (b[it][d] >> lane) & 1u;
+        const uint32_t dst = !alive[it] ? j : left ? st[it] + e : mid + (j - st[it] - e);
+        lst[cur ^ 1][d][dst] = (uint16_t)x[it][d];
       }
     }
     __syncthreads();
@@ -1611,7 +1668,7 @@ k_subtree(SubArgs a) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
       if (!alive[it]) continue;
-      uint32_t j = tid * IT + it;
+      uint32_t j = it * NT + tid;
       uint32_t mid = st[it] + ct[it] / 2;
       if (j < mid) {
         ct[it] = ct[it] / 2;
@@ -1633,7 +1690,7 @@ k_subtree(SubArgs a) {
   uint32_t ow[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    uint32_t j = tid * IT + it;
+    uint32_t j = it * NT + tid;
     ow[it] = 0;
     if (j < n0) {
       ow[it] = a.in.oid[ids[lst[cur][0][j]]];
@@ -1643,18 +1700,24 @@ k_subtree(SubArgs a) {
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    uint32_t j = tid * IT + it;
+    uint32_t j = it * NT + tid;
     if (j >= n0) continue;
     uint32_t rank = 0;
     for (uint32_t q = st[it]; q < st[it] + ct[it]; ++q) rank += oidl[q] < ow[it] ? 1u : 0u;
     permloc[st[it] + rank] = lst[cur][0][j];
   }
   __syncthreads();
-  for (uint32_t i = tid; i < n0; i += NT) {
-    const uint32_t w = ids[permloc[i]];
+  double bx[IT], by[IT], bz[IT], bm[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const uint32_t i = it * NT + tid;
+    bx[it] = by[it] = bz[it] = bm[it] = 0.0;
+    if (i >= n0) continue;
+    const uint32_t li = permloc[i], w = ids[li];
     const uint32_t tpos = s0 + i;
     a.perm[tpos] = w;
-    double x = a.in.x[w], y = a.in.y[w], z = a.in.z[w], m = a.in.m[w];
+    const double x = FEW ? sc[0][li] : a.in.x[w], y = FEW ? sc[1][li] : a.in.y[w],
+                 z = FEW ? sc[2][li] : a.in.z[w], m = a.in.m[w];
     a.out.x[tpos] = x;
     a.out.y[tpos] = y;
     a.out.z[tpos] = z;
@@ -1666,69 +1729,106 @@ k_subtree(SubArgs a) {
     // the walk's body records, for the arithmetic that reads them
     if (t.recs & (REC_64 | REC_D)) a.pos64[tpos] = make_double4(x, y, z, m);
     if (t.recs & REC_32) a.pos32[tpos] = make_float4((float)x, (float)y, (float)z, (float)m);
+    bm[it] = m;
+    bx[it] = m * x;
+    by[it] = m * y;
+    bz[it] = m * z;
   }
   __threadfence_block();
   __syncthreads();
-  // Node moments (m, m x, m y, m z).  The members' terms of one quantity at a
-  // time are staged in LDS in tree order; each leaf's first thread adds its
-  // members in canonical order, and the internal nodes are summed bottom-up
-  // (left + right) in LDS, one level per barrier, so no level waits on
-  // global memory.  Every sum also goes to the node arrays.  When the node
-  // sums of all four quantities fit beside the staged terms (nslot heap
-  // slots of the subtree each: the ring's segments of ~1220 bodies need 511),
-  // the four bottom-up passes share their barriers; otherwise each quantity
-  // takes its own pass with SUB_MAX slots (the deepest leaf of at most
-  // SUB_MAX bodies lies above depth log2(SUB_MAX)).
+  // Node moments (m, m x, m y, m z).  The members' terms are staged in LDS in
+  // tree order, as many quantities at a time as fit; each leaf's first thread
+  // adds its members in canonical order, and the internal nodes are summed
+  // bottom-up (left + right) in LDS.  Every sum also goes to the node arrays.
+  // nslot: heap slots of the subtree (the ring's segments of ~1220 bodies
+  // have 511).  When the node sums of all four quantities fit beside the
+  // staged terms, a wavefront sums the subtree below one node of depth 3 by
+  // itself and the first one the nodes above, with one barrier between;
+  // otherwise each quantity takes its own pass with a barrier a level and
+  // SUB_MAX slots (the deepest leaf of at most SUB_MAX bodies lies above
+  // depth log2(SUB_MAX)).
   double *stg = reinterpret_cast<double *>(smem);
-  static_assert(sizeof(smem) >= 2 * SUB_MAX * sizeof(double), "moments need 16 SUB_MAX bytes");
+  static_assert(SMEM >= 2 * SUB_MAX * sizeof(double), "moments need 16 SUB_MAX bytes");
   double *const dsts[4] = {t.mm, t.mx, t.my, t.mz};
   const uint32_t nslot = (2u << lam_end) - 1;
-  const bool joint = (n0 + 4 * nslot) * sizeof(double) <= sizeof(smem);
+  constexpr uint32_t CAP = SMEM / sizeof(double);
+  const bool joint = n0 + 4 * nslot <= CAP;
+  // quantities staged at a time
+  const int G = 4 * n0 + 4 * nslot <= CAP ? 4 : 2 * n0 + 4 * nslot <= CAP ? 2 : 1;
   // node sums: quantity q's at nsum + q * qstride
-  double *nsum = joint ? stg + n0 : stg + SUB_MAX;
+  double *nsum = joint ? stg + G * n0 : stg + SUB_MAX;
   const uint32_t qstride = joint ? nslot : 0;
+#pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const double *pc = q == 1 ? a.out.x : (q == 2 ? a.out.y : a.out.z);
-    for (uint32_t i = tid; i < n0; i += NT) {
-      const double bm = a.out.m[s0 + i];
-      stg[i] = q == 0 ? bm : bm * pc[s0 + i];
-    }
-    __syncthreads();
-    double *dst = dsts[q];
-    double *ns = nsum + q * qstride;
+    const double *bq = q == 0 ? bm : q == 1 ? bx : q == 2 ? by : bz;
+    double *sq = stg + (q & (G - 1)) * n0;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const uint32_t j = tid * IT + it;
+      const uint32_t i = it * NT + tid;
+      if (i < n0) sq[i] = bq[it];
+    }
+    if ((q + 1) & (G - 1)) continue;  // the group's other quantities first
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t j = it * NT + tid;
       if (j >= n0 || j != st[it]) continue;
-      double sum = 0.0;
-      for (uint32_t r = 0; r < ct[it]; ++r) sum += stg[st[it] + r];
-      dst[hl[it]] = sum;
       // the leaf's slot in the subtree's own heap: hl + 1 = 2^(level + lam)
       // + (k << lam) + index within depth lam
       const uint32_t lam = (31 - __clz(hl[it] + 1)) - level;
-      ns[hl[it] + (1u << lam) - (1u << (level + lam)) - (k << lam)] = sum;
+      const uint32_t rel = hl[it] + (1u << lam) - (1u << (level + lam)) - (k << lam);
+      for (int r = q + 1 - G; r <= q; ++r) {
+        const double *sr = stg + (r & (G - 1)) * n0;
+        double sum = 0.0;
+        for (uint32_t x = 0; x < ct[it]; ++x) sum += sr[st[it] + x];
+        dsts[r][hl[it]] = sum;
+        nsum[r * qstride + rel] = sum;
+      }
     }
     __syncthreads();
-    if (joint && q < 3) continue;  // the bottom-up sums of all four follow the last
+    if (joint) continue;  // the bottom-up sums of all four follow the last
     for (int lam = lam_end - 1; lam >= 0; --lam) {
       const uint32_t hbase = (1u << (level + lam)) - 1 + (k << lam);
       for (uint32_t c = tid; c < (1u << lam); c += NT) {
-        uint32_t s, cnt;
-        if (!sub_node(c, lam, n0, leaf, s, cnt) || cnt <= (uint32_t)leaf) continue;
         const uint32_t rel = (1u << lam) - 1 + c;
-        for (int r = joint ? 0 : q; r <= q; ++r) {
-          double *nr = nsum + r * qstride;
-          const double v = nr[2 * rel + 1] + nr[2 * rel + 2];
-          nr[rel] = v;
-          dsts[r][hbase + c] = v;
-        }
+        if (!inner[rel]) continue;
+        const double v = nsum[2 * rel + 1] + nsum[2 * rel + 2];
+        nsum[rel] = v;
+        dsts[q][hbase + c] = v;
       }
       __syncthreads();
     }
   }
+  if (joint) {
+    auto add_up = [&](uint32_t c, int lam) {
+      const uint32_t rel = (1u << lam) - 1 + c, h = (1u << (level + lam)) - 1 + (k << lam) + c;
+      if (!inner[rel]) return;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        double *nr = nsum + r * qstride;
+        const double v = nr[2 * rel + 1] + nr[2 * rel + 2];
+        nr[rel] = v;
+        dsts[r][h] = v;
+      }
+    };
+    static_assert(NT / 64 == 8, "a wavefront a node of depth 3");
+    for (int lam = lam_end - 1; lam >= 3; --lam) {
+      for (uint32_t c = lane; c < (1u << (lam - 3)); c += 64) add_up((wv << (lam - 3)) + c, lam);
+      wave_sync();
+    }
+    __syncthreads();
+    if (wv == 0) {
+      for (int lam = min(lam_end - 1, 2); lam >= 0; --lam) {
+        if (lane < (1u << lam)) add_up(lane, lam);
+        wave_sync();
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    const uint32_t j = tid * IT + it;
+    const uint32_t j = it * NT + tid;
     if (j < n0 && j == st[it]) write_leaf_rec(t, hl[it], s0l + st[it], ct[it]);
   }
   // internal records, over the subtree's heap slots (at most two a thread):
@@ -1736,9 +1836,9 @@ k_subtree(SubArgs a) {
   for (uint32_t rel = tid; rel + 1 < (1u << lam_end); rel += NT) {
     const int lam = 31 - __clz(rel + 1);
     const uint32_t c = rel + 1 - (1u << lam);
-    uint32_t s, cnt;
-    if (!sub_node(c, lam, n0, leaf, s, cnt) || cnt <= (uint32_t)leaf) continue;
-    write_internal_rec(t, (1u << (level + lam)) - 1 + (k << lam) + c, s0l + s, cnt, a.theta2);
+    if (!inner[rel]) continue;
+    const uint32_t h = (1u << (level + lam)) - 1 + (k << lam) + c;
+    write_internal_rec(t, h, t.seg_start[h], t.seg_count[h], a.theta2);
   }
 }
 
@@ -1835,6 +1935,17 @@ size_t sort_temp_bytes(uint32_t n, int /*nsys*/) {
   return bytes;
 }
 
+bool one_segment(const Forest &f) { return f.nsys == 1 && f.max_sub_level == 0; }
+
+// Workgroups of the subtree builder up to which each has a CU to itself (two
+// of the FEW form do not fit a CU).  Builds in us, without / with it: 196 / 177
+// at 5,000 ring bodies (4 workgroups), 321 / 307 at 100,000 (64), 505 / 481 at
+// 500,000 (256); 538 / 563 at 700,000 (512) with the limit at 512.
+#ifndef KD_FEW_GROUPS
+#define KD_FEW_GROUPS 256
+#endif
+constexpr uint32_t FEW_GROUPS = KD_FEW_GROUPS;
+
 // Tiles per segment at a device-wide level.
 static uint32_t level_tiles(const Forest &f, int lev) {
   const uint32_t nseg = 1u << lev;
@@ -1903,8 +2014,11 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
                         bool mid) {
   const double *coord[3] = {in.x, in.y, in.z};
   const unsigned ny = (unsigned)f.nsys;
-  hipError_t e;
-  if (report) {
+  hipError_t e = hipSuccess;
+  // one segment holds the whole system: the subtree builder sorts it, and the
+  // coordinate range, the lists and the report are not needed
+  const bool whole = one_segment(f);
+  if (report && !whole) {
     e = hipMemsetAsync(b.viol, 0, sizeof(uint32_t), s);
     if (e != hipSuccess) return e;
   }
@@ -1913,7 +2027,7 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
   // order at [list_off, list_off + n) (padding last)
   const uint32_t nsort = f.nsys == 1 ? f.max_n : f.total;
   if (sort_temp_bytes(nsort, f.nsys) > b.sort_tmp_bytes) return hipErrorInvalidValue;
-  if (!range_ready) {
+  if (!range_ready && !whole) {
     k_range_init<<<1, 64, 0, s>>>(b.range);
     k_range<<<std::min<uint32_t>((nsort + 255) / 256, RANGE_BLOCKS), 256, 0, s>>>(
         in.x, in.y, in.z, nsort, b.range);
@@ -1921,10 +2035,11 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
   // the three coordinate sorts are independent: dimension 0 runs on s,
   // dimensions 1 and 2 on the side streams, forked after the range and
   // joined before the levels (a graph capture of s follows the fork)
-  e = hipEventRecord(b.fork, s);
-  for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipStreamWaitEvent(b.side[i], b.fork, 0);
+  if (!whole) e = hipEventRecord(b.fork, s);
+  for (int i = 0; i < 2 && e == hipSuccess && !whole; ++i)
+    e = hipStreamWaitEvent(b.side[i], b.fork, 0);
   if (e != hipSuccess) return e;
-  for (int d = 0; d < 3; ++d) {
+  for (int d = 0; d < 3 && !whole; ++d) {
     const hipStream_t sd = d == 0 ? s : b.side[d - 1];
     if (d == lazy) continue;  // sorted per segment by the subtree builder
     uint32_t *key32 = b.keys_in[d];
@@ -1941,7 +2056,7 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
         key32_out, b.L[d], coord[d], nsort, b.range + 2 * d, b.runs[d]);
     k_fix_long<<<256, 256, 0, sd>>>(b.runs[d], key32_out, nsort, b.L[d], b.ids_in[d], coord[d]);
   }
-  for (int i = 0; i < 2 && e == hipSuccess; ++i) {
+  for (int i = 0; i < 2 && e == hipSuccess && !whole; ++i) {
     e = hipEventRecord(b.join[i], b.side[i]);
     if (e == hipSuccess) e = hipStreamWaitEvent(s, b.join[i], 0);
   }
@@ -1977,7 +2092,7 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
     k_level_mid<<<f.n_mid_tasks, MID_THREADS, 0, s>>>(LB, P, t, f.sys, f.mid_tasks, in.oid,
                                                       b.range, lazy, report ? b.viol : nullptr,
                                                       b.flags);
-  if (report) {
+  if (report && !whole) {
     e = hipMemcpyAsync(b.viol_host, b.viol, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
     // (a captured build is waited for by the stream, not the event)
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2001,7 +2116,12 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
   a.theta2 = theta * theta;
   a.lazy = lazy;
   a.tasks = f.nsys > 1 ? f.sub_tasks : nullptr;
-  k_subtree<<<f.nsys > 1 ? f.n_sub_tasks : 1u << f.max_sub_level, SUB_THREADS, 0, s>>>(a);
+  a.sort_all = whole;
+  const uint32_t groups = f.nsys > 1 ? f.n_sub_tasks : 1u << f.max_sub_level;
+  if (groups <= FEW_GROUPS)
+    k_subtree<true><<<groups, SUB_THREADS, 0, s>>>(a);
+  else
+    k_subtree<false><<<groups, SUB_THREADS, 0, s>>>(a);
   if (f.max_sub_level > 0) k_moments_top<<<ny, 1024, 0, s>>>(t, f.sys, theta * theta);
   return hipGetLastError();
 }

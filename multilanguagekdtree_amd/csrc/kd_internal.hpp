@@ -275,6 +275,9 @@ struct BuildBufs {
   hipEvent_t ev_viol = nullptr;
 };
 
+// Whether the build of f is the subtree builder alone (a single system of at
+// most SUB_MAX bodies): it reads no coordinate range and reports nothing.
+bool one_segment(const Forest &f);
 Shape make_shape(int64_t n, int leaf);
 SysDesc make_sys(const Shape &sh, uint32_t body_off, uint32_t node_off, uint32_t list_off);
 size_t sort_temp_bytes(uint32_t n, int nsys);
