@@ -77,3 +77,24 @@ def test_all_equal_and_single():
     assert ix[1234] == 1234  # ties go by index
     check_post(ix, 1234, vals, before)
     assert K.quickstat_index([0], 0, [1.0]).tolist() == [0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 4096, 4097, 16384, 16385, 131072, 131073, 1_000_003,
+                               4_200_001, 9_000_001])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "sorted", "few", "equal"])
+def test_narrowing_bounds(n, kind):
+    # sizes around every change in the number of rounds, ranks at the ends
+    # and inside, and values whose ties send the call to the radix passes
+    rng = np.random.default_rng(n)
+    vals = {"uniform": lambda: rng.random(n), "normal": lambda: rng.normal(size=n) * 1e3,
+            "sorted": lambda: np.sort(rng.random(n))[::-1].copy(),
+            "few": lambda: rng.integers(0, 9, n).astype(np.float64),
+            "equal": lambda: np.full(n, -2.5)}[kind]()
+    ranks = {0, n - 1, n // 2, int(rng.integers(0, n))} if n < 10**6 else {n // 3}
+    before = rng.permutation(n).astype(np.int64)
+    order = np.lexsort((np.arange(n), vals))
+    for goal in ranks:
+        ix = K.quickstat_index(before, goal, vals)
+        assert ix[goal] == order[goal]
+        check_post(ix, goal, vals, before)
