@@ -16,6 +16,20 @@
 // dc/dm_j = (p_j - c) / M, dM/dm_j = 1.  All adjoint sums are FP64 (global
 // FP64 atomics); the mixed path evaluates its terms in FP32 like its forward
 // walk.  Adjoint arrays are in original body order.
+//
+// What bounds the walk is latency: at 100,000 bodies there are 1,563
+// wavefronts of 64 bodies, each a chain of some 1,000 node and 750 leaf-body
+// visits.  So a workgroup of S wavefronts walks 64 bodies, each taking every
+// S-th subtree of depth log2(S) + 2 (the sums are atomic, so their order is
+// free); leaf bodies come in batches of scalar loads; and the reactions of a
+// batch, one column of 64 lanes per value, are summed in registers by
+// exchanging halves: a stage adds two columns into one (the lanes of one half
+// keep the first, of the other half the second), 16 columns take 15 such adds
+// and 2 more, and one atomic instruction adds the batch to consecutive words (the
+// reactions are kept in tree order).  At 100,000 ring bodies the mixed walk
+// takes 0.90 ms against 1.57 with one wavefront, bodies one by one and the
+// reactions through LDS (a row of 34 doubles a lane, 17 KB a wavefront); the
+// atomics are 0.18 ms of it.
 #include <algorithm>
 
 #include "kd_internal.hpp"
@@ -26,41 +40,37 @@ __device__ __forceinline__ uint32_t uni_a(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
 }
 
-__device__ __forceinline__ uint32_t heap_next_a(uint32_t h, int &depth) {
-  int t = __builtin_ctz(~h);
-  h >>= t;
-  depth -= t;
-  return h == 0 ? 0 : h + 1;
-}
-
-// gd = d/dd (u . f(d, mq)), gm = d/dmq (u . f(d, mq)), FP64.
-__device__ __forceinline__ void vjp64(double dx, double dy, double dz, double mq, double ux,
-                                      double uy, double uz, double &gx, double &gy, double &gz,
-                                      double &gm) {
+// gd = d/dd (u . f(d, mq)), gm = d/dmq (u . f(d, mq)), FP64; d2 = |d|^2.
+__device__ __forceinline__ void vjp64(double dx, double dy, double dz, double d2, double mq,
+                                      double ux, double uy, double uz, double &gx, double &gy,
+                                      double &gz, double &gm) {
 #pragma clang fp contract(off)
-  const double d2 = dx * dx + dy * dy + dz * dz;
   const double r = sqrt(d2);
-  const double r3 = d2 * r;
+  const double ri3 = 1.0 / (d2 * r);  // one division a term
+  const double ri2 = r * ri3;
   const double du = dx * ux + dy * uy + dz * uz;
-  const double k = 3.0 * du / (r3 * d2);
-  gx = -mq * (ux / r3 - k * dx);
-  gy = -mq * (uy / r3 - k * dy);
-  gz = -mq * (uz / r3 - k * dz);
-  gm = -du / r3;
-}
-
-// The same in FP32 with a hardware reciprocal square root (mixed path).
-__device__ __forceinline__ void vjp32(float dx, float dy, float dz, float mq, float ux, float uy,
-                                      float uz, float &gx, float &gy, float &gz, float &gm) {
-  const float d2 = dx * dx + dy * dy + dz * dz;
-  const float ri = __builtin_amdgcn_rsqf(d2);
-  const float ri2 = ri * ri;
-  const float ri3 = ri2 * ri;
-  const float du = dx * ux + dy * uy + dz * uz;
-  const float k = 3.f * du * ri3 * ri2;
+  const double k = 3.0 * du * ri3 * ri2;
   gx = -mq * (ux * ri3 - k * dx);
   gy = -mq * (uy * ri3 - k * dy);
   gz = -mq * (uz * ri3 - k * dz);
+  gm = -du * ri3;
+}
+
+// The same in FP32 with a hardware reciprocal square root (mixed path), from
+// the differences and their d2.  The fused operations are written out, so that
+// a term's rounding does not depend on the code around it.
+__device__ __forceinline__ void vjp32(float dx, float dy, float dz, float d2, float mq, float ux,
+                                      float uy, float uz, float &gx, float &gy, float &gz,
+                                      float &gm) {
+#pragma clang fp contract(off)
+  const float ri = __builtin_amdgcn_rsqf(d2);
+  const float ri2 = ri * ri;
+  const float ri3 = ri2 * ri;
+  const float du = __builtin_fmaf(dz, uz, __builtin_fmaf(dx, ux, dy * uy));
+  const float k = 3.f * du * ri3 * ri2;
+  gx = -mq * __builtin_fmaf(ux, ri3, -(k * dx));
+  gy = -mq * __builtin_fmaf(uy, ri3, -(k * dy));
+  gz = -mq * __builtin_fmaf(uz, ri3, -(k * dz));
   gm = -du * ri3;
 }
 
@@ -71,183 +81,233 @@ struct AdjWalk {
   const float4 *pos32;
   const uint32_t *oid;     // tree position -> original index
   const double *ux, *uy, *uz;  // seed, original order
-  double *lpx, *lpy, *lpz, *lm;  // adjoint accumulators, original order
-  double *gx, *gy, *gz, *gh;     // per node: d/dc_n and d/dM_n
-  double *body[4];               // lpx, lpy, lpz, lm
-  double *node[4];               // gx, gy, gz, gh
+  double *react;  // per tree position: d/dp (x, y, z) and d/dm of this step
+  double *gnode;  // per heap slot: d/dc (x, y, z) and d/dM
   uint32_t n;
   uint32_t leaf;
   double theta2;
 };
 
-// Reaction terms (to a partner body or to a node) are summed over the
-// wavefront before their FP64 atomics.  Instead of four 64-lane reductions
-// per term, a wavefront buffers up to EV terms in LDS, one row of 4 EV values
-// per lane, then lane l sums column l over the 64 rows (in row order) and
-// issues the one atomic for value l: the EV terms' 4 EV atomics go out as
-// one instruction.  The buffer is private to the wavefront and every access
-// happens in wave-uniform control flow, so no workgroup barrier is needed:
-// the flush waits for the wavefront's own LDS writes (lgkmcnt 0) before the
-// column reads, and the asm barriers keep the compiler from moving them.
-constexpr int EV = 8;
-constexpr int EV_ROW = 4 * EV + 2;  // doubles per lane row; rows stay 16-byte aligned
-constexpr int ADJ_THREADS = 256;
-constexpr uint32_t EV_NODE = 0x80000000u;  // tag bit: node arrays, else body arrays
-
-struct EvBuf {
-  double (*v)[EV_ROW];  // this wavefront's 64 rows
-  uint32_t *tag;        // per buffered term: target index | EV_NODE
-  uint32_t n;           // buffered terms (wave-uniform)
-};
-
-__device__ __forceinline__ void ev_flush(EvBuf &b, const AdjWalk &a) {
-  const uint32_t lane = threadIdx.x & 63;
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt left at their maximum
-  if (lane < 4 * b.n) {
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll 4
-    for (int k = 0; k < 64; k += 4) {
-      s0 += b.v[k][lane];
-      s1 += b.v[k + 1][lane];
-      s2 += b.v[k + 2][lane];
-      s3 += b.v[k + 3][lane];
-    }
-    const double sum = (s0 + s1) + (s2 + s3);
-    const uint32_t tag = b.tag[lane >> 2], c = lane & 3u;
-    double *const *arr = (tag & EV_NODE) ? a.node : a.body;
-    atomicAdd(arr[c] + (tag & ~EV_NODE), sum);
+// a + b, where lane l of a column gives to lane l ^ 32 (SWAP 32) or l ^ 16
+// (SWAP 16) and the lanes with that bit clear keep column a, the others b.
+template <int SWAP>
+__device__ __forceinline__ double fold_swap(double a, double b) {
+  typedef uint32_t pair __attribute__((ext_vector_type(2)));
+  const uint32_t al = (uint32_t)__double2loint(a), ah = (uint32_t)__double2hiint(a);
+  const uint32_t bl = (uint32_t)__double2loint(b), bh = (uint32_t)__double2hiint(b);
+  pair lo, hi;
+  if (SWAP == 32) {
+    lo = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+    hi = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+  } else {
+    lo = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    hi = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
   }
-  asm volatile("" ::: "memory");
-  b.n = 0;
+  return __hiloint2double((int)hi.x, (int)lo.x) + __hiloint2double((int)hi.y, (int)lo.y);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+// The same within a row of 16, where CTRL takes lane l to one whose bit
+// differs and `second` says whether the lane keeps column b.
+template <int CTRL>
+__device__ __forceinline__ double fold_row(double a, double b, bool second) {
+  const double keep = second ? b : a, give = second ? a : b;
+  return keep + dpp_f64<CTRL>(give);
+}
+constexpr int ROW_ROR8 = 0x128, ROW_HALF_MIRROR = 0x141, QUAD_2301 = 0x4E, QUAD_1032 = 0xB1;
+
+// Sums of the wavefront's 4 columns v: lane 16 q + r holds column
+// fold4_col(lane).
+__device__ __forceinline__ double fold4(const double v[4]) {
+  double s = fold_swap<16>(fold_swap<32>(v[0], v[1]), fold_swap<32>(v[2], v[3]));
+  s += dpp_f64<ROW_ROR8>(s);
+  s += dpp_f64<ROW_HALF_MIRROR>(s);
+  s += dpp_f64<QUAD_2301>(s);
+  s += dpp_f64<QUAD_1032>(s);
+  return s;
+}
+__device__ __forceinline__ uint32_t fold4_col(uint32_t lane) {
+  return (lane >> 5) | ((lane >> 3) & 2u);
+}
+// Sums of 16 columns: lane l holds column fold16_col(l).
+__device__ __forceinline__ double fold16(const double v[16], uint32_t lane) {
+  double a[8], b[4], c[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = fold_swap<32>(v[2 * i], v[2 * i + 1]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = fold_swap<16>(a[2 * i], a[2 * i + 1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    c[i] = fold_row<ROW_ROR8>(b[2 * i], b[2 * i + 1], (lane & 8u) != 0);
+  double s = fold_row<ROW_HALF_MIRROR>(c[0], c[1], (lane & 4u) != 0);
+  s += dpp_f64<QUAD_2301>(s);
+  s += dpp_f64<QUAD_1032>(s);
+  return s;
+}
+__device__ __forceinline__ uint32_t fold16_col(uint32_t lane) {
+  return (lane >> 5) | ((lane >> 3) & 2u) | ((lane >> 1) & 4u) | ((lane << 1) & 8u);
 }
 
-// Add one term (this lane's four values; lanes without a term pass zeros).
-// Called only where some lane has a term (wave-uniform).
-__device__ __forceinline__ void ev_add(EvBuf &b, const AdjWalk &a, double x, double y, double z,
-                                       double w, uint32_t tag) {
-  const uint32_t lane = threadIdx.x & 63;
-  double *row = b.v[lane] + 4 * b.n;
-  row[0] = x;
-  row[1] = y;
-  row[2] = z;
-  row[3] = w;
-  if (lane == 0) b.tag[b.n] = tag;
-  if (++b.n == (uint32_t)EV) ev_flush(b, a);
+template <class Rec>
+__device__ __forceinline__ Rec adj_rec(const Rec *nodes_m1, uint32_t off) {
+  typedef uint32_t words __attribute__((ext_vector_type(sizeof(Rec) / 4)));
+  const words w =
+      *reinterpret_cast<const words *>(reinterpret_cast<const char *>(nodes_m1) + uni_a(off));
+  Rec r;
+  __builtin_memcpy(&r, &w, sizeof(Rec));
+  return r;
 }
 
 template <bool MIXED>
-__global__ __launch_bounds__(ADJ_THREADS) void k_adj_walk(AdjWalk a) {
+struct AdjForm {
+  using Rec = NodeRec64;
+  using Body = double4;
+  __device__ static const Rec *nodes(const AdjWalk &a) { return a.rec64 - 1; }
+  __device__ static const Body *bodies(const AdjWalk &a) { return a.pos64; }
+};
+template <>
+struct AdjForm<true> {
+  using Rec = NodeRec32;
+  using Body = float4;
+  __device__ static const Rec *nodes(const AdjWalk &a) { return a.rec32 - 1; }
+  __device__ static const Body *bodies(const AdjWalk &a) { return a.pos32; }
+};
+
+// Positions in the tree are byte offsets h RS of the records, and a lane's
+// acceptance level is kept as in the forward walk (kd_traverse.hip).
+template <bool MIXED, int S>
+__global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
 #pragma clang fp contract(off)
-  __shared__ __align__(16) double ev_v[ADJ_THREADS / 64][64][EV_ROW];
-  __shared__ uint32_t ev_t[ADJ_THREADS / 64][EV];
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wbase = (xcd_block() * blockDim.x + threadIdx.x) & ~63u;
-  if (wbase >= a.n) return;
+  using F = AdjForm<MIXED>;
+  using Rec = typename F::Rec;
+  using Body = typename F::Body;
+  constexpr uint32_t RS = sizeof(Rec);
+  constexpr int RSL = RS == 32 ? 5 : 6;
+  constexpr int BATCH = 4;  // leaf bodies whose reactions are summed together
+  const Rec *nodes = F::nodes(a);
+  const Body *bodies = F::bodies(a);
+  const uint32_t wbase = xcd_block() * 64u, lane = threadIdx.x & 63;
+  const uint32_t w = uni_a(threadIdx.x >> 6);
   const uint32_t me = wbase + lane;
   const bool valid = me < a.n;
   const uint32_t ms = valid ? me : wbase;
-  const double4 p = a.pos64[ms];
-  const float4 pf = a.pos32[ms];
+  const Body p = bodies[ms];
   const uint32_t o = a.oid[ms];
   const double ux = valid ? a.ux[o] : 0.0, uy = valid ? a.uy[o] : 0.0,
                uz = valid ? a.uz[o] : 0.0;
   const float uxf = (float)ux, uyf = (float)uy, uzf = (float)uz;
   double sx = 0.0, sy = 0.0, sz = 0.0;
-  int D = valid ? 0x7fffffff : -1;
-  EvBuf eb;
-  eb.v = ev_v[threadIdx.x >> 6];
-  eb.tag = ev_t[threadIdx.x >> 6];
-  eb.n = 0;
-  uint32_t h = 1;
-  int depth = 0;
-  while (h != 0) {
-    const NodeRec64 r = a.rec64[uni_a(h) - 1];
-    const bool active = depth <= D;
-    if (r.count <= a.leaf) {
-      for (uint32_t jj = 0; jj < r.count; ++jj) {
-        const uint32_t j = r.start + jj;
-        const bool use = active && j != me;
-        double gx = 0.0, gy = 0.0, gz = 0.0, gm = 0.0;
-        if (use) {
-          if (MIXED) {
-            const float4 q = a.pos32[j];
-            float fx, fy, fz, fm;
-            vjp32(pf.x - q.x, pf.y - q.y, pf.z - q.z, q.w, uxf, uyf, uzf, fx, fy, fz, fm);
-            gx = fx, gy = fy, gz = fz, gm = fm;
-          } else {
-            const double4 q = a.pos64[j];
-            vjp64(p.x - q.x, p.y - q.y, p.z - q.z, q.w, ux, uy, uz, gx, gy, gz, gm);
-          }
-          sx += gx;
-          sy += gy;
-          sz += gz;
-        }
-        if (__any(use)) ev_add(eb, a, -gx, -gy, -gz, gm, uni_a(a.oid[j]));
-      }
-      h = heap_next_a(h, depth);
-      continue;
+  int E = valid ? -RSL : 32 - RSL;
+  const uint32_t col4 = fold4_col(lane), col16 = fold16_col(lane);
+
+  // one term of a lane that takes it (use), 0 otherwise: the lane's own sum,
+  // and the reaction v
+  auto term = [&](auto dx, auto dy, auto dz, auto d2, auto m, bool use, double v[4]) {
+    double gx, gy, gz, gm;
+    if constexpr (MIXED) {
+      float fx, fy, fz, fm;
+      vjp32(dx, dy, dz, d2, m, uxf, uyf, uzf, fx, fy, fz, fm);
+      gx = use ? fx : 0.f, gy = use ? fy : 0.f, gz = use ? fz : 0.f, gm = use ? fm : 0.f;
+    } else {
+      vjp64(dx, dy, dz, d2, m, ux, uy, uz, gx, gy, gz, gm);
+      gx = use ? gx : 0.0, gy = use ? gy : 0.0, gz = use ? gz : 0.0, gm = use ? gm : 0.0;
     }
+    sx += gx;
+    sy += gy;
+    sz += gz;
+    v[0] = -gx, v[1] = -gy, v[2] = -gz, v[3] = gm;
+  };
+  auto inner = [&](const Rec &r, uint32_t h, int lz, bool mine) {
+    const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
+    const auto dx = p.x - r.cx, dy = p.y - r.cy, dz = p.z - r.cz;
+    const auto d2 = dx * dx + dy * dy + dz * dz;
     bool ok;
-    double dx, dy, dz;
-    float fdx = 0.f, fdy = 0.f, fdz = 0.f;
-    if (MIXED) {
-      const NodeRec32 q = a.rec32[h - 1];
-      fdx = pf.x - q.cx;
-      fdy = pf.y - q.cy;
-      fdz = pf.z - q.cz;
-      const float d2 = fdx * fdx + fdy * fdy + fdz * fdz;
-      ok = q.size2 < d2;  // size^2 / theta^2 < d2, as the forward walk
-      dx = dy = dz = 0.0;
-    } else {
-      dx = p.x - r.cx;
-      dy = p.y - r.cy;
-      dz = p.z - r.cz;
-      const double d2 = dx * dx + dy * dy + dz * dz;
+    if constexpr (MIXED)
+      ok = r.size2 < d2;  // size^2 / theta^2 < d2, as the forward walk
+    else
       ok = r.size2 < a.theta2 * d2;
+    const uint64_t tm = actm & __builtin_amdgcn_ballot_w64(ok);
+    const uint64_t om = actm & ~tm;
+    if (mine && tm) {
+      double v[4];
+      term(dx, dy, dz, d2, r.m, __builtin_amdgcn_inverse_ballot_w64(tm), v);
+      const double s = fold4(v);
+      if ((lane & 15u) == 0) atomicAdd(a.gnode + 4 * (size_t)(h / RS - 1) + col4, s);
     }
-    const bool take = active && ok;
-    const bool open = active && !ok;
-    double gx = 0.0, gy = 0.0, gz = 0.0, gm = 0.0;
-    if (take) {
-      if (MIXED) {
-        float fx, fy, fz, fm;
-        vjp32(fdx, fdy, fdz, (float)r.m, uxf, uyf, uzf, fx, fy, fz, fm);
-        gx = fx, gy = fy, gz = fz, gm = fm;
-      } else {
-        vjp64(dx, dy, dz, r.m, ux, uy, uz, gx, gy, gz, gm);
+    E = __builtin_amdgcn_inverse_ballot_w64(om) ? -RSL : max(E, lz);
+    return om ? 2 * h : r.skip;
+  };
+  auto leaf = [&](const Rec &r, int lz) {
+    const bool active = lz >= E;
+    for (uint32_t b = 0; b < r.count; b += BATCH) {
+      const uint32_t j0 = r.start + b, m = min((uint32_t)BATCH, r.count - b);
+      Body q[BATCH];  // past the leaf: still inside the padded body arrays
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) q[i] = bodies[j0 + i];
+      double v[4 * BATCH];
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) {
+        if ((uint32_t)i < m) {  // wave-uniform
+          const auto dx = p.x - q[i].x, dy = p.y - q[i].y, dz = p.z - q[i].z;
+          auto d2 = dx * dx + dy * dy + dz * dz;
+          if constexpr (MIXED) d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
+          term(dx, dy, dz, d2, q[i].w, active && j0 + i != me, v + 4 * i);
+        } else {
+          v[4 * i] = v[4 * i + 1] = v[4 * i + 2] = v[4 * i + 3] = 0.0;
+        }
       }
-      sx += gx;
-      sy += gy;
-      sz += gz;
+      const double s = fold16(v, lane);
+      if ((lane & 3u) == 0 && col16 < 4 * m) atomicAdd(a.react + 4 * (size_t)j0 + col16, s);
     }
-    if (__any(take)) ev_add(eb, a, -gx, -gy, -gz, gm, (h - 1) | EV_NODE);
-    D = take ? depth : (open ? 0x7fffffff : D);
-    if (__any(open)) {
-      h = 2 * h;
-      ++depth;
+  };
+
+  uint32_t h = RS, parts = 0;
+  bool mine = w == 0;
+  do {
+    const int lz = __builtin_clz(h);
+    if (lz == lzd) {
+      mine = (parts++ & (S - 1u)) == w;
+      uint32_t x = h / RS;
+      x >>= __builtin_ctz(~x);
+      const uint32_t next = x == 0 ? 0 : (x + 1) * RS;
+      if (mine) {
+        do {
+          const Rec r = adj_rec(nodes, h);
+          const int l = __builtin_clz(h);
+          if (r.count <= a.leaf) {
+            leaf(r, l);
+            h = r.skip;
+          } else {
+            h = inner(r, h, l, true);
+          }
+        } while (h != next);
+      }
+      h = next;
     } else {
-      h = heap_next_a(h, depth);
+      h = inner(adj_rec(nodes, h), h, lz, mine);
     }
-  }
-  if (eb.n) ev_flush(eb, a);
+  } while (h != 0);
   if (valid) {
-    atomicAdd(a.lpx + o, sx);
-    atomicAdd(a.lpy + o, sy);
-    atomicAdd(a.lpz + o, sz);
+    atomicAdd(a.react + 4 * (size_t)me, sx);
+    atomicAdd(a.react + 4 * (size_t)me + 1, sy);
+    atomicAdd(a.react + 4 * (size_t)me + 2, sz);
   }
 }
 
-// Node terms to the members.  One thread per heap slot that is a leaf: the
-// sums over its internal ancestors of A = G/M and B = H - c.A give
-//   lp_j += m_j A,  lm_j += p_j . A + B  for every member j.
-__global__ void k_adj_nodes(const uint32_t *__restrict__ seg_count,
-                            const NodeRec64 *__restrict__ rec64,
-                            const double4 *__restrict__ pos64, const uint32_t *__restrict__ oid,
-                            const double *__restrict__ gx, const double *__restrict__ gy,
-                            const double *__restrict__ gz, const double *__restrict__ gh,
-                            uint32_t slots, uint32_t leaf, double *lpx, double *lpy, double *lpz,
-                            double *lm) {
+// The step's reactions to the bodies' adjoints, with the node terms: one
+// thread per heap slot that is a leaf.  The sums over its ancestors of
+// A = G/M and B = H - c.A give  lp_j += m_j A,  lm_j += p_j . A + B  for every
+// member j.  (The ancestors' slots are known beforehand, so four are loaded at
+// a time.)
+__global__ __launch_bounds__(256) void k_adj_nodes(
+    const uint32_t *__restrict__ seg_count, const NodeRec64 *__restrict__ rec64,
+    const double4 *__restrict__ pos64, const uint32_t *__restrict__ oid,
+    const double4 *__restrict__ gnode, const double4 *__restrict__ react, uint32_t slots,
+    uint32_t leaf, double *lpx, double *lpy, double *lpz, double *lm) {
 #pragma clang fp contract(off)
   const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= slots) return;
@@ -256,34 +316,48 @@ __global__ void k_adj_nodes(const uint32_t *__restrict__ seg_count,
   if (h > 0 && seg_count[(h - 1) / 2] <= leaf) return;  // below a leaf: unused slot
   double ax = 0.0, ay = 0.0, az = 0.0, b = 0.0;
   for (uint32_t q = h; q > 0;) {
-    q = (q - 1) / 2;
-    if (gx[q] == 0.0 && gy[q] == 0.0 && gz[q] == 0.0 && gh[q] == 0.0) continue;
-    const NodeRec64 r = rec64[q];
-    const double Ax = gx[q] / r.m, Ay = gy[q] / r.m, Az = gz[q] / r.m;
-    ax += Ax;
-    ay += Ay;
-    az += Az;
-    b += gh[q] - (r.cx * Ax + r.cy * Ay + r.cz * Az);
+    double4 g[4];
+    NodeRec64 r[4];
+    bool use[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      use[i] = q > 0;
+      q = q > 0 ? (q - 1) / 2 : 0;
+      g[i] = gnode[q];
+      r[i] = rec64[q];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!use[i] || (g[i].x == 0.0 && g[i].y == 0.0 && g[i].z == 0.0 && g[i].w == 0.0)) continue;
+      const double Ax = g[i].x / r[i].m, Ay = g[i].y / r[i].m, Az = g[i].z / r[i].m;
+      ax += Ax;
+      ay += Ay;
+      az += Az;
+      b += g[i].w - (r[i].cx * Ax + r[i].cy * Ay + r[i].cz * Az);
+    }
   }
-  if (ax == 0.0 && ay == 0.0 && az == 0.0 && b == 0.0) return;
   const NodeRec64 lr = rec64[h];
   for (uint32_t t = lr.start; t < lr.start + lr.count; ++t) {
-    const double4 p = pos64[t];
+    const double4 p = pos64[t], v = react[t];
     const uint32_t o = oid[t];
-    lpx[o] += p.w * ax;
-    lpy[o] += p.w * ay;
-    lpz[o] += p.w * az;
-    lm[o] += p.x * ax + p.y * ay + p.z * az + b;
+    lpx[o] += p.w * ax + v.x;
+    lpy[o] += p.w * ay + v.y;
+    lpz[o] += p.w * az + v.z;
+    lm[o] += p.x * ax + p.y * ay + p.z * az + b + v.w;
   }
 }
 
-// lv += dt lp;  u = dt lv  (original order).
-__global__ void k_adj_integrate(double *lpx, double *lpy, double *lpz, double *lvx, double *lvy,
-                                double *lvz, double *ux, double *uy, double *uz, uint32_t n,
-                                double dt) {
+// lv += dt lp;  u = dt lv  (original order); clears the step's reactions and
+// node adjoints.
+__global__ void k_adj_begin(double *lpx, double *lpy, double *lpz, double *lvx, double *lvy,
+                            double *lvz, double *ux, double *uy, double *uz, uint32_t n, double dt,
+                            double4 *react, double4 *gnode, uint32_t slots) {
 #pragma clang fp contract(off)
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const double4 zero = make_double4(0.0, 0.0, 0.0, 0.0);
+  if (i < slots) gnode[i] = zero;
   if (i >= n) return;
+  react[i] = zero;
   double a = lvx[i] + dt * lpx[i], b = lvy[i] + dt * lpy[i], c = lvz[i] + dt * lpz[i];
   lvx[i] = a;
   lvy[i] = b;
@@ -293,55 +367,49 @@ __global__ void k_adj_integrate(double *lpx, double *lpy, double *lpz, double *l
   uz[i] = dt * c;
 }
 
-__global__ void k_zero(double *p, size_t count) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-       i += (size_t)gridDim.x * blockDim.x)
-    p[i] = 0.0;
+// The depth of the subtrees dealt to the wavefronts of a workgroup (0: one
+// wavefront).  Backward of a step (with its recomputed forward, 630 us at
+// 100,000 ring bodies, 410 at 10,000, 165 at 2,000) in us at depths 0, 3, 4, 5,
+// 6: mixed 1835, 1734, 1541, 1579, 1754 at 100,000 and 1087, 921, 726, 615, 586
+// at 10,000; FP64 574, 439, 346, 292, 283 at 2,000.
+static int adj_depth(uint32_t n) { return n <= 16384 ? 6 : n <= 65536 ? 5 : n <= 200000 ? 4 : 0; }
+
+template <bool MIXED>
+static void launch_adj_walk(const AdjWalk &a, int levels, hipStream_t s) {
+  const unsigned groups = (a.n + 63) / 64;
+  int d = adj_depth(a.n);
+  if (d > levels - 2) d = levels - 2;  // every node above the depth is internal
+  if (d < 3) d = 0;
+  const int lzd = 31 - (MIXED ? 5 : 6) - d;
+  if (d == 0)
+    k_adj_walk<MIXED, 1><<<groups, 64, 0, s>>>(a, lzd);
+  else if (d == 3)
+    k_adj_walk<MIXED, 2><<<groups, 128, 0, s>>>(a, lzd);
+  else if (d == 4)
+    k_adj_walk<MIXED, 4><<<groups, 256, 0, s>>>(a, lzd);
+  else if (d == 5)
+    k_adj_walk<MIXED, 8><<<groups, 512, 0, s>>>(a, lzd);
+  else
+    k_adj_walk<MIXED, 16><<<groups, 1024, 0, s>>>(a, lzd);
 }
 
 hipError_t launch_adj_step(const AdjStep &st, hipStream_t s) {
-  const uint32_t n = st.n;
-  const unsigned nb = (n + 255) / 256;
-  k_adj_integrate<<<nb, 256, 0, s>>>(st.lp[0], st.lp[1], st.lp[2], st.lv[0], st.lv[1], st.lv[2],
-                                     st.u[0], st.u[1], st.u[2], n, st.dt);
-  const size_t zc = 4 * (size_t)st.slots;
-  k_zero<<<(unsigned)std::min<size_t>((zc + 255) / 256, 4096), 256, 0, s>>>(st.gnode, zc);
-  AdjWalk a;
-  a.rec64 = st.rec64;
-  a.rec32 = st.rec32;
-  a.pos64 = st.pos64;
-  a.pos32 = st.pos32;
-  a.oid = st.oid;
-  a.ux = st.u[0];
-  a.uy = st.u[1];
-  a.uz = st.u[2];
-  a.lpx = st.lp[0];
-  a.lpy = st.lp[1];
-  a.lpz = st.lp[2];
-  a.lm = st.lm;
-  a.gx = st.gnode;
-  a.gy = st.gnode + st.slots;
-  a.gz = st.gnode + 2 * (size_t)st.slots;
-  a.gh = st.gnode + 3 * (size_t)st.slots;
-  a.body[0] = a.lpx;
-  a.body[1] = a.lpy;
-  a.body[2] = a.lpz;
-  a.body[3] = a.lm;
-  a.node[0] = a.gx;
-  a.node[1] = a.gy;
-  a.node[2] = a.gz;
-  a.node[3] = a.gh;
-  a.n = n;
-  a.leaf = st.leaf;
-  a.theta2 = st.theta * st.theta;
-  const unsigned wb = (n + ADJ_THREADS - 1) / ADJ_THREADS;
+  const uint32_t n = st.n, work = std::max(n, st.slots);
+  double4 *react = reinterpret_cast<double4 *>(st.react);
+  double4 *gnode = reinterpret_cast<double4 *>(st.gnode);
+  k_adj_begin<<<(work + 255) / 256, 256, 0, s>>>(st.lp[0], st.lp[1], st.lp[2], st.lv[0], st.lv[1],
+                                                 st.lv[2], st.u[0], st.u[1], st.u[2], n, st.dt,
+                                                 react, gnode, st.slots);
+  const AdjWalk a{st.rec64, st.rec32, st.pos64, st.pos32, st.oid, st.u[0], st.u[1], st.u[2],
+                  st.react, st.gnode, n, st.leaf, st.theta * st.theta};
+  const int levels = make_shape(n, (int)st.leaf).levels;
   if (st.mixed)
-    k_adj_walk<true><<<wb, ADJ_THREADS, 0, s>>>(a);
+    launch_adj_walk<true>(a, levels, s);
   else
-    k_adj_walk<false><<<wb, ADJ_THREADS, 0, s>>>(a);
+    launch_adj_walk<false>(a, levels, s);
   k_adj_nodes<<<(st.slots + 255) / 256, 256, 0, s>>>(st.seg_count, st.rec64, st.pos64, st.oid,
-                                                     a.gx, a.gy, a.gz, a.gh, st.slots, st.leaf,
-                                                     st.lp[0], st.lp[1], st.lp[2], st.lm);
+                                                     gnode, react, st.slots, st.leaf, st.lp[0],
+                                                     st.lp[1], st.lp[2], st.lm);
   return hipGetLastError();
 }
 

@@ -1687,7 +1687,7 @@ struct kd_adj {
   int64_t slots = 0;
   double *lp[3] = {nullptr, nullptr, nullptr}, *lv[3] = {nullptr, nullptr, nullptr},
          *u[3] = {nullptr, nullptr, nullptr};
-  double *lm = nullptr, *gnode = nullptr;
+  double *lm = nullptr, *react = nullptr, *gnode = nullptr;
   std::vector<void *> allocs;
   bool forward_done = false;
 };
@@ -1730,7 +1730,6 @@ extern "C" int kd_adj_create(int64_t n, int64_t steps, int64_t every, const kd_p
     g_err = msg;
     return rc;
   }
-  a->c->extra_recs = REC_64 | REC_32;  // the reverse sweep reads both
   a->n = n;
   a->steps = steps;
   a->every = std::min(every, steps);
@@ -1745,11 +1744,18 @@ extern "C" int kd_adj_create(int64_t n, int64_t steps, int64_t every, const kd_p
   };
   if ((rc = adj_alloc(a, &a->ck, (size_t)a->nck * 7 * N)) ||
       (rc = adj_alloc(a, &a->ck_oid, (size_t)a->nck * N)) ||
-      (rc = adj_alloc(a, &a->t_pos64, E * N)) || (rc = adj_alloc(a, &a->t_pos32, E * N)) ||
+      (rc = adj_alloc(a, &a->t_pos64, E * N + BODY_PAD)) ||
+      (rc = adj_alloc(a, &a->t_pos32, E * N + BODY_PAD)) ||
       (rc = adj_alloc(a, &a->t_oid, E * N)) || (rc = adj_alloc(a, &a->t_rec64, E * S)) ||
       (rc = adj_alloc(a, &a->t_rec32, E * S)) || (rc = adj_alloc(a, &a->lm, N)) ||
-      (rc = adj_alloc(a, &a->gnode, 4 * S)))
+      (rc = adj_alloc(a, &a->react, 4 * N)) || (rc = adj_alloc(a, &a->gnode, 4 * S)))
     return bail(rc);
+  // body loads past a leaf reach the next slot or the padding: finite values
+  if (hipMemset(a->t_pos64, 0, sizeof(double4) * (E * N + BODY_PAD)) != hipSuccess ||
+      hipMemset(a->t_pos32, 0, sizeof(float4) * (E * N + BODY_PAD)) != hipSuccess) {
+    fail(KD_ERR_HIP, "clearing the tape failed");
+    return bail(KD_ERR_HIP);
+  }
   for (int d = 0; d < 3; ++d)
     if ((rc = adj_alloc(a, &a->lp[d], N)) || (rc = adj_alloc(a, &a->lv[d], N)) ||
         (rc = adj_alloc(a, &a->u[d], N)))
@@ -1784,13 +1790,18 @@ static int adj_restore(kd_adj *a, int64_t slot) {
   return KD_OK;
 }
 
-static int adj_step_forward(kd_adj *a) {
+// The rest of a step whose tree is built: the walk advances the bodies as it
+// finishes them and leaves the range that the next step's build takes (as
+// kd_step does).
+static int adj_advance(kd_adj *a) {
   kd_ctx *c = a->c;
-  int rc = build_impl(c);
-  if (rc) return rc;
-  if ((rc = traverse_impl(c))) return rc;
-  HIP_TRY(launch_kick_drift(c->st[c->cur], c->acc[0], c->acc[1], c->acc[2], (uint32_t)c->n,
-                            c->params.dt, c->bad, c->stream));
+  const uint32_t n = (uint32_t)c->n;
+  const bool range = !one_segment(c->forest);
+  const KickDrift kd{c->st[c->cur], c->params.dt, c->bad, range ? c->wave_range : nullptr};
+  HIP_TRY(launch_traverse_kick(c->params.precision, c->traverse_variant, c->tree, c->pos64,
+                               c->pos32, n, c->params.theta, c->params.leaf_size, kd, c->stream));
+  if (range)
+    HIP_TRY(launch_range_from_waves(c->wave_range, (n + 63) / 64, c->b.range, c->stream));
   return KD_OK;
 }
 
@@ -1809,7 +1820,7 @@ extern "C" int kd_adj_forward(kd_adj *a, const double *x0, const double *y0, con
   HIP_TRY(hipMemsetAsync(c->bad, 0, sizeof(int), c->stream));
   for (int64_t k = 0; k < a->steps; ++k) {
     if (k % a->every == 0 && (rc = adj_save(a, k / a->every))) return rc;
-    if ((rc = adj_step_forward(a))) return rc;
+    if ((rc = build_impl(c, k > 0)) || (rc = adj_advance(a))) return rc;
   }
   int bad = 0;
   HIP_TRY(hipMemcpyAsync(&bad, c->bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -1843,24 +1854,31 @@ extern "C" int kd_adj_backward(kd_adj *a, const double *gpx, const double *gpy, 
     const int64_t k0 = seg * a->every;
     const int64_t len = std::min(a->every, a->steps - k0);
     if ((rc = adj_restore(a, seg))) return rc;
-    for (int64_t j = 0; j < len; ++j) {
-      if ((rc = build_impl(c))) return rc;
-      HIP_TRY(hipMemcpyAsync(a->t_pos64 + j * N, c->pos64, 32 * N, hipMemcpyDeviceToDevice,
-                             c->stream));
-      HIP_TRY(hipMemcpyAsync(a->t_pos32 + j * N, c->pos32, 16 * N, hipMemcpyDeviceToDevice,
-                             c->stream));
-      HIP_TRY(hipMemcpyAsync(a->t_oid + j * N, c->st[c->cur].oid, 4 * N,
-                             hipMemcpyDeviceToDevice, c->stream));
-      HIP_TRY(hipMemcpyAsync(a->t_rec64 + j * S, c->tree.rec64, sizeof(NodeRec64) * S,
-                             hipMemcpyDeviceToDevice, c->stream));
-      HIP_TRY(hipMemcpyAsync(a->t_rec32 + j * S, c->tree.rec32, sizeof(NodeRec32) * S,
-                             hipMemcpyDeviceToDevice, c->stream));
-      if (j + 1 < len) {
-        if ((rc = traverse_impl(c))) return rc;
-        HIP_TRY(launch_kick_drift(c->st[c->cur], c->acc[0], c->acc[1], c->acc[2],
-                                  (uint32_t)c->n, c->params.dt, c->bad, c->stream));
-      }
+    // the segment's steps again, each building its records and body arrays
+    // in its own slot of the tape
+    const TreeDev tree = c->tree;
+    double4 *const pos64 = c->pos64;
+    float4 *const pos32 = c->pos32;
+    c->extra_recs = REC_64;  // the node terms are carried in FP64
+    rc = KD_OK;
+    for (int64_t j = 0; j < len && rc == KD_OK; ++j) {
+      c->tree.rec64 = a->t_rec64 + j * S;
+      c->tree.rec32 = a->t_rec32 + j * S;
+      c->pos64 = a->t_pos64 + j * N;
+      c->pos32 = a->t_pos32 + j * N;
+      if ((rc = build_impl(c, j > 0))) break;
+      if (hipMemcpyAsync(a->t_oid + j * N, c->st[c->cur].oid, 4 * N, hipMemcpyDeviceToDevice,
+                         c->stream) != hipSuccess)
+        rc = fail(KD_ERR_HIP, "recording a step failed");
+      else if (j + 1 < len)
+        rc = adj_advance(a);
     }
+    c->tree = tree;
+    c->pos64 = pos64;
+    c->pos32 = pos32;
+    c->extra_recs = 0;
+    c->has_tree = false;  // the last tree's records are the tape's
+    if (rc) return rc;
     for (int64_t j = len - 1; j >= 0; --j) {
       AdjStep st;
       st.rec64 = a->t_rec64 + j * S;
@@ -1875,6 +1893,7 @@ extern "C" int kd_adj_backward(kd_adj *a, const double *gpx, const double *gpy, 
         st.u[d] = a->u[d];
       }
       st.lm = a->lm;
+      st.react = a->react;
       st.gnode = a->gnode;
       st.n = (uint32_t)N;
       st.slots = (uint32_t)S;

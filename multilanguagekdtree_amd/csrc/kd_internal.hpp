@@ -358,6 +358,7 @@ struct AdjStep {
   const uint32_t *seg_count;
   double *lp[3], *lv[3], *u[3];
   double *lm;
+  double *react;  // 4 * n: d/dp (x, y, z) and d/dm per tree position
   double *gnode;  // 4 * slots: d/dc (x, y, z) and d/dM per node
   uint32_t n, slots, leaf;
   double theta, dt;
