@@ -354,6 +354,7 @@ static int create_impl(kd_ctx *c, int64_t cap, const Sizing &z) {
   HIP_TRY(hipMemsetAsync(c->pos64, 0, sizeof(double4) * (N + BODY_PAD), c->stream));
   HIP_TRY(hipMemsetAsync(c->pos32, 0, sizeof(float4) * (N + BODY_PAD), c->stream));
   ALLOC(c->allocs, c->b.cnt, z.cnt_entries);
+  ALLOC(c->allocs, c->b.words, z.nsys == 1 ? level_words(z.cnt_entries) : 1);
   ALLOC(c->allocs, c->dsys, z.nsys);
   ALLOC(c->allocs, c->dsys_mid, z.nsys);
   c->dmid_cap = mid_tasks_max(cap, z.nsys);
@@ -537,7 +538,7 @@ static int build_impl(kd_ctx *c, bool range_ready = false) {
   if (mid && c->forest.n_mid_tasks > 0) ++c->mid_builds;
   HIP_TRY(launch_build(c->forest, c->params.leaf_size, c->st[c->cur], c->st[nxt], c->tree, c->b,
                        c->pos64, c->pos32, c->params.theta, c->stream, range_ready, lazy,
-                       report, mid));
+                       report, c->tree_order, c->mid_levels));
   if (report) {
     // a system of one segment has no device-wide split, so any dimension may
     // be skipped there
@@ -554,7 +555,7 @@ static int build_impl(kd_ctx *c, bool range_ready = false) {
         ++c->lazy_redos;
         HIP_TRY(launch_build(c->forest, c->params.leaf_size, c->st[c->cur], c->st[nxt], c->tree,
                              c->b, c->pos64, c->pos32, c->params.theta, c->stream, true, 3,
-                             true, mid));
+                             true, c->tree_order, c->mid_levels));
         HIP_TRY(hipEventSynchronize(c->b.ev_viol));
         unsafe = *c->b.viol_host;
         full = true;
@@ -1248,7 +1249,7 @@ static int batch_step_enqueue(kd_batch *b, int lazy) {
   // eagerly with the kernel-by-kernel levels)
   HIP_TRY(launch_build(c->forest, c->params.leaf_size, c->st[c->cur], c->st[nxt], c->tree, c->b,
                        c->pos64, c->pos32, c->params.theta, c->stream, true, lazy, b->lazy_on,
-                       c->mid_levels && c->tree_order));
+                       c->tree_order, c->mid_levels));
   c->cur = nxt;
   c->has_tree = true;
   c->tree_order = true;

@@ -441,20 +441,20 @@ struct ListBufs {
   __device__ uint32_t *out(uint32_t m, int d) const { return ((m >> d) & 1u) ? A.l[d] : B.l[d]; }
 };
 
-// A run of equal keys straddles the median of segment h (list ls of its
-// split dimension, [s, s + c)): the run's members that go left are those
-// with the smallest original indices.  The block radix-selects the threshold
-// index (the original index of the first body that goes right)
-// and stably partitions the run (scratch = the same list's output buffer,
-// not live for this node).
+// A run of equal keys straddles the median of a segment (list ls of its split
+// dimension, [s, s + c)): the run's members that go left are those with the
+// smallest original indices.  tie_threshold finds the run [r0, r1) and the
+// threshold (the original index of the first body that goes right) by a radix
+// selection; tie_fix also partitions the run stably (tmp = the same list's
+// output buffer, not live for this node).
 template <int NT>
-__device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
-                        const uint32_t *__restrict__ oid, uint32_t s, uint32_t c) {
+__device__ uint32_t tie_threshold(const uint32_t *ls, const double *key,
+                                  const uint32_t *__restrict__ oid, uint32_t s, uint32_t c,
+                                  uint32_t &r0, uint32_t &r1) {
   const uint32_t mid = s + c / 2;
   const double kv = key[ls[mid]];
   __shared__ uint32_t r0s, r1s, need_s, prefix_s, mask_s;
   __shared__ uint32_t hist[256];
-  __shared__ uint32_t scan_sh[NT / 64];
   if (threadIdx.x == 0) {
     // keys are sorted non-decreasing inside [s, s+c)
     uint32_t lo = s, hi = mid;  // first position with key == kv
@@ -462,21 +462,22 @@ __device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
       uint32_t m = lo + (hi - lo) / 2;
       if (key[ls[m]] < kv) lo = m + 1; else hi = m;
     }
-    uint32_t r0 = lo;
+    const uint32_t first = lo;
     lo = mid + 1;
     hi = s + c;  // first position with key > kv
     while (lo < hi) {
       uint32_t m = lo + (hi - lo) / 2;
       if (key[ls[m]] > kv) hi = m; else lo = m + 1;
     }
-    r0s = r0;
+    r0s = first;
     r1s = lo;
-    need_s = mid - r0;
+    need_s = mid - first;
     prefix_s = 0;
     mask_s = 0;
   }
   __syncthreads();
-  const uint32_t r0 = r0s, r1 = r1s;
+  r0 = r0s;
+  r1 = r1s;
   for (int shift = 24; shift >= 0; shift -= 8) {
     for (int i = threadIdx.x; i < 256; i += NT) hist[i] = 0;
     __syncthreads();
@@ -498,8 +499,16 @@ __device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
     }
     __syncthreads();
   }
-  const uint32_t thr_oid = prefix_s;  // original index of the first body that goes right
-  uint32_t nleft = mid - r0;
+  return prefix_s;
+}
+
+template <int NT>
+__device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
+                        const uint32_t *__restrict__ oid, uint32_t s, uint32_t c) {
+  __shared__ uint32_t scan_sh[NT / 64];
+  uint32_t r0, r1;
+  const uint32_t thr_oid = tie_threshold<NT>(ls, key, oid, s, c, r0, r1);
+  uint32_t nleft = s + c / 2 - r0;
   uint32_t off_l = 0, off_r = nleft;
   for (uint32_t base = r0; base < r1; base += NT) {
     uint32_t p = base + threadIdx.x;
@@ -545,13 +554,15 @@ __device__ __forceinline__ int split_dim_of(const double e[3]) {
 // With viol set and lazy == 3, the block reports every dimension d that the
 // rule would pick with its extent raised to its global extent.
 constexpr int SPLIT_THREADS = 256;
-// The split of segment h ([s, s + c) of its lists, list-buffer mask m): the
-// node's dimension, value and size, the children's masks, and whether equal
-// keys straddle the median (the caller then orders that run).
+// The split of segment h ([s, s + c) of its lists, list-buffer mask m): its
+// dimension and value kv, whether equal keys straddle the median (the caller
+// then orders that run), and, where `write` is set, the node's dimension,
+// value and size, the children's masks and the report.
 __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P, const TreeDev &t,
                                             uint32_t h, uint32_t s, uint32_t c, uint32_t m,
                                             const unsigned long long *range, int lazy,
-                                            uint32_t *viol, bool &tie) {
+                                            uint32_t *viol, bool &tie, bool write,
+                                            double &kv) {
   double ext[3], glob[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -567,12 +578,12 @@ __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P,
   }
   int sd;
   if (lazy < 3) {
-    if (split_dim_of(ext) == lazy) atomicOr(viol, 1u << lazy);
+    if (write && split_dim_of(ext) == lazy) atomicOr(viol, 1u << lazy);
     ext[lazy] = -1.0;
     sd = split_dim_of(ext);
   } else {
     sd = split_dim_of(ext);
-    if (viol != nullptr) {
+    if (write && viol != nullptr) {
       uint32_t unsafe = 0;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
@@ -584,15 +595,16 @@ __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P,
     }
   }
   const uint32_t mid = s + c / 2;
-  const double kv = P.c[sd][LB.in(m, sd)[mid]];
+  kv = P.c[sd][LB.in(m, sd)[mid]];
   const double kp = P.c[sd][LB.in(m, sd)[mid - 1]];
+  tie = kp == kv;
+  if (!write) return sd;
   const uint8_t cm = (uint8_t)(m ^ (7u ^ (1u << sd)));
   t.lmask[2 * h + 1] = cm;
   t.lmask[2 * h + 2] = cm;
   t.split_dim[h] = (uint8_t)sd;
   t.split_val[h] = kv;
   t.size[h] = ext[sd];
-  tie = kp == kv;
   return sd;
 }
 
@@ -612,7 +624,8 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_level_split(ListBufs LB, Coor
   __shared__ int sd_s, tie_s;
   if (threadIdx.x == 0) {
     bool tie;
-    sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie);
+    double kv;
+    sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, true, kv);
     tie_s = tie;
   }
   __syncthreads();
@@ -805,6 +818,154 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_scatter(ListBufs LB,
   }
 }
 
+// A single system's device-wide level in two launches.  The six kernels above
+// are mostly launches and waits in systems of up to a million bodies (22 us a
+// level at 100,000; these take 11).  k_level_mark: every tile decides its
+// segment's split for itself, marks the bodies of the lists that move by their
+// coordinates against the split value (a bit a position) and counts its lefts.  k_level_move: every tile adds up the counts of the
+// tiles before it and places its bodies.  Where equal keys straddle the
+// median, a tile of the first launch finds the threshold index for itself, and
+// the segment's first tile of the second orders the run.
+// From an upload's order the coordinates of a larger system's list entries are
+// gathered from all of memory, and the packed flags of the split list are
+// cheaper.  Builds in us, six kernels a level / two, ring: 175 / 159 at 5,000,
+// 303 / 242 at 100,000, 597 / 504 at 1 M, 2773 / 2683 at 10 M from tree order;
+// first build after an upload 624 / 570 at 300,000, 1090 / 1065 at 1 M, 2440 /
+// 2600 at 3 M, 8340 / 9309 at 10 M.
+constexpr uint32_t PAIR_MAX = 1000000;
+constexpr uint32_t TILE_WORDS = LVL_TILE / 64;
+static_assert(TILE_WORDS == 16, "a tile's words are scanned within a row of 16 lanes");
+
+__global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
+    ListBufs LB, Coords P, TreeDev t, const uint32_t *__restrict__ oid, uint32_t level, uint32_t T,
+    const unsigned long long *range, int lazy, uint32_t *viol, uint64_t *words, uint32_t *cnt) {
+  __shared__ int sd_s, tie_s;
+  __shared__ double kv_s;
+  __shared__ uint32_t sh[3][LVL_THREADS / 64];
+  const uint32_t nseg = 1u << level, k = blockIdx.x / T, q = blockIdx.x % T;
+  const uint32_t h = nseg - 1 + k;
+  const uint32_t s = t.seg_start[h], c = t.seg_count[h], e = s + c;
+  const uint32_t base = s + q * LVL_TILE;
+  if (c == 0 || base >= e) return;
+  const uint32_t m = t.lmask[h], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  // the tile's entries of every list, before the split is known
+  uint32_t id[3][LVL_ITEMS];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d == lazy) continue;
+    const uint32_t *ld = LB.in(m, d);
+#pragma unroll
+    for (int i = 0; i < LVL_ITEMS; ++i)
+      id[d][i] = ld[min(base + i * LVL_THREADS + threadIdx.x, e - 1)];
+  }
+  if (threadIdx.x == 0) {
+    bool tie;
+    double kv;
+    sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, q == 0, kv);
+    kv_s = kv;
+    tie_s = tie;
+  }
+  __syncthreads();
+  const int sd = sd_s;
+  const double kv = kv_s;
+  const double *key = P.c[sd];
+  uint32_t thr = 0, r0, r1;
+  if (tie_s) thr = tie_threshold<LVL_THREADS>(LB.in(m, sd), key, oid, s, c, r0, r1);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d == sd || d == lazy) continue;  // not partitioned, or not kept
+    double x[LVL_ITEMS];
+#pragma unroll
+    for (int i = 0; i < LVL_ITEMS; ++i) x[i] = key[id[d][i]];
+    uint32_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < LVL_ITEMS; ++i) {
+      bool left = x[i] < kv;
+      if (tie_s) left = left || (x[i] == kv && oid[id[d][i]] < thr);
+      const uint64_t b =
+          __builtin_amdgcn_ballot_w64(left && base + i * LVL_THREADS + threadIdx.x < e);
+      sum += (uint32_t)__builtin_popcountll(b);
+      if (lane == 0)
+        words[(((size_t)d * nseg + k) * T + q) * TILE_WORDS + i * (LVL_THREADS / 64) + w] = b;
+    }
+    if (lane == 0) sh[d][w] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3 && (int)threadIdx.x != sd && (int)threadIdx.x != lazy) {
+    uint32_t tot = 0;
+#pragma unroll
+    for (int v = 0; v < LVL_THREADS / 64; ++v) tot += sh[threadIdx.x][v];
+    cnt[((size_t)threadIdx.x * nseg + k) * T + q] = tot;
+  }
+}
+
+__global__ __launch_bounds__(LVL_THREADS) void k_level_move(
+    ListBufs LB, Coords P, TreeDev t, const uint32_t *__restrict__ oid, uint32_t level, uint32_t T,
+    int lazy, const uint64_t *__restrict__ words, const uint32_t *__restrict__ cnt) {
+  __shared__ uint32_t sh[3][LVL_THREADS / 64];
+  const uint32_t nseg = 1u << level, k = blockIdx.x / T, q = blockIdx.x % T;
+  const uint32_t h = nseg - 1 + k;
+  const uint32_t s = t.seg_start[h], c = t.seg_count[h], e = s + c, mid = s + c / 2;
+  const uint32_t base = s + q * LVL_TILE;
+  if (c == 0 || base >= e) return;
+  const uint32_t m = t.lmask[h], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int sd = t.split_dim[h];
+  uint32_t id[3][LVL_ITEMS], pre[3];
+  uint64_t word[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d == sd || d == lazy) continue;
+    const uint32_t *ld = LB.in(m, d);
+    const size_t row = ((size_t)d * nseg + k) * T;
+#pragma unroll
+    for (int i = 0; i < LVL_ITEMS; ++i)
+      id[d][i] = ld[min(base + i * LVL_THREADS + threadIdx.x, e - 1)];
+    word[d] = words[(row + q) * TILE_WORDS + (lane & (TILE_WORDS - 1u))];
+    uint32_t sum = 0;  // lefts in the tiles before this one
+    for (uint32_t i = threadIdx.x; i < q; i += LVL_THREADS) sum += cnt[row + i];
+    const uint32_t inc = lane_scan<true>(sum);
+    if (lane == 63) sh[d][w] = inc;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d == sd || d == lazy) continue;
+    uint32_t *od = LB.out(m, d);
+    uint32_t before = 0;
+#pragma unroll
+    for (int v = 0; v < LVL_THREADS / 64; ++v) before += sh[d][v];
+    // lefts before each of the tile's words (every row of 16 lanes alike)
+    const uint32_t p = (uint32_t)__builtin_popcountll(word[d]);
+    uint32_t inc = p;
+    inc += dpp_u32<0x111, 0xF>(inc);
+    inc += dpp_u32<0x112, 0xF>(inc);
+    inc += dpp_u32<0x114, 0xF>(inc);
+    inc += dpp_u32<0x118, 0xF>(inc);
+    pre[d] = before + inc - p;
+#pragma unroll
+    for (int i = 0; i < LVL_ITEMS; ++i) {
+      const uint32_t wi = i * (LVL_THREADS / 64) + w;
+      const uint64_t b =
+          ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(word[d] >> 32),
+                                                         __builtin_amdgcn_readfirstlane(wi))
+           << 32) |
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)word[d],
+                                              __builtin_amdgcn_readfirstlane(wi));
+      const uint32_t l = (uint32_t)__builtin_amdgcn_readlane(
+                             (int)pre[d], __builtin_amdgcn_readfirstlane(wi)) +
+                         lanes_below(b);
+      const uint32_t j = base + i * LVL_THREADS + threadIdx.x;
+      if (j < e) od[(b >> lane) & 1u ? s + l : mid + (j - s - l)] = id[d][i];
+    }
+  }
+  if (q != 0) return;
+  // the run of equal keys at the median, if there is one
+  uint32_t *ls = LB.in(m, sd);
+  const double *key = P.c[sd];
+  if (key[ls[mid - 1]] == key[ls[mid]])  // uniform: read by every thread before the run moves
+    tie_fix<LVL_THREADS>(ls, LB.out(m, sd), key, oid, s, c);
+}
+
 // Device-wide levels [mid_level, sub_level) of each system, one workgroup per
 // segment of level mid_level (at most MID_MAX bodies; a task lists the
 // system and the segment): each level takes the same splits and
@@ -849,7 +1010,8 @@ k_level_mid(ListBufs LB, Coords P, TreeDev t0, const SysDesc *sys, const uint2 *
       const uint32_t s = t.seg_start[h] + S.list_off, c = t.seg_count[h];
       const uint32_t m = t.lmask[h];
       bool tie;
-      s_sd[j] = (uint8_t)split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie);
+      double kv;
+      s_sd[j] = (uint8_t)split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, true, kv);
       s_start[j] = s;
       s_cnt[j] = c;
       s_mask[j] = (uint8_t)m;
@@ -1953,6 +2115,8 @@ static uint32_t level_tiles(const Forest &f, int lev) {
   return (maxseg + LVL_TILE - 1) / LVL_TILE;
 }
 
+size_t level_words(size_t cnt_entries) { return cnt_entries * TILE_WORDS; }
+
 size_t level_cnt_entries(const Forest &f) {
   size_t m = 1;
   for (int lev = 0; lev < f.max_sub_level; ++lev)
@@ -2011,7 +2175,7 @@ void set_mid_levels(std::vector<SysDesc> &sys, std::vector<uint2> &tasks) {
 hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const StateDev &out,
                         const TreeDev &t, BuildBufs &b, double4 *pos64, float4 *pos32,
                         double theta, hipStream_t s, bool range_ready, int lazy, bool report,
-                        bool mid) {
+                        bool tree_order, bool mid) {
   const double *coord[3] = {in.x, in.y, in.z};
   const unsigned ny = (unsigned)f.nsys;
   hipError_t e = hipSuccess;
@@ -2068,10 +2232,17 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
   // every system's deeper device-wide levels (segments of at most MID_MAX
   // bodies) run in one launch, one workgroup per segment; the kernel-by-
   // kernel levels before them read the table whose sub_level is mid_level
-  const bool use_mid = mid && f.n_mid_tasks > 0;
+  const bool use_mid = mid && tree_order && f.n_mid_tasks > 0;
   const SysDesc *lsys = use_mid ? f.sys_mid : f.sys;
   const int lev_end = use_mid ? f.max_mid_level : f.max_sub_level;
-  for (int lev = 0; lev < lev_end; ++lev) {
+  const bool pair = f.nsys == 1 && (tree_order || f.max_n <= PAIR_MAX);
+  for (int lev = 0; lev < lev_end && pair; ++lev) {
+    const uint32_t nseg = 1u << lev, T = level_tiles(f, lev);
+    k_level_mark<<<nseg * T, LVL_THREADS, 0, s>>>(LB, P, t, in.oid, lev, T, b.range, lazy,
+                                                  report ? b.viol : nullptr, b.words, b.cnt);
+    k_level_move<<<nseg * T, LVL_THREADS, 0, s>>>(LB, P, t, in.oid, lev, T, lazy, b.words, b.cnt);
+  }
+  for (int lev = 0; lev < lev_end && !pair; ++lev) {
     const uint32_t nseg = 1u << lev;
     const uint32_t T = level_tiles(f, lev);
     k_level_split<<<dim3(nseg, ny), SPLIT_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev,

@@ -265,6 +265,7 @@ struct BuildBufs {
   uint32_t flag_words;  // 32-bit words of bits
   uint32_t *loc;     // working id -> local index inside a subtree block
   uint32_t *cnt;     // per-tile left counts of the device-wide levels
+  uint64_t *words;   // their left flags, a bit a position (single systems)
   uint32_t *perm;    // tree position -> working id
   // lazy dimension (single systems): bit d of *viol is set when dimension d
   // could be the split dimension of a device-wide segment, judged by its
@@ -283,6 +284,8 @@ SysDesc make_sys(const Shape &sh, uint32_t body_off, uint32_t node_off, uint32_t
 size_t sort_temp_bytes(uint32_t n, int nsys);
 // per-tile count entries the device-wide levels of a forest need
 size_t level_cnt_entries(const Forest &f);
+// flag words a single system's levels need beside that many counts
+size_t level_words(size_t cnt_entries);
 hipError_t launch_shape(const TreeDev &t, const Forest &f, int leaf, hipStream_t s);
 // range_ready: b.range already holds the range of `in` (computed by the
 // kick-drift that produced it), so the build skips its own range pass.
@@ -290,8 +293,9 @@ hipError_t launch_shape(const TreeDev &t, const Forest &f, int leaf, hipStream_t
 // nor partitioned at the device-wide levels, whose splits take its global
 // extent as the bound of every segment's, and the subtree builder sorts it
 // per segment; the tree is exact unless bit `lazy` of *b.viol is set.
-// mid: a single system's device-wide levels from mid_level(f) on run as one
-// launch of one workgroup per segment (mid_level(f) == f.max_sub_level: none).
+// tree_order: `in` is in a previous build's tree order.  mid: from tree order,
+// a system's device-wide levels from its mid_level on run as one launch of one
+// workgroup per segment.
 // report: clear *b.viol before the levels, then copy it to b.viol_host and
 // record b.ev_viol after them (a full build reports every dimension that a
 // lazy build could not have skipped).
@@ -307,7 +311,7 @@ size_t sub_tasks_max(int64_t n, int nsys);
 hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const StateDev &out,
                         const TreeDev &t, BuildBufs &b, double4 *pos64, float4 *pos32,
                         double theta, hipStream_t s, bool range_ready = false, int lazy = 3,
-                        bool report = false, bool mid = true);
+                        bool report = false, bool tree_order = false, bool mid = true);
 // Bits of a walk's variant: predicated leaf batches; every body's mass lies
 // within the bounds of the FP64 walk's shorter arithmetic.
 constexpr int WALK_PREDICATED = 2, WALK_MASSES_IN_RANGE = 8;
