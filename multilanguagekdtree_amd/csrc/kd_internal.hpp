@@ -387,6 +387,14 @@ hipError_t launch_range_reset(unsigned long long *range, hipStream_t s);
 hipError_t launch_to_original(const uint32_t *oid, const double *a0, const double *a1,
                               const double *a2, double *o0, double *o1, double *o2,
                               uint32_t n, hipStream_t st);
+// A forest's bodies from the caller's layout (systems back to back) to the
+// padded one, and three tree-ordered arrays back to it in original order.
+hipError_t launch_spread(const SysDesc *sys, const uint32_t *sob, const double *cat,
+                         double *padded, uint32_t total, hipStream_t st);
+hipError_t launch_gather_original(const uint32_t *oid, const SysDesc *sys, const uint32_t *sob,
+                                  const double *a0, const double *a1, const double *a2,
+                                  double *o0, double *o1, double *o2, uint32_t total,
+                                  hipStream_t st);
 hipError_t launch_inverse(const uint32_t *oid, uint32_t *inv, uint32_t n, hipStream_t st);
 hipError_t launch_iota(uint32_t *v, uint32_t n, hipStream_t st);
 hipError_t launch_sanitize(const StateDev &s, uint32_t n, int *bad, hipStream_t st);

@@ -58,6 +58,36 @@ __global__ void k_to_original(const uint32_t *__restrict__ oid, const double *__
   if (o2) o2[o] = a2[i];
 }
 
+// A forest's body positions between the caller's layout (systems back to back,
+// as in the sorted lists) and the padded one; padding positions become 0.
+__global__ void k_spread(const SysDesc *__restrict__ sys, const uint32_t *__restrict__ sob,
+                         const double *__restrict__ cat, double *__restrict__ padded,
+                         uint32_t total) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const SysDesc S = sys[sob[i >> 6]];
+  const uint32_t j = i - S.body_off;
+  padded[i] = j < S.n ? cat[S.list_off + j] : 0.0;
+}
+
+// out[original index, systems back to back] = a[t] for three components.
+__global__ void k_gather_original(const uint32_t *__restrict__ oid,
+                                  const SysDesc *__restrict__ sys,
+                                  const uint32_t *__restrict__ sob,
+                                  const double *__restrict__ a0, const double *__restrict__ a1,
+                                  const double *__restrict__ a2, double *__restrict__ o0,
+                                  double *__restrict__ o1, double *__restrict__ o2,
+                                  uint32_t total) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const SysDesc S = sys[sob[i >> 6]];
+  if (i - S.body_off >= S.n) return;
+  const uint32_t o = oid[i] - S.body_off + S.list_off;
+  o0[o] = a0[i];
+  o1[o] = a1[i];
+  o2[o] = a2[i];
+}
+
 __global__ void k_inverse(const uint32_t *__restrict__ oid, uint32_t *__restrict__ inv,
                           uint32_t n) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -148,6 +178,21 @@ hipError_t launch_to_original(const uint32_t *oid, const double *a0, const doubl
                               const double *a2, double *o0, double *o1, double *o2,
                               uint32_t n, hipStream_t st) {
   k_to_original<<<(n + 255) / 256, 256, 0, st>>>(oid, a0, a1, a2, o0, o1, o2, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_spread(const SysDesc *sys, const uint32_t *sob, const double *cat,
+                         double *padded, uint32_t total, hipStream_t st) {
+  k_spread<<<(total + 255) / 256, 256, 0, st>>>(sys, sob, cat, padded, total);
+  return hipGetLastError();
+}
+
+hipError_t launch_gather_original(const uint32_t *oid, const SysDesc *sys, const uint32_t *sob,
+                                  const double *a0, const double *a1, const double *a2,
+                                  double *o0, double *o1, double *o2, uint32_t total,
+                                  hipStream_t st) {
+  k_gather_original<<<(total + 255) / 256, 256, 0, st>>>(oid, sys, sob, a0, a1, a2, o0, o1, o2,
+                                                         total);
   return hipGetLastError();
 }
 
