@@ -354,7 +354,7 @@ static int create_impl(kd_ctx *c, int64_t cap, const Sizing &z) {
   HIP_TRY(hipMemsetAsync(c->pos64, 0, sizeof(double4) * (N + BODY_PAD), c->stream));
   HIP_TRY(hipMemsetAsync(c->pos32, 0, sizeof(float4) * (N + BODY_PAD), c->stream));
   ALLOC(c->allocs, c->b.cnt, z.cnt_entries);
-  ALLOC(c->allocs, c->b.words, z.nsys == 1 ? level_words(z.cnt_entries) : 1);
+  if (const size_t words = level_words(z.cnt_entries)) ALLOC(c->allocs, c->b.words, words);
   ALLOC(c->allocs, c->dsys, z.nsys);
   ALLOC(c->allocs, c->dsys_mid, z.nsys);
   c->dmid_cap = mid_tasks_max(cap, z.nsys);
@@ -1192,7 +1192,7 @@ struct kd_batch {
   // two halves of pinned memory through which results reach the caller's
   // arrays: a copy straight into pageable memory that was never touched ran at
   // 9 GB/s (16.5 MB arrays), through here at 30
-  static constexpr size_t STAGE = (size_t)4 << 20;
+  static constexpr size_t STAGE = (size_t)1 << 20;
   char *stage = nullptr;
   hipEvent_t staged[2] = {};
   // one step from state buffer 0 / 1, with lazy dimension 0, 1, 2 or none

@@ -818,7 +818,7 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_scatter(ListBufs LB,
   }
 }
 
-// A single system's device-wide level in two launches.  The six kernels above
+// A device-wide level in two launches.  The six kernels above
 // are mostly launches and waits in systems of up to a million bodies (22 us a
 // level at 100,000; these take 11).  k_level_mark: every tile decides its
 // segment's split for itself, marks the bodies of the lists that move by their
@@ -836,15 +836,28 @@ constexpr uint32_t PAIR_MAX = 1000000;
 constexpr uint32_t TILE_WORDS = LVL_TILE / 64;
 static_assert(TILE_WORDS == 16, "a tile's words are scanned within a row of 16 lanes");
 
+// FOREST: the system in blockIdx.y (a single system's table entry is not read:
+// it would be one more wait).
+template <bool FOREST>
 __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
-    ListBufs LB, Coords P, TreeDev t, const uint32_t *__restrict__ oid, uint32_t level, uint32_t T,
-    const unsigned long long *range, int lazy, uint32_t *viol, uint64_t *words, uint32_t *cnt) {
+    ListBufs LB, Coords P, TreeDev t, const SysDesc *__restrict__ sys,
+    const uint32_t *__restrict__ oid, uint32_t level, uint32_t T, const unsigned long long *range,
+    int lazy, uint32_t *viol, uint64_t *words, uint32_t *cnt) {
   __shared__ int sd_s, tie_s;
   __shared__ double kv_s;
   __shared__ uint32_t sh[3][LVL_THREADS / 64];
   const uint32_t nseg = 1u << level, k = blockIdx.x / T, q = blockIdx.x % T;
   const uint32_t h = nseg - 1 + k;
-  const uint32_t s = t.seg_start[h], c = t.seg_count[h], e = s + c;
+  uint32_t list_off = 0;
+  if (FOREST) {
+    const SysDesc S = sys[blockIdx.y];
+    if (level >= S.sub_level) return;
+    t = tree_at(t, S.node_off);
+    list_off = S.list_off;
+    words += (size_t)blockIdx.y * 3 * nseg * T * TILE_WORDS;
+    cnt += (size_t)blockIdx.y * 3 * nseg * T;
+  }
+  const uint32_t s = t.seg_start[h] + list_off, c = t.seg_count[h], e = s + c;
   const uint32_t base = s + q * LVL_TILE;
   if (c == 0 || base >= e) return;
   const uint32_t m = t.lmask[h], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -899,13 +912,24 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
   }
 }
 
+template <bool FOREST>
 __global__ __launch_bounds__(LVL_THREADS) void k_level_move(
-    ListBufs LB, Coords P, TreeDev t, const uint32_t *__restrict__ oid, uint32_t level, uint32_t T,
-    int lazy, const uint64_t *__restrict__ words, const uint32_t *__restrict__ cnt) {
+    ListBufs LB, Coords P, TreeDev t, const SysDesc *__restrict__ sys,
+    const uint32_t *__restrict__ oid, uint32_t level, uint32_t T, int lazy,
+    const uint64_t *__restrict__ words, const uint32_t *__restrict__ cnt) {
   __shared__ uint32_t sh[3][LVL_THREADS / 64];
   const uint32_t nseg = 1u << level, k = blockIdx.x / T, q = blockIdx.x % T;
   const uint32_t h = nseg - 1 + k;
-  const uint32_t s = t.seg_start[h], c = t.seg_count[h], e = s + c, mid = s + c / 2;
+  uint32_t list_off = 0;
+  if (FOREST) {
+    const SysDesc S = sys[blockIdx.y];
+    if (level >= S.sub_level) return;
+    t = tree_at(t, S.node_off);
+    list_off = S.list_off;
+    words += (size_t)blockIdx.y * 3 * nseg * T * TILE_WORDS;
+    cnt += (size_t)blockIdx.y * 3 * nseg * T;
+  }
+  const uint32_t s = t.seg_start[h] + list_off, c = t.seg_count[h], e = s + c, mid = s + c / 2;
   const uint32_t base = s + q * LVL_TILE;
   if (c == 0 || base >= e) return;
   const uint32_t m = t.lmask[h], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -2115,7 +2139,12 @@ static uint32_t level_tiles(const Forest &f, int lev) {
   return (maxseg + LVL_TILE - 1) / LVL_TILE;
 }
 
-size_t level_words(size_t cnt_entries) { return cnt_entries * TILE_WORDS; }
+size_t level_words(size_t cnt_entries) {
+  // 128 bytes a count, up to half a gigabyte: a forest whose largest system is
+  // far from the others (the counts are laid out for the largest) and a system
+  // of hundreds of millions keep the six kernels
+  return cnt_entries <= ((size_t)1 << 22) ? cnt_entries * TILE_WORDS : 0;
+}
 
 size_t level_cnt_entries(const Forest &f) {
   size_t m = 1;
@@ -2133,9 +2162,9 @@ hipError_t launch_shape(const TreeDev &t, const Forest &f, int leaf, hipStream_t
 }
 
 size_t mid_tasks_max(int64_t n, int nsys) {
-  // segments at a mid_level above MID_MIN_LEVEL hold more than MID_MAX / 2
+  // segments at a mid_level above MID_MIN_LEVEL hold more than MID_MAX / 8
   // bodies; at MID_MIN_LEVEL there are 2^MID_MIN_LEVEL of them
-  return (size_t)(2 * n / MID_MAX) + (size_t)nsys + ((size_t)1 << MID_MIN_LEVEL) + 1;
+  return (size_t)(8 * n / MID_MAX) + (size_t)nsys + ((size_t)1 << MID_MIN_LEVEL) + 1;
 }
 
 void set_sub_tasks(const std::vector<SysDesc> &sys, std::vector<uint2> &tasks) {
@@ -2153,11 +2182,22 @@ size_t sub_tasks_max(int64_t n, int nsys) {
 
 void set_mid_levels(std::vector<SysDesc> &sys, std::vector<uint2> &tasks) {
   tasks.clear();
+  // a forest's segments: as many as give every CU two, of MID_MAX bodies at
+  // most and a quarter of that at least.  Its step in ms with 65,536 /
+  // 32,768 / 16,384 / 8,192: 2.48 / 2.32 / 2.28 / 2.26 for 48 systems of 2,000
+  // to 200,000 bodies, 0.62 / 0.65 / 0.65 / 0.64 for 30 of 7,000 to 14,000 (whose
+  // levels all run here with 16,384 or more), 7.98 / 7.97 / 7.98 / 8.05 for 200.
+  size_t total = 0;
+  for (const SysDesc &d : sys) total += d.n;
+  const uint32_t most =
+      sys.size() == 1 ? MID_MAX
+                      : (uint32_t)std::min<size_t>(MID_MAX, std::max<size_t>(MID_MAX / 4,
+                                                                             total / 512));
   for (size_t q = 0; q < sys.size(); ++q) {
     SysDesc &d = sys[q];
     uint32_t mx = d.n;
     int l = 0;
-    while (mx > MID_MAX) {
+    while (mx > most) {
       mx = (mx + 1) / 2;
       ++l;
     }
@@ -2235,12 +2275,22 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
   const bool use_mid = mid && tree_order && f.n_mid_tasks > 0;
   const SysDesc *lsys = use_mid ? f.sys_mid : f.sys;
   const int lev_end = use_mid ? f.max_mid_level : f.max_sub_level;
-  const bool pair = f.nsys == 1 && (tree_order || f.max_n <= PAIR_MAX);
+  const bool pair = b.words != nullptr && (tree_order || f.max_n <= PAIR_MAX);
   for (int lev = 0; lev < lev_end && pair; ++lev) {
     const uint32_t nseg = 1u << lev, T = level_tiles(f, lev);
-    k_level_mark<<<nseg * T, LVL_THREADS, 0, s>>>(LB, P, t, in.oid, lev, T, b.range, lazy,
-                                                  report ? b.viol : nullptr, b.words, b.cnt);
-    k_level_move<<<nseg * T, LVL_THREADS, 0, s>>>(LB, P, t, in.oid, lev, T, lazy, b.words, b.cnt);
+    const dim3 grid(nseg * T, ny);
+    uint32_t *viol = report ? b.viol : nullptr;
+    if (f.nsys == 1) {
+      k_level_mark<false><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, b.range,
+                                                       lazy, viol, b.words, b.cnt);
+      k_level_move<false><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, lazy,
+                                                       b.words, b.cnt);
+    } else {
+      k_level_mark<true><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, b.range,
+                                                      lazy, viol, b.words, b.cnt);
+      k_level_move<true><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, lazy,
+                                                      b.words, b.cnt);
+    }
   }
   for (int lev = 0; lev < lev_end && !pair; ++lev) {
     const uint32_t nseg = 1u << lev;

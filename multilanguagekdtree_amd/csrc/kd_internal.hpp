@@ -265,7 +265,7 @@ struct BuildBufs {
   uint32_t flag_words;  // 32-bit words of bits
   uint32_t *loc;     // working id -> local index inside a subtree block
   uint32_t *cnt;     // per-tile left counts of the device-wide levels
-  uint64_t *words;   // their left flags, a bit a position (single systems)
+  uint64_t *words = nullptr;  // their left flags, a bit a position (may be absent)
   uint32_t *perm;    // tree position -> working id
   // lazy dimension (single systems): bit d of *viol is set when dimension d
   // could be the split dimension of a device-wide segment, judged by its
@@ -284,7 +284,7 @@ SysDesc make_sys(const Shape &sh, uint32_t body_off, uint32_t node_off, uint32_t
 size_t sort_temp_bytes(uint32_t n, int nsys);
 // per-tile count entries the device-wide levels of a forest need
 size_t level_cnt_entries(const Forest &f);
-// flag words a single system's levels need beside that many counts
+// flag words the levels use beside that many counts (0: too many to keep)
 size_t level_words(size_t cnt_entries);
 hipError_t launch_shape(const TreeDev &t, const Forest &f, int leaf, hipStream_t s);
 // range_ready: b.range already holds the range of `in` (computed by the

@@ -1,0 +1,49 @@
+"""The device-wide levels in two launches: runs of equal keys across medians
+(where a tile finds the threshold for itself and the first tile orders the
+run), tiles of every remainder, and forests, where the workgroup levels begin
+at sizes that depend on the whole.  Trees against the oracle's, bit for bit,
+from the upload's order and from tree order."""
+import numpy as np
+import pytest
+
+from helpers import compare_trees, pscale
+from multilanguagekdtree_amd import kdtree as K
+
+pytestmark = pytest.mark.gpu
+
+
+def points(kind, n, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "grid":  # a cubic lattice, every coordinate shared by many
+        k = int(np.ceil(n ** (1 / 3)))
+        p = np.stack(np.meshgrid(*[np.arange(k)] * 3), -1).reshape(-1, 3)[rng.permutation(k ** 3)[:n]]
+    elif kind == "few":  # nine values along x and y, so that runs cross tiles
+        p = np.stack([rng.integers(0, 9, n), rng.integers(0, 9, n), rng.normal(size=n)], 1)
+    else:
+        p = rng.normal(size=(n, 3))
+    p = np.ascontiguousarray(p.T, np.float64)
+    return dict(zip(K.FIELDS, (*p, *np.zeros((3, n)), rng.uniform(0.5, 1.5, n) / n)))
+
+
+@pytest.mark.parametrize("kind", ["grid", "few", "normal"])
+@pytest.mark.parametrize("n", [2049, 3073, 4097, 9999, 70_000, 131_071])
+def test_trees_match_oracle(orc, n, kind):
+    b = points(kind, n, n)
+    r = orc.build_tree(b)
+    with K.Simulation(n) as s:
+        s.upload(b)
+        for _ in range(3):
+            s.build()
+            compare_trees(s.export_tree(K.KD_LAYOUT_COMPACT), r, pscale(b))
+
+
+def test_forest_trees_match_oracle(orc):
+    sizes = [70_000, 5, 16_385, 40_000, 2049, 9000, 33_000]
+    parts = [points(("grid", "few", "normal")[i % 3], n, i) for i, n in enumerate(sizes)]
+    bodies = {f: np.concatenate([p[f] for p in parts]) for f in K.FIELDS}
+    with K.Batch(sizes, precision=K.KD_PREC_FP64) as bt:
+        bt.upload(bodies)
+        for _ in range(2):
+            bt.accel()
+            for i, b in enumerate(parts):
+                compare_trees(bt.export_tree(i), orc.build_tree(b), pscale(b))
