@@ -197,6 +197,12 @@ hipError_t launch_range(const StateDev &st, uint32_t n, unsigned long long *rang
 // and never share a key with a body.
 constexpr uint32_t PAD_KEY = 0xFFFFFFFFu;
 
+// A coordinate as the build compares it.  A step whose bodies reach a
+// non-finite position is only reported when the call ends, so later builds of
+// the call meet NaN: ordered as +inf, every list stays a permutation and every
+// split leaves exactly half a segment's bodies on its left.
+__device__ __forceinline__ double ordered(double v) { return fmin(v, INFINITY); }
+
 // The sort key of every body position j (the values the sort carries are
 // the positions themselves, read from a counting iterator).  In a forest
 // (sob set) the key is the system index in the top sysbits bits over the
@@ -214,7 +220,7 @@ __global__ void k_make_keys32(const double *__restrict__ p, const unsigned long 
   if (j >= n) return;
   const double lo = 0.5 * ordkey_inv(range[0]), hi = 0.5 * ordkey_inv(range[1]);
   const double scale = hi > lo ? 4294967294.0 / (hi - lo) : 0.0;
-  const double v = 0.5 * p[j];
+  const double v = 0.5 * ordered(p[j]);
   uint32_t k = (uint32_t)fmin(fmax((v - lo) * scale, 0.0), 4294967294.0);
   if (sob != nullptr) {
     const uint32_t q = sob[j >> 6];
@@ -229,7 +235,7 @@ __global__ void k_make_keys32(const double *__restrict__ p, const unsigned long 
 // k_fix_long, which finds its length and checks its coordinates in parallel.
 
 __device__ __forceinline__ bool coord_lt(const double *p, uint32_t a, uint32_t b) {
-  const double pa = p[a], pb = p[b];
+  const double pa = ordered(p[a]), pb = ordered(p[b]);
   return pa < pb || (pa == pb && a < b);
 }
 
@@ -249,8 +255,8 @@ __device__ void fix_run(const uint32_t *__restrict__ keys, uint32_t *__restrict_
     return;
   }
   bool distinct = false;
-  const double p0 = p[ids[i]];
-  for (uint32_t a = i + 1; a < j; ++a) distinct |= p[ids[a]] != p0;
+  const double p0 = ordered(p[ids[i]]);
+  for (uint32_t a = i + 1; a < j; ++a) distinct |= ordered(p[ids[a]]) != p0;
   if (!distinct) return;  // equal coordinates: the stable order stands
   for (uint32_t a = i + 1; a < j; ++a) {
     const uint32_t v = ids[a];
@@ -343,7 +349,7 @@ __device__ void sort_chunk(uint32_t *ids, uint32_t len, const double *__restrict
   for (uint32_t t = threadIdx.x; t < m; t += blockDim.x) {
     if (t < len) {
       si[t] = ids[t];
-      sk[t] = p[si[t]];
+      sk[t] = ordered(p[si[t]]);
     } else {
       si[t] = 0xffffffffu;
       sk[t] = __longlong_as_double(0x7ff0000000000000ll);  // +inf: padding sorts last
@@ -381,10 +387,10 @@ __global__ __launch_bounds__(256) void k_fix_long(const uint32_t *runs,
     }
     const uint32_t len = end - st;
     // equal coordinates throughout: the stable order stands
-    const double p0 = p[ids[st]];
+    const double p0 = ordered(p[ids[st]]);
     int distinct = 0;
     for (uint32_t j = st + 1 + threadIdx.x; j < end; j += blockDim.x)
-      distinct |= p[ids[j]] != p0 ? 1 : 0;
+      distinct |= ordered(p[ids[j]]) != p0 ? 1 : 0;
     if (!__syncthreads_or(distinct)) continue;
     uint32_t *a = ids + st, *b = scratch + st;
     for (uint32_t c = 0; c < len; c += LONG_LDS)
@@ -452,7 +458,7 @@ __device__ uint32_t tie_threshold(const uint32_t *ls, const double *key,
                                   const uint32_t *__restrict__ oid, uint32_t s, uint32_t c,
                                   uint32_t &r0, uint32_t &r1) {
   const uint32_t mid = s + c / 2;
-  const double kv = key[ls[mid]];
+  const double kv = ordered(key[ls[mid]]);
   __shared__ uint32_t r0s, r1s, need_s, prefix_s, mask_s;
   __shared__ uint32_t hist[256];
   if (threadIdx.x == 0) {
@@ -460,14 +466,14 @@ __device__ uint32_t tie_threshold(const uint32_t *ls, const double *key,
     uint32_t lo = s, hi = mid;  // first position with key == kv
     while (lo < hi) {
       uint32_t m = lo + (hi - lo) / 2;
-      if (key[ls[m]] < kv) lo = m + 1; else hi = m;
+      if (ordered(key[ls[m]]) < kv) lo = m + 1; else hi = m;
     }
     const uint32_t first = lo;
     lo = mid + 1;
     hi = s + c;  // first position with key > kv
     while (lo < hi) {
       uint32_t m = lo + (hi - lo) / 2;
-      if (key[ls[m]] > kv) hi = m; else lo = m + 1;
+      if (ordered(key[ls[m]]) > kv) hi = m; else lo = m + 1;
     }
     r0s = first;
     r1s = lo;
@@ -597,7 +603,7 @@ __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P,
   const uint32_t mid = s + c / 2;
   kv = P.c[sd][LB.in(m, sd)[mid]];
   const double kp = P.c[sd][LB.in(m, sd)[mid - 1]];
-  tie = kp == kv;
+  tie = ordered(kp) == ordered(kv);
   if (!write) return sd;
   const uint8_t cm = (uint8_t)(m ^ (7u ^ (1u << sd)));
   t.lmask[2 * h + 1] = cm;
@@ -875,7 +881,7 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
     bool tie;
     double kv;
     sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, q == 0, kv);
-    kv_s = kv;
+    kv_s = ordered(kv);
     tie_s = tie;
   }
   __syncthreads();
@@ -889,7 +895,7 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
     if (d == sd || d == lazy) continue;  // not partitioned, or not kept
     double x[LVL_ITEMS];
 #pragma unroll
-    for (int i = 0; i < LVL_ITEMS; ++i) x[i] = key[id[d][i]];
+    for (int i = 0; i < LVL_ITEMS; ++i) x[i] = ordered(key[id[d][i]]);
     uint32_t sum = 0;
 #pragma unroll
     for (int i = 0; i < LVL_ITEMS; ++i) {
@@ -986,7 +992,8 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_move(
   // the run of equal keys at the median, if there is one
   uint32_t *ls = LB.in(m, sd);
   const double *key = P.c[sd];
-  if (key[ls[mid - 1]] == key[ls[mid]])  // uniform: read by every thread before the run moves
+  // (uniform: read by every thread before the run moves)
+  if (ordered(key[ls[mid - 1]]) == ordered(key[ls[mid]]))
     tie_fix<LVL_THREADS>(ls, LB.out(m, sd), key, oid, s, c);
 }
 

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from helpers import compare_trees, pscale
-from multilanguagekdtree_amd import kdtree as K
+from multilanguagekdtree_amd import _lib, kdtree as K
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,39 @@ def test_forest_trees_match_oracle(orc):
             bt.accel()
             for i, b in enumerate(parts):
                 compare_trees(bt.export_tree(i), orc.build_tree(b), pscale(b))
+
+
+@pytest.mark.parametrize("n", [2049, 5000, 70_000])
+def test_bodies_lost_in_a_call(n):
+    # two bodies at one position: FP64 forces are NaN, the steps left in the
+    # call build trees of NaN coordinates, then of nothing else, and the call
+    # reports it; the next upload starts from a clean state
+    good = points("normal", n, 3)
+    bad = {f: v.copy() for f, v in good.items()}
+    for f in "xyz":
+        bad[f][n // 3] = bad[f][1]
+    other = points("grid", 4097, 5)
+    join = lambda b: {f: np.concatenate([other[f] + 0.5 * (f == "x"), b[f]]) for f in K.FIELDS}
+    with K.Simulation(n) as s, K.Simulation(n) as fresh:
+        for steps in (2, 3, 5):
+            s.upload(bad)
+            with pytest.raises(_lib.KdError) as e:
+                s.step(steps)
+            assert e.value.code == _lib.KD_ERR_NONFINITE
+        for c in (s, fresh):
+            c.upload(good)
+            c.step(2)
+        a, b = s.download(), fresh.download()
+    for f in a:
+        np.testing.assert_array_equal(a[f], b[f])
+    with K.Batch([4097, n], precision=K.KD_PREC_FP64) as bt:
+        for steps in (2, 5):
+            bt.upload(join(bad))
+            with pytest.raises(_lib.KdError) as e:
+                bt.step(steps)
+            assert e.value.code == _lib.KD_ERR_NONFINITE
+        bt.upload(join(good))
+        bt.step(2)
+        got = bt.download()
+    for f in a:
+        np.testing.assert_array_equal(got[f][4097:], a[f])
