@@ -173,9 +173,11 @@ static int alloc_nodes(kd_ctx *c, int64_t s) {
     ALLOC(c->node_allocs, t.mx, s);
     ALLOC(c->node_allocs, t.my, s);
     ALLOC(c->node_allocs, t.mz, s);
-    ALLOC(c->node_allocs, t.rec64, s);
-    ALLOC(c->node_allocs, t.rec32, s);
-    ALLOC(c->node_allocs, t.recd, s);
+    // one record before the first: a walk that ends has read position 0
+    ALLOC(c->node_allocs, t.rec64, s + 1);
+    ALLOC(c->node_allocs, t.rec32, s + 1);
+    ALLOC(c->node_allocs, t.recd, s + 1);
+    ++t.rec64, ++t.rec32, ++t.recd;
     ALLOC(c->node_allocs, t.lmask, s);
     c->slots_alloc = s;
   }
@@ -1762,10 +1764,11 @@ extern "C" int kd_adj_create(int64_t n, int64_t steps, int64_t every, const kd_p
       (rc = adj_alloc(a, &a->ck_oid, (size_t)a->nck * N)) ||
       (rc = adj_alloc(a, &a->t_pos64, E * N + BODY_PAD)) ||
       (rc = adj_alloc(a, &a->t_pos32, E * N + BODY_PAD)) ||
-      (rc = adj_alloc(a, &a->t_oid, E * N)) || (rc = adj_alloc(a, &a->t_rec64, E * S)) ||
-      (rc = adj_alloc(a, &a->t_rec32, E * S)) || (rc = adj_alloc(a, &a->lm, N)) ||
+      (rc = adj_alloc(a, &a->t_oid, E * N)) || (rc = adj_alloc(a, &a->t_rec64, E * S + 1)) ||
+      (rc = adj_alloc(a, &a->t_rec32, E * S + 1)) || (rc = adj_alloc(a, &a->lm, N)) ||
       (rc = adj_alloc(a, &a->react, 4 * N)) || (rc = adj_alloc(a, &a->gnode, 4 * S)))
     return bail(rc);
+  ++a->t_rec64, ++a->t_rec32;  // a record before the first, as in alloc_nodes
   // body loads past a leaf reach the next slot or the padding: finite values
   if (hipMemset(a->t_pos64, 0, sizeof(double4) * (E * N + BODY_PAD)) != hipSuccess ||
       hipMemset(a->t_pos32, 0, sizeof(float4) * (E * N + BODY_PAD)) != hipSuccess) {

@@ -254,7 +254,7 @@ struct F32 {
     f.dx = p.x - r.cx;
     f.dy = p.y - r.cy;
     f.dz = p.z - r.cz;
-    f.d2 = f.dx * f.dx + f.dy * f.dy + f.dz * f.dz;
+    f.d2 = __builtin_fmaf(f.dz, f.dz, __builtin_fmaf(f.dx, f.dx, f.dy * f.dy));
     return r.size2 < f.d2;  // size2 holds size^2 / theta^2
   }
   // Every lane evaluates the term; lanes that do not accept add +0.  This
@@ -304,7 +304,7 @@ struct D64 {
     f.dx = (float)(p.x - r.cx);
     f.dy = (float)(p.y - r.cy);
     f.dz = (float)(p.z - r.cz);
-    f.d2 = f.dx * f.dx + f.dy * f.dy + f.dz * f.dz;
+    f.d2 = __builtin_fmaf(f.dz, f.dz, __builtin_fmaf(f.dx, f.dx, f.dy * f.dy));
     return r.size2 < f.d2;
   }
   // Every lane evaluates the term; lanes that do not accept add +0.  This
@@ -581,6 +581,23 @@ __device__ __forceinline__ float4 *walk_slots() {
   }
 }
 
+// A copy in scalar registers of its own.
+__device__ __forceinline__ uint32_t scalar_copy(uint32_t v) {
+  uint32_t r;
+  asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ float scalar_copy(float v) {
+  float r;
+  asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ double scalar_copy(double v) {
+  double r;
+  asm("s_mov_b64 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+
 // Counts of one lane (COUNT kernels): node tests, accepted nodes, pairs, and
 // the wavefront's node and leaf visits.
 struct LaneCounts {
@@ -589,9 +606,18 @@ struct LaneCounts {
 
 // One internal node r at position h: the lanes in actm test it, the far-field
 // term is added when `mine` (wave-uniform), E takes the new acceptance level,
-// and the next position is returned.
+// the next position is returned and r becomes its record.
+//   That record is fetched as soon as its position is known: a visit is a
+// chain of a scalar load and some forty dependent instructions, so the load
+// runs beside the far-field term, and in a leaf beside its bodies.  What the
+// rest of the visit needs of the node it leaves is copied first (one scalar
+// register), and the load then takes the old record's registers.  Walks in us
+// with the load at the top of a visit / here: mixed ring 150 / 137 at 5,000,
+// 293 / 254 at 100,000, 9630 / 8943 at 10 M; 300,000 bodies of a ball, FP64
+// differences, 8318 / 7436; FP64 ring 446 / 430 at 100,000.
 template <class P, bool COUNT>
-__device__ __forceinline__ uint32_t visit_inner(const typename P::Rec &r, uint32_t h, int lz,
+__device__ __forceinline__ uint32_t visit_inner(const typename P::Rec *__restrict__ nodes_m1,
+                                                typename P::Rec &r, uint32_t h, int lz,
                                                 uint64_t actm, bool active, bool mine,
                                                 double theta2, const typename P::Self &p, int &E,
                                                 typename P::Acc &acc, LaneCounts &c) {
@@ -610,10 +636,13 @@ __device__ __forceinline__ uint32_t visit_inner(const typename P::Rec &r, uint32
       : "=&s"(om), "=s"(hn)
       : "s"(actm), "s"(okm), "s"(2 * h), "s"(r.skip)
       : "scc");
+  typename P::Rec node;
+  node.m = scalar_copy(r.m);
+  r = load_rec_at(nodes_m1, uni(hn));
   const bool take = __builtin_amdgcn_inverse_ballot_w64(actm & okm);
   const bool open = __builtin_amdgcn_inverse_ballot_w64(om);
   // wave-uniform: the far-field term is evaluated only when a lane takes it
-  if (mine && (actm & okm)) P::m2p_sel(acc, r, f, take);
+  if (mine && (actm & okm)) P::m2p_sel(acc, node, f, take);
   // D = open ? unbounded : min(D, level): a taking lane had D >= level,
   // a lane outside D < level
   E = open ? -RSL : max(E, lz);
@@ -632,8 +661,8 @@ __device__ __forceinline__ void walk_nodes(const typename P::Rec *__restrict__ n
                                            const typename P::Self &p, int &E,
                                            typename P::Acc &acc, float4 *__restrict__ slot,
                                            uint32_t h, uint32_t stop, LaneCounts &c) {
+  typename P::Rec r = load_rec_at(nodes_m1, uni(h));
   do {
-    const typename P::Rec r = load_rec_at(nodes_m1, uni(h));
     const int lz = __builtin_clz(h);  // 32 - level(h) - log2(RS)
     // the lanes taking part, as a scalar mask (kept on the scalar unit) and
     // as the lane's own condition
@@ -642,24 +671,26 @@ __device__ __forceinline__ void walk_nodes(const typename P::Rec *__restrict__ n
     if (COUNT) ++c.wv;
     if (r.count <= leaf) {
       if (COUNT) ++c.wl;
+      const uint32_t start = scalar_copy(r.start), count = scalar_copy(r.count);
+      h = r.skip;
+      r = load_rec_at(nodes_m1, uni(h));
       bool split = false;
       if constexpr (P::COMPACT) {
         const uint32_t k = mask_count(actm);
         if (k <= SPLIT_MAX) {
-          leaf_split<P, COUNT>(acc, p, bodies + r.start, r.count, r.start, me, actm, active, slot,
+          leaf_split<P, COUNT>(acc, p, bodies + start, count, start, me, actm, active, slot,
                                c.np);
           split = true;
         }
       }
       if (!split)
-        for (uint32_t b = 0; b < r.count; b += P::CHUNK)
-          leaf_batch<P, P::CHUNK, COUNT, PRED>(acc, p, bodies + (r.start + b),
-                                               min((uint32_t)P::CHUNK, r.count - b),
-                                               r.start + b, me, active, c.np);
+        for (uint32_t b = 0; b < count; b += P::CHUNK)
+          leaf_batch<P, P::CHUNK, COUNT, PRED>(acc, p, bodies + (start + b),
+                                               min((uint32_t)P::CHUNK, count - b),
+                                               start + b, me, active, c.np);
       P::fold(acc);  // on every lane (a fold is valid at any point): no exec-mask change
-      h = r.skip;
     } else {
-      h = visit_inner<P, COUNT>(r, h, lz, actm, active, true, theta2, p, E, acc, c);
+      h = visit_inner<P, COUNT>(nodes_m1, r, h, lz, actm, active, true, theta2, p, E, acc, c);
     }
   } while (h != stop);
 }
@@ -696,11 +727,11 @@ __device__ __forceinline__ uint32_t walk_parts(const typename P::Rec *__restrict
       if (mine) walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, h, next, c);
       h = next;
     } else {
-      const typename P::Rec r = load_rec_at(nodes_m1, uni(h));
+      typename P::Rec r = load_rec_at(nodes_m1, uni(h));
       const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
       const bool active = __builtin_amdgcn_inverse_ballot_w64(actm);
       if (COUNT) ++c.wv;
-      h = visit_inner<P, COUNT>(r, h, lz, actm, active, mine, theta2, p, E, acc, c);
+      h = visit_inner<P, COUNT>(nodes_m1, r, h, lz, actm, active, mine, theta2, p, E, acc, c);
     }
   } while (h != 0);
   return parts > 0 ? parts : 1;
