@@ -123,6 +123,23 @@ __device__ __forceinline__ void range_commit(uint64_t lo[3], uint64_t hi[3], uin
   }
 }
 
+// A copy in scalar registers of its own.
+__device__ __forceinline__ uint32_t scalar_copy(uint32_t v) {
+  uint32_t r;
+  asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ float scalar_copy(float v) {
+  float r;
+  asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ double scalar_copy(double v) {
+  double r;
+  asm("s_mov_b64 %0, %1" : "=s"(r) : "s"(v));
+  return r;
+}
+
 // Tree-ordered body arrays carry this many padding entries so that batched
 // leaf loads (up to 8 bodies) never leave the allocation.
 constexpr int BODY_PAD = 32;
