@@ -27,9 +27,12 @@
 // keep the first, of the other half the second), 16 columns take 15 such adds
 // and 2 more, and one atomic instruction adds the batch to consecutive words (the
 // reactions are kept in tree order).  At 100,000 ring bodies the mixed walk
-// takes 0.90 ms against 1.57 with one wavefront, bodies one by one and the
+// takes 0.63 ms against 1.57 with one wavefront, bodies one by one and the
 // reactions through LDS (a row of 34 doubles a lane, 17 KB a wavefront); the
-// atomics are 0.18 ms of it.
+// atomics are 0.18 ms of it.  0.27 ms of the difference came with records and
+// bodies through the scalar unit (uniform_load), the next record fetched while
+// a node is worked on: FP64 needs 84 registers instead of 110, five wavefronts
+// a SIMD instead of four.
 #include <algorithm>
 
 #include "kd_internal.hpp"
@@ -152,14 +155,22 @@ __device__ __forceinline__ uint32_t fold16_col(uint32_t lane) {
   return (lane >> 5) | ((lane >> 3) & 2u) | ((lane >> 1) & 4u) | ((lane << 1) & 8u);
 }
 
+// A node record or a body at a wave-uniform byte offset.  The address is given
+// as constant memory, so that the scalar unit loads it: beside the walk's
+// atomics the compiler takes a plain load for one that may change, and loads
+// into vector registers, a lane each, what every lane reads alike.
+template <class T>
+__device__ __forceinline__ T uniform_load(const T *base, uint64_t off) {
+  typedef uint32_t words __attribute__((ext_vector_type(sizeof(T) / 4), aligned(16)));
+  typedef const words __attribute__((address_space(4))) *ptr;
+  const words w = *(ptr)(reinterpret_cast<uintptr_t>(base) + off);
+  T r;
+  __builtin_memcpy(&r, &w, sizeof(T));
+  return r;
+}
 template <class Rec>
 __device__ __forceinline__ Rec adj_rec(const Rec *nodes_m1, uint32_t off) {
-  typedef uint32_t words __attribute__((ext_vector_type(sizeof(Rec) / 4)));
-  const words w =
-      *reinterpret_cast<const words *>(reinterpret_cast<const char *>(nodes_m1) + uni_a(off));
-  Rec r;
-  __builtin_memcpy(&r, &w, sizeof(Rec));
-  return r;
+  return uniform_load(nodes_m1, uni_a(off));
 }
 
 template <bool MIXED>
@@ -221,7 +232,8 @@ __global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
     sz += gz;
     v[0] = -gx, v[1] = -gy, v[2] = -gz, v[3] = gm;
   };
-  auto inner = [&](const Rec &r, uint32_t h, int lz, bool mine) {
+  // the next record is loaded as soon as its position is known
+  auto inner = [&](Rec &r, uint32_t h, int lz, bool mine) {
     const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
     const auto dx = p.x - r.cx, dy = p.y - r.cy, dz = p.z - r.cz;
     const auto d2 = dx * dx + dy * dy + dz * dz;
@@ -232,22 +244,29 @@ __global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
       ok = r.size2 < a.theta2 * d2;
     const uint64_t tm = actm & __builtin_amdgcn_ballot_w64(ok);
     const uint64_t om = actm & ~tm;
+    const uint32_t hn = om ? 2 * h : r.skip;
+    const auto m = scalar_copy(r.m);
+    r = adj_rec(nodes, hn);
     if (mine && tm) {
       double v[4];
-      term(dx, dy, dz, d2, r.m, __builtin_amdgcn_inverse_ballot_w64(tm), v);
+      term(dx, dy, dz, d2, m, __builtin_amdgcn_inverse_ballot_w64(tm), v);
       const double s = fold4(v);
       if ((lane & 15u) == 0) atomicAdd(a.gnode + 4 * (size_t)(h / RS - 1) + col4, s);
     }
     E = __builtin_amdgcn_inverse_ballot_w64(om) ? -RSL : max(E, lz);
-    return om ? 2 * h : r.skip;
+    return hn;
   };
-  auto leaf = [&](const Rec &r, int lz) {
+  auto leaf = [&](uint32_t start, uint32_t count, int lz) {
     const bool active = lz >= E;
-    for (uint32_t b = 0; b < r.count; b += BATCH) {
-      const uint32_t j0 = r.start + b, m = min((uint32_t)BATCH, r.count - b);
-      Body q[BATCH];  // past the leaf: still inside the padded body arrays
-#pragma unroll
-      for (int i = 0; i < BATCH; ++i) q[i] = bodies[j0 + i];
+    for (uint32_t b = 0; b < count; b += BATCH) {
+      const uint32_t j0 = start + b, m = min((uint32_t)BATCH, count - b);
+      struct Batch {
+        Body q[BATCH];
+      };
+      // past the leaf: still inside the padded body arrays
+      const Batch t = uniform_load(reinterpret_cast<const Batch *>(bodies),
+                                   (uint64_t)j0 * sizeof(Body));
+      const Body *q = t.q;
       double v[4 * BATCH];
 #pragma unroll
       for (int i = 0; i < BATCH; ++i) {
@@ -275,12 +294,14 @@ __global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
       x >>= __builtin_ctz(~x);
       const uint32_t next = x == 0 ? 0 : (x + 1) * RS;
       if (mine) {
+        Rec r = adj_rec(nodes, h);
         do {
-          const Rec r = adj_rec(nodes, h);
           const int l = __builtin_clz(h);
           if (r.count <= a.leaf) {
-            leaf(r, l);
+            const uint32_t start = scalar_copy(r.start), count = scalar_copy(r.count);
             h = r.skip;
+            r = adj_rec(nodes, h);
+            leaf(start, count, l);
           } else {
             h = inner(r, h, l, true);
           }
@@ -288,7 +309,8 @@ __global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
       }
       h = next;
     } else {
-      h = inner(adj_rec(nodes, h), h, lz, mine);
+      Rec r = adj_rec(nodes, h);
+      h = inner(r, h, lz, mine);
     }
   } while (h != 0);
   if (valid) {
@@ -368,11 +390,12 @@ __global__ void k_adj_begin(double *lpx, double *lpy, double *lpz, double *lvx, 
 }
 
 // The depth of the subtrees dealt to the wavefronts of a workgroup (0: one
-// wavefront).  Backward of a step (with its recomputed forward, 630 us at
-// 100,000 ring bodies, 410 at 10,000, 165 at 2,000) in us at depths 0, 3, 4, 5,
-// 6: mixed 1835, 1734, 1541, 1579, 1754 at 100,000 and 1087, 921, 726, 615, 586
-// at 10,000; FP64 574, 439, 346, 292, 283 at 2,000.
-static int adj_depth(uint32_t n) { return n <= 16384 ? 6 : n <= 65536 ? 5 : n <= 200000 ? 4 : 0; }
+// wavefront).  Backward of a step (with its recomputed forward, 506 us at
+// 100,000 ring bodies, 350 at 10,000, 162 at 2,000) in us at depths 0, 3, 4, 5,
+// 6: mixed 1272, 1250, 1166, 1224 (to 5) at 100,000, 2216, 2171, 2129, 2214 (to
+// 5) at 300,000 and 783, 673, 550, 488, 470 at 10,000; FP64 466, 364, 290, 253,
+// 247 at 2,000.
+static int adj_depth(uint32_t n) { return n <= 16384 ? 6 : n <= 65536 ? 5 : n <= 400000 ? 4 : 0; }
 
 template <bool MIXED>
 static void launch_adj_walk(const AdjWalk &a, int levels, hipStream_t s) {
