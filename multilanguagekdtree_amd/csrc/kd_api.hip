@@ -328,7 +328,7 @@ static int create_impl(kd_ctx *c, int64_t cap, const Sizing &z) {
   ALLOC(c->allocs, c->wave_range, 6 * ((N + 63) / 64));
   c->b.sort_tmp_bytes = z.sort_bytes;
   for (int d = 0; d < 3; ++d) {
-    ALLOC(c->allocs, c->b.keys_in[d], N);
+    ALLOC(c->allocs, c->b.keys_in[d], N + SORT_CHUNK);
     ALLOC(c->allocs, c->b.keys_out[d], N);
     ALLOC(c->allocs, c->b.ids_in[d], N);
     ALLOC(c->allocs, c->b.runs[d], 2 * (N / FIX_SHORT + 1) + 2);

@@ -203,6 +203,18 @@ constexpr uint32_t PAD_KEY = 0xFFFFFFFFu;
 // split leaves exactly half a segment's bodies on its left.
 __device__ __forceinline__ double ordered(double v) { return fmin(v, INFINITY); }
 
+struct KeyMap {
+  double lo, scale;
+  __device__ __forceinline__ explicit KeyMap(const unsigned long long *range) {
+    lo = 0.5 * ordkey_inv(range[0]);
+    const double hi = 0.5 * ordkey_inv(range[1]);
+    scale = hi > lo ? 4294967294.0 / (hi - lo) : 0.0;
+  }
+  __device__ __forceinline__ uint32_t operator()(double p) const {
+    return (uint32_t)fmin(fmax((0.5 * ordered(p) - lo) * scale, 0.0), 4294967294.0);
+  }
+};
+
 // The sort key of every body position j (the values the sort carries are
 // the positions themselves, read from a counting iterator).  In a forest
 // (sob set) the key is the system index in the top sysbits bits over the
@@ -218,16 +230,179 @@ __global__ void k_make_keys32(const double *__restrict__ p, const unsigned long 
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j == 0) runs[0] = 0;
   if (j >= n) return;
-  const double lo = 0.5 * ordkey_inv(range[0]), hi = 0.5 * ordkey_inv(range[1]);
-  const double scale = hi > lo ? 4294967294.0 / (hi - lo) : 0.0;
-  const double v = 0.5 * ordered(p[j]);
-  uint32_t k = (uint32_t)fmin(fmax((v - lo) * scale, 0.0), 4294967294.0);
+  const KeyMap map(range);
+  uint32_t k = map(p[j]);
   if (sob != nullptr) {
     const uint32_t q = sob[j >> 6];
     const SysDesc S = sys[q];
     k = j - S.body_off >= S.n ? PAD_KEY : (q << (32 - sysbits)) | (k >> sysbits);
   }
   keys[j] = k;
+}
+
+// The sort of a single system of at most CHUNKED_MAX bodies, every dimension
+// in one launch: a workgroup forms the keys of a chunk of positions and sorts
+// it in LDS (four stable passes of 8 bits, ranked by ballots as in lz_radix),
+// then every body adds to its place in its chunk the number of bodies before
+// it in every other chunk, found by binary search.  At these sizes the sort
+// library merges in some fourteen launches a dimension, each of a few us and
+// most of that the launch; here the searches cost least, eight chunks' at a
+// time, and grow with the square of n.  Builds in us, with the library's sort
+// / here, ring: 133 / 95 at 2,100, 156 / 120 at 5,000, 207 / 161 at 30,000,
+// 241 / 194 at 100,000, 269 / 244 at 200,000, 337 (329 with SORT_MERGE_MAX) /
+// 309 at 300,000, 465 / 1137 at 1 M.
+constexpr int CHUNK_THREADS = 1024, CHUNK_ITEMS = 4;
+static_assert(SORT_CHUNK == CHUNK_THREADS * CHUNK_ITEMS);
+constexpr uint32_t CHUNKED_MAX = 300000;
+
+// Per dimension: coordinates, sorted keys and ids, what the fix passes use,
+// and the sorted chunks.
+struct SortDims {
+  const double *p[3];
+  uint32_t *keys[3], *ids[3], *runs[3];
+  uint32_t *ckeys[3], *cids[3];
+};
+
+__global__ __launch_bounds__(CHUNK_THREADS) void k_sort_chunks(SortDims sd, uint32_t n,
+                                                               const unsigned long long *range,
+                                                               int lazy) {
+  constexpr int NT = CHUNK_THREADS, IT = CHUNK_ITEMS, NW = NT / 64, ND = 256;
+  static_assert(NW * ND == 4 * NT, "four counters a thread");
+  __shared__ uint32_t key[2][SORT_CHUNK];
+  __shared__ uint16_t idx[2][SORT_CHUNK];
+  __shared__ uint32_t cnt[NW * ND], sh[NW];
+  const int d = blockIdx.y;
+  if (d == lazy) return;
+  const uint32_t first = blockIdx.x * SORT_CHUNK, n0 = min(SORT_CHUNK, n - first);
+  const int tid = threadIdx.x;
+  const uint32_t wv = tid >> 6, lane = tid & 63;
+  if (blockIdx.x == 0 && tid == 0) sd.runs[d][0] = 0;
+  const KeyMap map(range + 2 * d);
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const uint32_t i = it * NT + tid;
+    if (i >= n0) break;
+    key[0][i] = map(sd.p[d][first + i]);
+    idx[0][i] = (uint16_t)i;
+  }
+  __syncthreads();
+  const uint32_t per = (n0 + NT - 1) / NT;  // rounds of 64 positions a wavefront
+  const uint32_t base = wv * per * 64;
+  uint32_t *my = cnt + wv * ND;
+  for (int pass = 0; pass < 4; ++pass) {
+    const uint32_t *v = key[pass & 1];
+    const uint16_t *l = idx[pass & 1];
+    const int shift = 8 * pass;
+    for (uint32_t q = lane; q < (uint32_t)ND; q += 64) my[q] = 0;
+    wave_sync();
+    uint32_t x[IT], r[IT];
+    uint16_t y[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const uint32_t i = base + it * 64 + lane;
+      const bool use = (uint32_t)it < per && i < n0;
+      x[it] = use ? v[i] : 0u;
+      y[it] = use ? l[i] : (uint16_t)0;
+    }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      if ((uint32_t)it >= per || base + it * 64 >= n0) break;  // wave-uniform
+      const bool use = base + it * 64 + lane < n0;
+      const uint32_t g = (x[it] >> shift) & (ND - 1);
+      uint64_t same = __builtin_amdgcn_ballot_w64(use);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const bool bit = (g >> b) & 1u;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(bit);
+        same &= bit ? m : ~m;
+      }
+      const uint32_t below = lanes_below(same);
+      const uint32_t before = use ? my[g] : 0u;
+      r[it] = before + below;
+      wave_sync();
+      if (use && below == 0) my[g] = before + (uint32_t)__builtin_popcountll(same);
+      wave_sync();
+    }
+    __syncthreads();
+    // exclusive scan over (digit, wavefront): thread t holds digit t / 4,
+    // wavefronts 4 (t mod 4) and the next three
+    const uint32_t dg = tid >> 2, w0 = 4 * (tid & 3);
+    uint32_t c[4], sum = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      c[q] = cnt[(w0 + q) * ND + dg];
+      sum += c[q];
+    }
+    const uint32_t inc = lane_scan<true>(sum);
+    if (lane == 63) sh[wv] = inc;
+    __syncthreads();
+    uint32_t off = inc - sum;
+    for (uint32_t q = 0; q < (uint32_t)NW; ++q) off += q < wv ? sh[q] : 0u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      cnt[(w0 + q) * ND + dg] = off;
+      off += c[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      if ((uint32_t)it >= per || base + it * 64 + lane >= n0) break;
+      const uint32_t to = my[(x[it] >> shift) & (ND - 1)] + r[it];
+      key[(pass & 1) ^ 1][to] = x[it];
+      idx[(pass & 1) ^ 1][to] = y[it];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const uint32_t i = it * NT + tid;
+    // padding up to whole chunks, for the searches
+    if (i < n0 || gridDim.x > 1) sd.ckeys[d][first + i] = i < n0 ? key[0][i] : PAD_KEY;
+    if (i < n0) sd.cids[d][first + i] = first + idx[0][i];
+  }
+}
+
+__global__ __launch_bounds__(256) void k_sort_rank(SortDims sd, uint32_t n, int lazy) {
+  constexpr uint32_t B = 8;  // chunks searched at a time
+  const int d = blockIdx.y;
+  if (d == lazy) return;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t *__restrict__ keys = sd.ckeys[d];
+  // (uniform in a wavefront: a chunk holds whole ones)
+  const uint32_t mine = __builtin_amdgcn_readfirstlane(i / SORT_CHUNK);
+  const uint32_t chunks = (n + SORT_CHUNK - 1) / SORT_CHUNK;
+  const uint32_t k = keys[i];
+  uint32_t rank = i - mine * SORT_CHUNK;
+  for (uint32_t c0 = 0; c0 < chunks; c0 += B) {
+    uint32_t pos[B];
+#pragma unroll
+    for (uint32_t q = 0; q < B; ++q) pos[q] = 0;
+    // pos: keys before lim among the first pos + 2 step - 1 of the chunk
+#pragma unroll
+    for (uint32_t step = SORT_CHUNK / 2; step > 0; step >>= 1) {
+#pragma unroll
+      for (uint32_t q = 0; q < B; ++q) {
+        const uint32_t c = min(c0 + q, chunks - 1);
+        // equal keys of an earlier chunk come before (a body's key is below
+        // 2^32 - 1, that of the padding)
+        const uint32_t lim = c < mine ? k + 1u : k;
+        const uint32_t v = (keys + c * SORT_CHUNK + (step - 1))[pos[q]];
+        pos[q] += v < lim ? step : 0u;
+      }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < B; ++q) {
+      const uint32_t c = min(c0 + q, chunks - 1);
+      const uint32_t lim = c < mine ? k + 1u : k;
+      pos[q] += (keys + c * SORT_CHUNK)[pos[q]] < lim ? 1u : 0u;
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < B; ++q)
+      if (c0 + q < chunks && c0 + q != mine) rank += pos[q];
+  }
+  sd.keys[d][rank] = k;
+  sd.ids[d][rank] = sd.cids[d][i];
 }
 
 // Runs of equal keys: a run of at most FIX_SHORT ids is put in (coordinate,
@@ -274,11 +449,16 @@ __device__ void fix_run(const uint32_t *__restrict__ keys, uint32_t *__restrict_
 // Runs are disjoint, so threads never touch the same ids.
 constexpr uint32_t FIX_PER = 8;
 
-__global__ __launch_bounds__(256) void k_fix_runs(const uint32_t *__restrict__ keys,
-                                                  uint32_t *__restrict__ ids,
-                                                  const double *__restrict__ p, uint32_t n,
-                                                  const unsigned long long *range,
-                                                  uint32_t *runs) {
+// The fix passes take dimension d0 + blockIdx.y.
+__global__ __launch_bounds__(256) void k_fix_runs(SortDims sd, int d0, int lazy, uint32_t n,
+                                                  const unsigned long long *range) {
+  const int d = d0 + (int)blockIdx.y;
+  if (d == lazy) return;
+  const uint32_t *__restrict__ keys = sd.keys[d];
+  uint32_t *__restrict__ ids = sd.ids[d];
+  const double *__restrict__ p = sd.p[d];
+  uint32_t *runs = sd.runs[d];
+  range += 2 * d;
   const uint32_t i0 = (blockIdx.x * blockDim.x + threadIdx.x) * FIX_PER;
   if (i0 >= n) return;
   // every coordinate of this dimension equal (a planar system's z): the
@@ -361,10 +541,13 @@ __device__ void sort_chunk(uint32_t *ids, uint32_t len, const double *__restrict
   __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_fix_long(const uint32_t *runs,
-                                                  const uint32_t *__restrict__ keys, uint32_t n,
-                                                  uint32_t *ids, uint32_t *scratch,
-                                                  const double *__restrict__ p) {
+__global__ __launch_bounds__(256) void k_fix_long(SortDims sd, int d0, int lazy, uint32_t n) {
+  const int d = d0 + (int)blockIdx.y;
+  if (d == lazy) return;
+  const uint32_t *runs = sd.runs[d];
+  const uint32_t *__restrict__ keys = sd.keys[d];
+  uint32_t *ids = sd.ids[d], *scratch = sd.cids[d];
+  const double *__restrict__ p = sd.p[d];
   __shared__ double sk[LONG_LDS];
   __shared__ uint32_t si[LONG_LDS];
   __shared__ uint32_t s_end;
@@ -2100,18 +2283,22 @@ SysDesc make_sys(const Shape &sh, uint32_t body_off, uint32_t node_off, uint32_t
 // Radix sort of (32-bit key, 32-bit id) pairs: 8-bit digits, 1024 threads x
 // 10 items per tile.  On gfx950 this sorts 10 M pairs in ~320 us, against
 // ~400 us for rocprim's default tile of 1024 x 16 (wider digits, 10 or 11
-// bits in three passes, measured slower).
+// bits in three passes, measured slower).  Up to SORT_MERGE_MAX pairs it
+// merges instead (the library's own line is 2^20).  Builds in us, merging /
+// not: 269 / 310 at 200,000 ring bodies, 341 / 327 at 300,000, 423 / 392 at
+// 600,000, 498 / 465 at 1 M.
 #ifndef KD_SORT_BITS
 #define KD_SORT_BITS 8
 #endif
 #ifndef KD_SORT_ITEMS
 #define KD_SORT_ITEMS 10
 #endif
+constexpr size_t SORT_MERGE_MAX = 262144;
 using SortCfg = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, KD_SORT_ITEMS>,
                                         rocprim::kernel_config<1024, KD_SORT_ITEMS>, KD_SORT_BITS,
-                                        rocprim::block_radix_rank_algorithm::match>>;
+                                        rocprim::block_radix_rank_algorithm::match>, SORT_MERGE_MAX>;
 
 static int bits_for(uint32_t v) {
   int b = 1;
@@ -2243,31 +2430,55 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
     k_range<<<std::min<uint32_t>((nsort + 255) / 256, RANGE_BLOCKS), 256, 0, s>>>(
         in.x, in.y, in.z, nsort, b.range);
   }
-  // the three coordinate sorts are independent: dimension 0 runs on s,
-  // dimensions 1 and 2 on the side streams, forked after the range and
+  SortDims sd;
+  for (int d = 0; d < 3; ++d) {
+    sd.p[d] = coord[d];
+    sd.keys[d] = b.keys_out[d];
+    sd.ids[d] = b.L[d];
+    sd.runs[d] = b.runs[d];
+    sd.ckeys[d] = b.keys_in[d];
+    sd.cids[d] = b.ids_in[d];
+  }
+  const bool chunked = !whole && f.nsys == 1 && nsort <= CHUNKED_MAX;
+  if (chunked) {
+    const unsigned chunks = (nsort + SORT_CHUNK - 1) / SORT_CHUNK;
+    SortDims first = sd;  // a single chunk is the whole order
+    for (int d = 0; d < 3 && chunks == 1; ++d) {
+      first.ckeys[d] = sd.keys[d];
+      first.cids[d] = sd.ids[d];
+    }
+    k_sort_chunks<<<dim3(chunks, 3), CHUNK_THREADS, 0, s>>>(first, nsort, b.range, lazy);
+    if (chunks > 1) k_sort_rank<<<dim3((nsort + 255) / 256, 3), 256, 0, s>>>(sd, nsort, lazy);
+    k_fix_runs<<<dim3((nsort + 256 * FIX_PER - 1) / (256 * FIX_PER), 3), 256, 0, s>>>(
+        sd, 0, lazy, nsort, b.range);
+    k_fix_long<<<dim3(256, 3), 256, 0, s>>>(sd, 0, lazy, nsort);
+  }
+  const bool forked = !whole && !chunked;
+  // otherwise the three coordinate sorts are independent: dimension 0 runs on
+  // s, dimensions 1 and 2 on the side streams, forked after the range and
   // joined before the levels (a graph capture of s follows the fork)
-  if (!whole) e = hipEventRecord(b.fork, s);
-  for (int i = 0; i < 2 && e == hipSuccess && !whole; ++i)
+  if (forked) e = hipEventRecord(b.fork, s);
+  for (int i = 0; i < 2 && e == hipSuccess && forked; ++i)
     e = hipStreamWaitEvent(b.side[i], b.fork, 0);
   if (e != hipSuccess) return e;
-  for (int d = 0; d < 3 && !whole; ++d) {
-    const hipStream_t sd = d == 0 ? s : b.side[d - 1];
+  for (int d = 0; d < 3 && forked; ++d) {
+    const hipStream_t on = d == 0 ? s : b.side[d - 1];
     if (d == lazy) continue;  // sorted per segment by the subtree builder
     uint32_t *key32 = b.keys_in[d];
     uint32_t *key32_out = b.keys_out[d];
-    k_make_keys32<<<(nsort + 255) / 256, 256, 0, sd>>>(
+    k_make_keys32<<<(nsort + 255) / 256, 256, 0, on>>>(
         coord[d], b.range + 2 * d, key32, nsort, b.runs[d],
         f.nsys > 1 ? f.sys_of_block : nullptr, f.sys, bits_for((uint32_t)f.nsys));
     size_t bytes = b.sort_tmp_bytes;
     e = rocprim::radix_sort_pairs<SortCfg>(b.sort_tmp[d], bytes, key32, key32_out,
                                            rocprim::counting_iterator<uint32_t>(0u), b.L[d],
-                                           nsort, 0, 32, sd);
+                                           nsort, 0, 32, on);
     if (e != hipSuccess) return e;
-    k_fix_runs<<<(nsort + 256 * FIX_PER - 1) / (256 * FIX_PER), 256, 0, sd>>>(
-        key32_out, b.L[d], coord[d], nsort, b.range + 2 * d, b.runs[d]);
-    k_fix_long<<<256, 256, 0, sd>>>(b.runs[d], key32_out, nsort, b.L[d], b.ids_in[d], coord[d]);
+    k_fix_runs<<<(nsort + 256 * FIX_PER - 1) / (256 * FIX_PER), 256, 0, on>>>(sd, d, lazy, nsort,
+                                                                              b.range);
+    k_fix_long<<<256, 256, 0, on>>>(sd, d, lazy, nsort);
   }
-  for (int i = 0; i < 2 && e == hipSuccess && !whole; ++i) {
+  for (int i = 0; i < 2 && e == hipSuccess && forked; ++i) {
     e = hipEventRecord(b.join[i], b.side[i]);
     if (e == hipSuccess) e = hipStreamWaitEvent(s, b.join[i], 0);
   }

@@ -140,6 +140,9 @@ __device__ __forceinline__ double scalar_copy(double v) {
   return r;
 }
 
+// Positions that one workgroup sorts; the key arrays carry as many spare ones.
+constexpr uint32_t SORT_CHUNK = 4096;
+
 // Tree-ordered body arrays carry this many padding entries so that batched
 // leaf loads (up to 8 bodies) never leave the allocation.
 constexpr int BODY_PAD = 32;

@@ -83,3 +83,17 @@ def test_bodies_lost_in_a_call(n):
         got = bt.download()
     for f in a:
         np.testing.assert_array_equal(got[f][4097:], a[f])
+
+
+@pytest.mark.parametrize("kind", ["grid", "few", "normal"])
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 8192, 8193, 33_001, 300_000, 300_001])
+def test_sorts_match_oracle(orc, n, kind):
+    # one chunk of 4096, its edges, ragged last chunks, and both sides of the
+    # size up to which chunks are sorted and searched
+    b = points(kind, n, n + 1)
+    r = orc.build_tree(b)
+    with K.Simulation(n) as s:
+        s.upload(b)
+        for _ in range(2):
+            s.build()
+            compare_trees(s.export_tree(K.KD_LAYOUT_COMPACT), r, pscale(b))
