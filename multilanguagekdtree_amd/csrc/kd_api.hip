@@ -325,7 +325,7 @@ static int create_impl(kd_ctx *c, int64_t cap, const Sizing &z) {
     ALLOC(c->allocs, c->acc[d], N);
     ALLOC(c->allocs, c->acc_o[d], N);
   }
-  ALLOC(c->allocs, c->wave_range, 6 * ((N + 63) / 64));
+  ALLOC(c->allocs, c->wave_range, 6 * ((N + 63) / 64 + WALK_FEW_WAVES));
   c->b.sort_tmp_bytes = z.sort_bytes;
   for (int d = 0; d < 3; ++d) {
     ALLOC(c->allocs, c->b.keys_in[d], N + SORT_CHUNK);
@@ -682,7 +682,10 @@ int kd_step(kd_ctx *c, int64_t steps) {
       HIP_TRY(launch_traverse_kick(c->params.precision, c->traverse_variant, c->tree, c->pos64,
                                    c->pos32, n, c->params.theta, c->params.leaf_size, kd,
                                    c->stream));
-      if (range) HIP_TRY(launch_range_from_waves(c->wave_range, (n + 63) / 64, c->b.range, c->stream));
+      if (range) {
+        const uint32_t g = walk_bodies(c->params.precision, c->traverse_variant, n);
+        HIP_TRY(launch_range_from_waves(c->wave_range, (n + g - 1) / g, c->b.range, c->stream));
+      }
       if ((rc = record(c, 2))) return rc;
     } else {
       if ((rc = traverse_impl(c))) return rc;
@@ -1819,8 +1822,10 @@ static int adj_advance(kd_adj *a) {
   const KickDrift kd{c->st[c->cur], c->params.dt, c->bad, range ? c->wave_range : nullptr};
   HIP_TRY(launch_traverse_kick(c->params.precision, c->traverse_variant, c->tree, c->pos64,
                                c->pos32, n, c->params.theta, c->params.leaf_size, kd, c->stream));
-  if (range)
-    HIP_TRY(launch_range_from_waves(c->wave_range, (n + 63) / 64, c->b.range, c->stream));
+  if (range) {
+    const uint32_t g = walk_bodies(c->params.precision, c->traverse_variant, n);
+    HIP_TRY(launch_range_from_waves(c->wave_range, (n + g - 1) / g, c->b.range, c->stream));
+  }
   return KD_OK;
 }
 

@@ -41,22 +41,6 @@ constexpr uint32_t FIX_SHORT = 16;
 
 constexpr int MAX_LEAF = 32;
 
-// The depth at which an FP64 walk's sum is cut into parts (kd_traverse.hip),
-// from the bodies and levels of the tree alone, so that a system's result does
-// not depend on what runs beside it; 0: one part.  A workgroup of 2^(d - 2)
-// wavefronts then walks 64 bodies.  It pays while the wavefronts alone leave
-// most of the GPU's 8192 slots empty: ring, FP64 walk in us, depth 0 / 4 / 5 /
-// 6: 155 / 69 / 57 / 61 at 1,000 bodies, 334 / 153 / 130 / 102 at 10,000, 406 /
-// 252 / 205 / 250 at 30,000, 541 / 448 / 605 / 1193 at 100,000, 584 / 636 / 884
-// / 1821 at 150,000 (every wavefront visits the nodes above the parts, and the
-// slowest part holds up the rest).  Every node above the depth is internal:
-// with L levels every node down to depth L - 3 is.
-__host__ __device__ inline int walk_depth(uint32_t n, int levels) {
-  int d = n <= 16384 ? 6 : n <= 65536 ? 5 : n <= 131072 ? 4 : 0;
-  if (d > levels - 2) d = levels - 2;
-  return d < 3 ? 0 : d;
-}
-
 // The block index a kernel should treat as its own so that each of the 8
 // XCDs runs one contiguous range of the grid: the dispatcher hands blocks to
 // the XCDs round robin (block b to XCD b mod 8), and neighbouring bodies
@@ -394,6 +378,22 @@ hipError_t launch_adj_step(const AdjStep &st, hipStream_t s);
 size_t select_workspace_bytes(int64_t n);
 hipError_t launch_select(int64_t *idx, const double *vals, int64_t n, int64_t nvals,
                          int64_t goal, void *ws, hipStream_t s);
+
+// Bodies that a wavefront of a single system's walk takes.  An FP64 body's sum
+// does not depend on the bodies beside it (the mixed forms fold their partial
+// sums where any lane reaches a leaf), so in a small system, whose wavefronts
+// leave the GPU waiting on chains of visits, fewer bodies a wavefront make
+// shorter chains, at the price of idle lanes.  Walks in us at 64, 32, 16, 8
+// bodies, ring: 140, 133, 119, 116 at 1,000, 298, 269, 232, 223 at 8,000, 366,
+// 301, 276, 278 at 16,000, 402, 370, 370, 435 at 30,000, 483, 450, 450, 544 at
+// 60,000, 538, 552, 550 (16), 757 at 100,000.  (Sums cut in parts for several
+// wavefronts took 53 at 1,000 and 429 at 100,000, but their rounding differs,
+// and a few steps with close pairs make that visible.)
+constexpr uint32_t WALK_FEW_WAVES = 2048;  // at most so many more than ceil(n / 64)
+inline uint32_t walk_bodies(int precision, int variant, uint32_t n) {
+  if (precision != 0 || (variant & WALK_PREDICATED)) return 64;
+  return n <= 10000 ? 8 : n <= 20000 ? 16 : n <= 70000 ? 32 : 64;
+}
 
 // Replace every memset node of a captured graph by a fill kernel node with
 // the same dependencies (memset nodes are not replayed reliably here).

@@ -80,7 +80,6 @@ struct F64 {
   static constexpr int CHUNK = 4;  // leaf bodies per batch of scalar loads
   static constexpr bool SELF_BY_INDEX = true;  // self pair dropped by a select
   static constexpr bool COMPACT = false;  // leaves are never split across lanes
-  static constexpr bool PARTS = true;     // the sum may be formed in parts (walk_parts)
   static constexpr bool CHECKED = false;  // terms hold for every operand
   using Rec = NodeRec64;
   using Body = double4;
@@ -237,7 +236,6 @@ struct F32 {
   static constexpr int CHUNK = 8;
   static constexpr bool SELF_BY_INDEX = false;
   static constexpr bool COMPACT = true;
-  static constexpr bool PARTS = false;
   static constexpr bool CHECKED = false;
   using Rec = NodeRec32;
   using Body = float4;
@@ -290,7 +288,6 @@ struct D64 {
   static constexpr int CHUNK = 4;
   static constexpr bool SELF_BY_INDEX = true;
   static constexpr bool COMPACT = false;
-  static constexpr bool PARTS = false;
   static constexpr bool CHECKED = false;
   using Rec = NodeRecD;
   using Body = double4;
@@ -588,8 +585,8 @@ struct LaneCounts {
 };
 
 // One internal node r at position h: the lanes in actm test it, the far-field
-// term is added when `mine` (wave-uniform), E takes the new acceptance level,
-// the next position is returned and r becomes its record.
+// term is added, E takes the new acceptance level, the next position is
+// returned and r becomes its record.
 //   That record is fetched as soon as its position is known: a visit is a
 // chain of a scalar load and some forty dependent instructions, so the load
 // runs beside the far-field term, and in a leaf beside its bodies.  What the
@@ -601,7 +598,7 @@ struct LaneCounts {
 template <class P, bool COUNT>
 __device__ __forceinline__ uint32_t visit_inner(const typename P::Rec *__restrict__ nodes_m1,
                                                 typename P::Rec &r, uint32_t h, int lz,
-                                                uint64_t actm, bool active, bool mine,
+                                                uint64_t actm, bool active,
                                                 double theta2, const typename P::Self &p, int &E,
                                                 typename P::Acc &acc, LaneCounts &c) {
   constexpr int RSL = sizeof(typename P::Rec) == 32 ? 5 : 6;
@@ -625,7 +622,7 @@ __device__ __forceinline__ uint32_t visit_inner(const typename P::Rec *__restric
   const bool take = __builtin_amdgcn_inverse_ballot_w64(actm & okm);
   const bool open = __builtin_amdgcn_inverse_ballot_w64(om);
   // wave-uniform: the far-field term is evaluated only when a lane takes it
-  if (mine && (actm & okm)) P::m2p_sel(acc, node, f, take);
+  if (actm & okm) P::m2p_sel(acc, node, f, take);
   // D = open ? unbounded : min(D, level): a taking lane had D >= level,
   // a lane outside D < level
   E = open ? -RSL : max(E, lz);
@@ -636,14 +633,15 @@ __device__ __forceinline__ uint32_t visit_inner(const typename P::Rec *__restric
   return hn;
 }
 
-// The walk from position h until it leaves for position `stop`.
+// The walk, from the root until the position is 0.
 template <class P, bool COUNT, bool PRED>
 __device__ __forceinline__ void walk_nodes(const typename P::Rec *__restrict__ nodes_m1,
                                            const typename P::Body *__restrict__ bodies,
                                            uint32_t leaf, double theta2, uint32_t me,
                                            const typename P::Self &p, int &E,
                                            typename P::Acc &acc, float4 *__restrict__ slot,
-                                           uint32_t h, uint32_t stop, LaneCounts &c) {
+                                           LaneCounts &c) {
+  uint32_t h = (uint32_t)sizeof(typename P::Rec);
   typename P::Rec r = load_rec_at(nodes_m1, uni(h));
   do {
     const int lz = __builtin_clz(h);  // 32 - level(h) - log2(RS)
@@ -675,64 +673,22 @@ __device__ __forceinline__ void walk_nodes(const typename P::Rec *__restrict__ n
                                                start + b, me, active, c.np);
       P::fold(acc);  // on every lane (a fold is valid at any point): no exec-mask change
     } else {
-      h = visit_inner<P, COUNT>(nodes_m1, r, h, lz, actm, active, true, theta2, p, E, acc, c);
+      h = visit_inner<P, COUNT>(nodes_m1, r, h, lz, actm, active, theta2, p, E, acc, c);
     }
-  } while (__builtin_expect(h != stop, 1));
-}
-
-// The walk in parts: the nodes above level d are visited first to last, and
-// every node met at level d (lzd: the leading zeros of its position) begins
-// part i = 0, 1, ... of the sum.  own(i) (wave-uniform): whether this
-// wavefront adds part i; a part it does not own is passed over, which leaves
-// the lanes taking part in what follows as they would be (a subtree leaves a
-// lane that took part in it with D >= d).  begin(i): called before part i > 0
-// begins.  The far-field terms above level d belong to the part at hand.
-// Returns the number of parts (at least 1).  Every node above level d is
-// internal (walk_depth).
-template <class P, bool COUNT, bool PRED, class Own, class Begin>
-__device__ __forceinline__ uint32_t walk_parts(const typename P::Rec *__restrict__ nodes_m1,
-                                               const typename P::Body *__restrict__ bodies,
-                                               uint32_t leaf, double theta2, uint32_t me,
-                                               const typename P::Self &p, int &E,
-                                               typename P::Acc &acc, float4 *__restrict__ slot,
-                                               int lzd, LaneCounts &c, Own own, Begin begin) {
-  constexpr uint32_t RS = sizeof(typename P::Rec);
-  uint32_t h = RS, parts = 0;
-  bool mine = own(0);
-  do {
-    const int lz = __builtin_clz(h);
-    if (lz == lzd) {
-      if (parts > 0) begin(parts);
-      mine = own(parts);
-      ++parts;
-      // the node after this subtree (position 0: none)
-      uint32_t x = h / RS;
-      x >>= __builtin_ctz(~x);
-      const uint32_t next = x == 0 ? 0 : (x + 1) * RS;
-      if (mine) walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, h, next, c);
-      h = next;
-    } else {
-      typename P::Rec r = load_rec_at(nodes_m1, uni(h));
-      const uint64_t actm = __builtin_amdgcn_ballot_w64(lz >= E);
-      const bool active = __builtin_amdgcn_inverse_ballot_w64(actm);
-      if (COUNT) ++c.wv;
-      h = visit_inner<P, COUNT>(nodes_m1, r, h, lz, actm, active, mine, theta2, p, E, acc, c);
-    }
-  } while (h != 0);
-  return parts > 0 ? parts : 1;
+  } while (__builtin_expect(h != 0, 1));
 }
 
 // What a wavefront does with its bodies' accelerations (x, y, z): the
 // kick-drift, or the acceleration arrays.
 template <bool KD, class A>
-__device__ __forceinline__ void walk_finish(const A &a, const BodyState &bs, uint32_t wbase,
-                                            uint32_t me, bool valid, double x, double y,
+__device__ __forceinline__ void walk_finish(const A &a, const BodyState &bs, uint32_t wave,
+                                            uint32_t lane, uint32_t me, bool valid, double x, double y,
                                             double z) {
   if (KD) {
     uint64_t lo[3] = {~0ull, ~0ull, ~0ull}, hi[3] = {0ull, 0ull, 0ull};
     if (valid) kick_drift_one(a.kd, me, bs, x, y, z, lo, hi);
     if (a.kd.wave_range)
-      wave_range_store(a.kd.wave_range + 6 * (size_t)(wbase >> 6), lo, hi, me & 63);
+      wave_range_store(a.kd.wave_range + 6 * (size_t)wave, lo, hi, lane);
   } else if (valid) {
     a.ax[me] = x;
     a.ay[me] = y;
@@ -754,63 +710,39 @@ __device__ __forceinline__ int walk_start(bool valid) {
   constexpr int RSL = RS == 32 ? 5 : 6;
   return valid ? -RSL : 32 - RSL;
 }
-// clz(off) of the nodes at depth d (root 0)
-template <class P>
-__device__ __forceinline__ int depth_lz(int d) {
-  return 31 - (sizeof(typename P::Rec) == 32 ? 5 : 6) - d;
-}
 
-// The sum of a wavefront's bodies: in one part, or (PARTS) in the parts of
-// depth d, added in order (the sum that k_walk_split forms with several
-// wavefronts).  Returns whether it holds (CHECKED policies: every lane's
-// operands were in range).
-template <class P, bool COUNT, bool PRED, bool PARTS>
+// The sum of a wavefront's bodies.  Returns whether it holds (CHECKED
+// policies: every lane's operands were in range).
+template <class P, bool COUNT, bool PRED>
 __device__ __forceinline__ bool walk_sum(const typename P::Rec *__restrict__ nodes_m1,
                                          const typename P::Body *__restrict__ bodies,
                                          uint32_t leaf, double theta2, uint32_t me, bool valid,
                                          const typename P::Self &p, float4 *__restrict__ slot,
-                                         int d, LaneCounts &c, double sum[3]) {
+                                         LaneCounts &c, double sum[3]) {
   typename P::Acc acc;
   int E = walk_start<P>(valid);
-  if constexpr (PARTS) {
-    sum[0] = sum[1] = sum[2] = 0.0;
-    walk_parts<P, COUNT, PRED>(
-        nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, depth_lz<P>(d), c,
-        [](uint32_t) { return true; },
-        [&](uint32_t) {
-          P::fold(acc);
+  walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot, c);
+  P::fold(acc);
 #pragma unroll
-          for (int q = 0; q < 3; ++q) sum[q] += P::result(acc, q);
-          P::clear(acc);
-        });
-    P::fold(acc);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) sum[q] += P::result(acc, q);
-  } else {
-    walk_nodes<P, COUNT, PRED>(nodes_m1, bodies, leaf, theta2, me, p, E, acc, slot,
-                               (uint32_t)sizeof(typename P::Rec), 0u, c);
-    P::fold(acc);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) sum[q] = P::result(acc, q);
-  }
+  for (int q = 0; q < 3; ++q) sum[q] = P::result(acc, q);
   if constexpr (P::CHECKED)
     return __builtin_amdgcn_ballot_w64(!P::in_range(acc)) == 0;
   else
     return true;
 }
 
-// The walk of one wavefront: bodies [wbase, wbase + 64) of a tree whose
+// The walk of one wavefront: bodies [wbase, wbase + G) of a tree whose
 // records start one before nodes_m1[1] and whose bodies start at bodies[0].
-template <class P, bool COUNT, bool PRED, bool KD = false, bool PARTS = false>
+template <class P, bool COUNT, bool PRED, bool KD = false, int G = 64>
 __device__ __forceinline__ void walk_wave(const typename P::Rec *__restrict__ nodes_m1,
                                           const typename P::Body *__restrict__ bodies,
                                           const WalkArgs<P> &a, uint32_t wbase_in,
-                                          float4 *__restrict__ slot, int d = 0) {
+                                          float4 *__restrict__ slot) {
   // wave-uniform by construction; readfirstlane lets the compiler know it
   const uint32_t wbase = uni(wbase_in);
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t me = wbase + lane;
-  const bool valid = me < a.n;
+  const bool valid = (G == 64 || lane < (uint32_t)G) && me < a.n;
   const typename P::Self p = P::self(bodies[valid ? me : wbase]);
   BodyState bs{};
   if (KD) bs = body_state(a.kd, valid ? me : wbase);
@@ -819,16 +751,15 @@ __device__ __forceinline__ void walk_wave(const typename P::Rec *__restrict__ no
   if constexpr (P::CHECKED) {
     bool done = a.masses_in_range && P::usable(nodes_m1[1], a.leaf);
     if (done)
-      done = walk_sum<P, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p,
-                                             slot, d, c, sum);
+      done = walk_sum<P, COUNT, PRED>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p, slot, c,
+                                      sum);
     if (!done)
-      walk_sum<typename P::Exact, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me,
-                                                      valid, p, slot, d, c, sum);
+      walk_sum<typename P::Exact, COUNT, PRED>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p,
+                                               slot, c, sum);
   } else {
-    walk_sum<P, COUNT, PRED, PARTS>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p, slot, d, c,
-                                    sum);
+    walk_sum<P, COUNT, PRED>(nodes_m1, bodies, a.leaf, a.theta2, me, valid, p, slot, c, sum);
   }
-  walk_finish<KD>(a, bs, wbase, me, valid, sum[0], sum[1], sum[2]);
+  walk_finish<KD>(a, bs, wbase / (uint32_t)G, lane, me, valid, sum[0], sum[1], sum[2]);
   if (COUNT) {
     c.nt = wave_sum_u64(c.nt);
     c.na = wave_sum_u64(c.na);
@@ -869,81 +800,14 @@ __device__ __forceinline__ uint32_t walk_block() {
   const uint32_t t = nb - full, q = t / 8u, r = t % 8u, it = (blockIdx.x - full) / 8u;
   return full + x * q + (x < r ? x : r) + it;
 }
-template <class P, bool COUNT, bool PRED, bool KD = false, bool PARTS = false>
+template <class P, bool COUNT, bool PRED, bool KD = false, int G = 64>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KD_WALK_WAVES))) void k_walk(
     const typename P::Rec *__restrict__ nodes_m1, const typename P::Body *__restrict__ bodies,
-    WalkArgs<P> a, int d) {
-  const uint32_t wbase = (walk_block() * blockDim.x + threadIdx.x) & ~63u;
-  if (wbase >= a.n) return;
-  walk_wave<P, COUNT, PRED, KD, PARTS>(nodes_m1, bodies, a, wbase, walk_slots<P, 256>(), d);
-}
-
-// The walk of one wavefront's 64 bodies by the S wavefronts of a workgroup,
-// for systems whose wavefronts alone leave the GPU waiting on serial chains
-// of node visits (walk_depth: where, and what it measured).  Part i of the sum (walk_parts, depth log2(S) + 2: at most
-// 4 parts a wavefront) is wavefront i mod S's; every wavefront visits the
-// nodes above the parts, and the parts are added in order at the end, so the
-// result is walk_wave's with PARTS, bit for bit.
-template <class P, bool KD, int S>
-__global__ __launch_bounds__(64 * S) void k_walk_split(
-    const typename P::Rec *__restrict__ nodes_m1, const typename P::Body *__restrict__ bodies,
     WalkArgs<P> a) {
-  static_assert(P::PARTS && !P::COMPACT, "a policy whose sums may be cut into parts");
-  constexpr int D = S == 2 ? 3 : S == 4 ? 4 : S == 8 ? 5 : 6;
-  static_assert((1 << D) == 4 * S, "four parts a wavefront");
-  __shared__ double tot[3][64];
-  const uint32_t wbase = xcd_block() * 64u;
-  const uint32_t w = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const uint32_t me = wbase + lane;
-  const bool valid = me < a.n;
-  const typename P::Self p = P::self(bodies[valid ? me : wbase]);
-  BodyState bs{};
-  if (KD && w == 0) bs = body_state(a.kd, valid ? me : wbase);
-  double part[4][3];
-  uint32_t parts = 0;
-  auto own = [&](uint32_t i) { return (i & (S - 1u)) == w; };
-  auto walk = [&](auto policy) {
-    using Q = decltype(policy);
-    typename Q::Acc acc;
-    LaneCounts c;
-    int E = walk_start<Q>(valid);
-    uint32_t k = 0;  // parts of this wavefront that are done
-    auto keep = [&]() {
-#pragma unroll
-      for (uint32_t q = 0; q < 4; ++q)
-        if (q == k)  // wave-uniform
-          for (int x = 0; x < 3; ++x) part[q][x] = Q::result(acc, x);
-      Q::clear(acc);
-      ++k;
-    };
-    parts = walk_parts<Q, false, false>(nodes_m1, bodies, a.leaf, a.theta2, me, p, E, acc, nullptr,
-                                        depth_lz<Q>(D), c, own, [&](uint32_t i) {
-                                          if (own(i - 1)) keep();
-                                        });
-    if (own(parts - 1)) keep();
-    if constexpr (Q::CHECKED)
-      return !__syncthreads_or(!Q::in_range(acc));
-    else
-      return true;
-  };
-  if constexpr (P::CHECKED) {
-    bool done = a.masses_in_range && P::usable(nodes_m1[1], a.leaf);
-    if (done) done = walk(P());
-    if (!done) walk(typename P::Exact());
-  } else {
-    walk(P());
-  }
-#pragma unroll
-  for (uint32_t q = 0; q < 4; ++q) {
-    for (uint32_t v = 0; v < S && q * S + v < parts; ++v) {
-      if (v == w)
-        for (int x = 0; x < 3; ++x)
-          tot[x][lane] = (q + v == 0 ? 0.0 : tot[x][lane]) + part[q][x];
-      __syncthreads();
-    }
-  }
-  if (w == 0)
-    walk_finish<KD>(a, bs, wbase, me, valid, tot[0][lane], tot[1][lane], tot[2][lane]);
+  static_assert(G == 64 || !P::COMPACT, "leaves are split by the wavefront's active lanes");
+  const uint32_t wbase = ((walk_block() * blockDim.x + threadIdx.x) >> 6) * (uint32_t)G;
+  if (wbase >= a.n) return;
+  walk_wave<P, COUNT, PRED, KD, G>(nodes_m1, bodies, a, wbase, walk_slots<P, 256>());
 }
 
 // Forest walk: a task is one wavefront of one system (x: system, y: first
@@ -992,9 +856,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
       st.vz += S.body_off;
       if (b.kd.wave_range) b.kd.wave_range += 6 * ((size_t)t - (task.y >> 6));
     }
-    const int d = P::PARTS ? walk_depth(S.n, (int)S.levels) : 0;
-    walk_wave<P, COUNT, false, KD, P::PARTS>(nodes + S.node_off - 1, bodies + S.body_off, b, task.y,
-                                         walk_slots<P, NT>(), d);
+    walk_wave<P, COUNT, false, KD>(nodes + S.node_off - 1, bodies + S.body_off, b, task.y,
+                                   walk_slots<P, NT>());
     if (!PERSIST) return;
   }
 }
@@ -1003,19 +866,19 @@ __global__ void k_queue_reset(uint32_t *queue) {
   if (threadIdx.x < 8) queue[threadIdx.x] = 0u;
 }
 
-template <class P, bool KD, bool PARTS>
-static void launch_whole(const WalkArgs<P> &a, bool count, bool pred, int d, hipStream_t s) {
+template <class P, bool KD>
+static void launch_whole(const WalkArgs<P> &a, bool count, bool pred, hipStream_t s) {
   const unsigned blocks = (a.n + 255) / 256;
   if (count) {
     if (pred)
-      k_walk<P, true, true, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+      k_walk<P, true, true, KD><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
     else
-      k_walk<P, true, false, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+      k_walk<P, true, false, KD><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
   } else {
     if (pred)
-      k_walk<P, false, true, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+      k_walk<P, false, true, KD><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
     else
-      k_walk<P, false, false, KD, PARTS><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
+      k_walk<P, false, false, KD><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
   }
 }
 
@@ -1023,26 +886,20 @@ static void launch_whole(const WalkArgs<P> &a, bool count, bool pred, int d, hip
 // predicated (padding bodies of a batch need a select of their own).
 template <bool KD>
 static void launch_f64(const WalkArgs<F64Short> &a, bool count, bool pred, hipStream_t s) {
-  const int d = walk_depth(a.n, make_shape(a.n, (int)a.leaf).levels);
-  const unsigned groups = (a.n + 63) / 64;
-  if (count || pred) {
-    const WalkArgs<F64> e{a.nodes, a.bodies, a.n, a.leaf, a.theta2, a.ax, a.ay, a.az, a.cnt, a.kd};
-    if (d == 0)
-      launch_whole<F64, KD, false>(e, count, pred, d, s);
-    else
-      launch_whole<F64, KD, true>(e, count, pred, d, s);
-  } else if (d == 0) {
-    k_walk<F64Short, false, false, KD, false>
-        <<<(a.n + 255) / 256, 256, 0, s>>>(a.nodes - 1, a.bodies, a, d);
-  } else if (d == 3) {
-    k_walk_split<F64Short, KD, 2><<<groups, 128, 0, s>>>(a.nodes - 1, a.bodies, a);
-  } else if (d == 4) {
-    k_walk_split<F64Short, KD, 4><<<groups, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
-  } else if (d == 5) {
-    k_walk_split<F64Short, KD, 8><<<groups, 512, 0, s>>>(a.nodes - 1, a.bodies, a);
-  } else {
-    k_walk_split<F64Short, KD, 16><<<groups, 1024, 0, s>>>(a.nodes - 1, a.bodies, a);
-  }
+  const uint32_t g = walk_bodies(0, pred ? WALK_PREDICATED : 0, a.n);
+  const unsigned blocks = (a.n + 4 * g - 1) / (4 * g);
+  if (count || pred)
+    launch_whole<F64, KD>(WalkArgs<F64>{a.nodes, a.bodies, a.n, a.leaf, a.theta2, a.ax, a.ay, a.az,
+                                        a.cnt, a.kd},
+                          count, pred, s);
+  else if (g == 64)
+    k_walk<F64Short, false, false, KD><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+  else if (g == 32)
+    k_walk<F64Short, false, false, KD, 32><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+  else if (g == 16)
+    k_walk<F64Short, false, false, KD, 16><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
+  else
+    k_walk<F64Short, false, false, KD, 8><<<blocks, 256, 0, s>>>(a.nodes - 1, a.bodies, a);
 }
 
 template <bool KD>
@@ -1058,13 +915,11 @@ static hipError_t launch_walk(int precision, bool count, int variant, const Tree
                                       masses},
                    count, pred, s);
   } else if (precision == 1) {
-    launch_whole<F32, KD, false>(
-        WalkArgs<F32>{t.rec32, pos32, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred,
-        0, s);
+    launch_whole<F32, KD>(
+        WalkArgs<F32>{t.rec32, pos32, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred, s);
   } else {
-    launch_whole<D64, KD, false>(
-        WalkArgs<D64>{t.recd, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred, 0,
-        s);
+    launch_whole<D64, KD>(
+        WalkArgs<D64>{t.recd, pos64, n, (uint32_t)leaf, theta2, ax, ay, az, c, kd}, count, pred, s);
   }
   return hipGetLastError();
 }

@@ -1,9 +1,8 @@
-"""The FP64 walk's forms: sums cut into parts that the wavefronts of a workgroup
-share (sizes around each change of depth, and leaf sizes whose trees are too
-shallow for it), and the shorter square root and quotient of a term.  The
-predicated walk runs the compiler's own square root and division with one
-wavefront for 64 bodies and forms the same sums, so every form must equal it
-bit for bit."""
+"""The FP64 walk's forms: fewer bodies a wavefront in small systems (sizes around
+each change, and leaf sizes whose trees are shallow), and the shorter square
+root and quotient of a term.  The predicated walk runs the compiler's own square
+root and division with 64 bodies a wavefront and forms the same sums, so every
+form must equal it bit for bit."""
 import numpy as np
 import pytest
 
@@ -28,7 +27,8 @@ def cloud(n, seed):
 
 @pytest.mark.parametrize("n,leaf", [
     (5, 7), (8, 7), (29, 7), (60, 7), (113, 7), (500, 32), (700, 32), (4097, 2), (16384, 7),
-    (16385, 7), (65536, 8), (65537, 7), (131072, 7), (131073, 7)])
+    (16385, 7), (65536, 8), (65537, 7), (131072, 7), (131073, 7), (10000, 7), (10001, 7), (20000, 8),
+    (20001, 7), (70000, 7), (70001, 7)])
 def test_forms_agree(n, leaf):
     for b in (K.ring(n, seed=n), cloud(n, n)):
         np.testing.assert_array_equal(accel(b, 0, leaf), accel(b, 1, leaf))
