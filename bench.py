@@ -529,8 +529,8 @@ def main():
     roofline = dict(bound="valu", achieved=round(achieved, 3), peak=peak, unit="TFLOP/s",
                     frac=round(achieved / peak, 4), traffic=traffic,
                     # the walk's kernel as rocprofv3 names it (profiles/step_kernels_*.md)
-                    kernel=("kd::k_walk<kd::F32, false, false, true>" if main_name == "mixed"
-                            else "kd::k_walk_f64<false, true>"),
+                    kernel=("kd::k_walk<kd::F32, false, false, true, 64>" if main_name == "mixed"
+                            else "kd::k_walk<kd::F64Short, false, false, true, 64>"),
                     kernel_ms=round(r["traverse_ms"], 3),
                     hbm_gbps=(None if traffic is None
                               else round(traffic / (r["traverse_ms"] * 1e-3) / 1e9, 1)),
