@@ -125,7 +125,6 @@ struct F64 {
   }
   __device__ static void fold(Acc &) {}
   __device__ static double result(const Acc &a, int i) { return a.s[i]; }
-  __device__ static void clear(Acc &a) { a.s[0] = a.s[1] = a.s[2] = 0.0; }
 };
 
 // The F64 policy with shorter sequences for the square root and the quotient
@@ -205,7 +204,6 @@ struct F64Short : F64 {
   }
   __device__ static void fold(Acc &) {}
   __device__ static double result(const Acc &a, int i) { return a.s[i]; }
-  __device__ static void clear(Acc &a) { a.s[0] = a.s[1] = a.s[2] = 0.0; }
 };
 
 // Blocked Kahan summation with the compensation carried in the partial:
@@ -278,7 +276,6 @@ struct F32 {
     a.p[2] += g * dz;
   }
   __device__ static void fold(Acc &a) { kahan_fold(a); }
-  __device__ static void clear(Acc &a) { a = Acc(); }
   __device__ static double result(const Acc &a, int i) {
     return (double)a.s[i] + (double)a.p[i];
   }
@@ -327,7 +324,6 @@ struct D64 {
     a.p[2] += g * dz;
   }
   __device__ static void fold(Acc &a) { kahan_fold(a); }
-  __device__ static void clear(Acc &a) { a = Acc(); }
   __device__ static double result(const Acc &a, int i) {
     return (double)a.s[i] + (double)a.p[i];
   }
@@ -594,7 +590,7 @@ struct LaneCounts {
 // register), and the load then takes the old record's registers.  Walks in us
 // with the load at the top of a visit / here: mixed ring 150 / 137 at 5,000,
 // 293 / 254 at 100,000, 9630 / 8943 at 10 M; 300,000 bodies of a ball, FP64
-// differences, 8318 / 7436; FP64 ring 446 / 430 at 100,000.
+// differences, 8318 / 7436.
 template <class P, bool COUNT>
 __device__ __forceinline__ uint32_t visit_inner(const typename P::Rec *__restrict__ nodes_m1,
                                                 typename P::Rec &r, uint32_t h, int lz,
