@@ -768,8 +768,12 @@ __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P,
   int sd;
   if (lazy < 3) {
     if (write && split_dim_of(ext) == lazy) atomicOr(viol, 1u << lazy);
-    ext[lazy] = -1.0;
-    sd = split_dim_of(ext);
+    // the larger of the two kept dimensions, never `lazy`: its list holds an
+    // earlier build's order, which the marks by coordinate do not cut in half
+    // (extents are NaN once bodies are lost in a call, so a rule over all
+    // three would pick dimension 0 whatever stood in for its extent)
+    const int a = lazy == 0 ? 1 : 0, b = lazy == 2 ? 1 : 2;
+    sd = ext[b] > ext[a] ? b : a;
   } else {
     sd = split_dim_of(ext);
     if (write && viol != nullptr) {
