@@ -141,21 +141,26 @@ struct F64 {
 // exact residual (d2 - g^2, -m - q den: one fma each), after which the error
 // before the last rounding is some 2^-100.
 // Operands: m is 0 or within 2^-452..2^431 (the upload checks the bodies'
-// masses), d2 below 2^300 (the root's size bounds every distance) and above
-// 2^-300, which the walk only knows afterwards: the accumulator keeps the
-// smallest d2 (its high word, which orders positive doubles) and a wavefront
-// that met a smaller one walks again with F64.
+// masses), d2 below 2^300 and above 2^-300.  A pair's d2 is bounded by the
+// root's size.  A node's is not: its centre of mass leaves the box of its
+// members by rounding (coincident bodies far from the origin) or by masses of
+// both signs, as far as infinity.  So the accumulator keeps the smallest d2 of
+// all terms and the largest of the nodes' (their high words, which order
+// positive doubles, infinities and NaN above them), and a wavefront that met
+// one outside walks again with F64.  (The largest costs one instruction a node
+// taken.)
 struct F64Short : F64 {
   static constexpr bool CHECKED = true;
   using Exact = F64;
   struct Acc {
     double s[3] = {0.0, 0.0, 0.0};
     uint32_t least = 0x7ff00000u;  // high word of the smallest d2
+    uint32_t most = 0u;            // of the largest d2 to a centre of mass
   };
-  static constexpr uint32_t LEAST = (1023u - 300u) << 20;
-  __device__ static bool in_range(const Acc &a) { return a.least > LEAST; }
+  static constexpr uint32_t LEAST = (1023u - 300u) << 20, MOST = (1023u + 300u) << 20;
+  __device__ static bool in_range(const Acc &a) { return a.least > LEAST && a.most < MOST; }
   // tree-wide: the root is internal and its extent small enough (every
-  // extent, and so every coordinate difference, is at most the root's size)
+  // extent, and so every difference of two bodies, is at most the root's size)
   __device__ static bool usable(const NodeRec64 &root, uint32_t leaf) {
     return root.count > leaf && root.size2 < 0x1p297;
   }
@@ -182,6 +187,7 @@ struct F64Short : F64 {
     root_of(f.d2, y, g);
     const double magi = quotient(r.m, f.d2 * g, y);
     a.least = min(a.least, (uint32_t)__double2hiint(f.d2));
+    a.most = max(a.most, (uint32_t)__double2hiint(f.d2));
     a.s[0] += f.dx * magi;
     a.s[1] += f.dy * magi;
     a.s[2] += f.dz * magi;
