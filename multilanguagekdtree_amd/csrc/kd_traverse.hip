@@ -132,9 +132,15 @@ struct F64 {
 // cover every operand (scaling, special values): a pair term takes 47 vector
 // instructions with them and 33 so; the 1 M ring FP64 walk takes 2.41 ms
 // against 3.21.
-// Both results are still the correctly rounded ones, so terms and sums are
-// F64's bit for bit (4e9 random operands over 2^-300..2^300 against sqrt()
-// and the division: no bit differs).  From y0 = v_rsq_f64(d2), relative error
+// The square root is the correctly rounded one (also of 85,308 operands built
+// to lie next to a midpoint).  The quotient is but where the exact one lies
+// some 2^-100 or less from a midpoint, which happens to about one ordinary
+// term in 10^14: it may then be the other neighbour (15 % of 40,000 quotients
+// built within 2^-106 of a midpoint; none of 4e9 random operands over
+// 2^-300..2^300).  So terms and sums are F64's but for an ulp of a term that
+// rarely.  A Newton step on the reciprocal, two instructions a term, gets all
+// of the 40,000 right; the walk of the 1 M ring takes 2.54 ms with it, of the
+// 1 M cube 13.5 against 12.9.  From y0 = v_rsq_f64(d2), relative error
 // below 2^-24.1, the third-order iteration y = y0 (1 + e/2 + 3 e^2 / 8),
 // e = 1 - d2 y0^2, leaves y within about an ulp of d2^-1/2; the square root
 // g = d2 y and the quotient q = -m y^3 then each take one correction by their
