@@ -24,6 +24,7 @@
 #include <rocprim/iterator/counting_iterator.hpp>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kd_internal.hpp"
 
@@ -632,41 +633,47 @@ struct ListBufs {
 
 // A run of equal keys straddles the median of a segment (list ls of its split
 // dimension, [s, s + c)): the run's members that go left are those with the
-// smallest original indices.  tie_threshold finds the run [r0, r1) and the
-// threshold (the original index of the first body that goes right) by a radix
-// selection; tie_fix also partitions the run stably (tmp = the same list's
-// output buffer, not live for this node).
-template <int NT>
-__device__ uint32_t tie_threshold(const uint32_t *ls, const double *key,
-                                  const uint32_t *__restrict__ oid, uint32_t s, uint32_t c,
-                                  uint32_t &r0, uint32_t &r1) {
-  const uint32_t mid = s + c / 2;
-  const double kv = ordered(key[ls[mid]]);
-  __shared__ uint32_t r0s, r1s, need_s, prefix_s, mask_s;
-  __shared__ uint32_t hist[256];
+// smallest original indices.  tie_run finds the run [r0, r1), tie_threshold
+// the threshold (the original index of the first body that goes right; it is
+// not 0) by a radix selection; tie_order partitions the run stably (tmp = the
+// same list's output buffer, not live for this node).
+__device__ __forceinline__ void tie_run(const uint32_t *ls, const double *key, uint32_t s,
+                                        uint32_t c, uint32_t &r0, uint32_t &r1) {
+  __shared__ uint32_t r0s, r1s;
   if (threadIdx.x == 0) {
+    const uint32_t mid = s + c / 2;
+    const double kv = ordered(key[ls[mid]]);
     // keys are sorted non-decreasing inside [s, s+c)
     uint32_t lo = s, hi = mid;  // first position with key == kv
     while (lo < hi) {
       uint32_t m = lo + (hi - lo) / 2;
       if (ordered(key[ls[m]]) < kv) lo = m + 1; else hi = m;
     }
-    const uint32_t first = lo;
+    r0s = lo;
     lo = mid + 1;
     hi = s + c;  // first position with key > kv
     while (lo < hi) {
       uint32_t m = lo + (hi - lo) / 2;
       if (ordered(key[ls[m]]) > kv) hi = m; else lo = m + 1;
     }
-    r0s = first;
     r1s = lo;
-    need_s = mid - first;
-    prefix_s = 0;
-    mask_s = 0;
   }
   __syncthreads();
   r0 = r0s;
   r1 = r1s;
+}
+
+// The member of [r0, r1) with `need` smaller indices.
+template <int NT>
+__device__ uint32_t tie_threshold(const uint32_t *ls, const uint32_t *__restrict__ oid,
+                                  uint32_t r0, uint32_t r1, uint32_t need) {
+  __shared__ uint32_t need_s, prefix_s, mask_s;
+  __shared__ uint32_t hist[256];
+  if (threadIdx.x == 0) {
+    need_s = need;
+    prefix_s = 0;
+    mask_s = 0;
+  }
   for (int shift = 24; shift >= 0; shift -= 8) {
     for (int i = threadIdx.x; i < 256; i += NT) hist[i] = 0;
     __syncthreads();
@@ -692,12 +699,9 @@ __device__ uint32_t tie_threshold(const uint32_t *ls, const double *key,
 }
 
 template <int NT>
-__device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
-                        const uint32_t *__restrict__ oid, uint32_t s, uint32_t c) {
+__device__ void tie_order(uint32_t *ls, uint32_t *tmp, const uint32_t *__restrict__ oid,
+                          uint32_t r0, uint32_t r1, uint32_t nleft, uint32_t thr_oid) {
   __shared__ uint32_t scan_sh[NT / 64];
-  uint32_t r0, r1;
-  const uint32_t thr_oid = tie_threshold<NT>(ls, key, oid, s, c, r0, r1);
-  uint32_t nleft = s + c / 2 - r0;
   uint32_t off_l = 0, off_r = nleft;
   for (uint32_t base = r0; base < r1; base += NT) {
     uint32_t p = base + threadIdx.x;
@@ -716,6 +720,16 @@ __device__ void tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
   }
   __syncthreads();
   for (uint32_t p = r0 + threadIdx.x; p < r1; p += NT) ls[p] = tmp[p];
+}
+
+template <int NT>
+__device__ uint32_t tie_fix(uint32_t *ls, uint32_t *tmp, const double *key,
+                            const uint32_t *__restrict__ oid, uint32_t s, uint32_t c) {
+  uint32_t r0, r1;
+  tie_run(ls, key, s, c, r0, r1);
+  const uint32_t nleft = s + c / 2 - r0, thr = tie_threshold<NT>(ls, oid, r0, r1, nleft);
+  tie_order<NT>(ls, tmp, oid, r0, r1, nleft, thr);
+  return thr;
 }
 
 // Split dimension of extents e: the largest, ties to the lower dimension
@@ -801,12 +815,21 @@ __device__ __forceinline__ int split_decide(const ListBufs &LB, const Coords &P,
   return sd;
 }
 
+// Where a level's first kernel leaves the threshold index of segment k's run
+// (0: no run at the median) for the next: the counts of the split dimension's
+// list, which does not move, are not used.
+__device__ __forceinline__ uint32_t *level_thr(uint32_t *cnt, uint32_t nseg, uint32_t k,
+                                                 uint32_t T, int sd) {
+  return cnt + ((size_t)sd * nseg + k) * T;
+}
+
 __global__ __launch_bounds__(SPLIT_THREADS) void k_level_split(ListBufs LB, Coords P,
                                                                TreeDev t0, const SysDesc *sys,
                                                                const uint32_t *oid,
                                                                uint32_t level,
                                                                const unsigned long long *range,
-                                                               int lazy, uint32_t *viol) {
+                                                               int lazy, uint32_t *viol,
+                                                               uint32_t *cnt, uint32_t T) {
   const SysDesc S = sys[blockIdx.y];
   if (level >= S.sub_level) return;
   const uint32_t k = blockIdx.x;
@@ -822,8 +845,11 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_level_split(ListBufs LB, Coor
     tie_s = tie;
   }
   __syncthreads();
+  uint32_t thr = 0;
   if (tie_s)
-    tie_fix<SPLIT_THREADS>(LB.in(m, sd_s), LB.out(m, sd_s), P.c[sd_s], oid, s, c);
+    thr = tie_fix<SPLIT_THREADS>(LB.in(m, sd_s), LB.out(m, sd_s), P.c[sd_s], oid, s, c);
+  if (cnt != nullptr && threadIdx.x == 0)
+    *level_thr(cnt + (size_t)blockIdx.y * (3u << level) * T, 1u << level, k, T, sd_s) = thr;
 }
 
 __global__ __launch_bounds__(LVL_THREADS) void k_level_flags(ListBufs LB, TreeDev t0,
@@ -1015,10 +1041,11 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_scatter(ListBufs LB,
 // are mostly launches and waits in systems of up to a million bodies (22 us a
 // level at 100,000; these take 11).  k_level_mark: every tile decides its
 // segment's split for itself, marks the bodies of the lists that move by their
-// coordinates against the split value (a bit a position) and counts its lefts.  k_level_move: every tile adds up the counts of the
-// tiles before it and places its bodies.  Where equal keys straddle the
-// median, a tile of the first launch finds the threshold index for itself, and
-// the segment's first tile of the second orders the run.
+// coordinates against the split value (a bit a position) and counts its lefts.
+// k_level_move: every tile adds up the counts of the tiles before it and places
+// its bodies.  Where equal keys straddle the median, a tile of the first launch
+// finds the threshold index for itself, and the segment's first tile of the
+// second orders the run.
 // From an upload's order the coordinates of a larger system's list entries are
 // gathered from all of memory, and the packed flags of the split list are
 // cheaper.  Builds in us, six kernels a level / two, ring: 175 / 159 at 5,000,
@@ -1026,12 +1053,25 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_scatter(ListBufs LB,
 // first build after an upload 624 / 570 at 300,000, 1090 / 1065 at 1 M, 2440 /
 // 2600 at 3 M, 8340 / 9309 at 10 M.
 constexpr uint32_t PAIR_MAX = 1000000;
+// What a tile does for itself grows with its segment: the run of equal keys at
+// the median (four passes over it) and the counts before the tile.  So above
+// PAIR_TILES tiles a segment k_level_split decides and orders the run once and
+// k_level_scan adds up the counts, as in the six kernels.  Builds from tree
+// order in ms, six kernels / every tile for itself / with the line at 1024, 256,
+// 64 tiles: a lattice of 4 M bodies 5.4 / 7.0 / 6.0 / 5.7 / 5.6, two values in two
+// dimensions 140 / 255 / 159 / 148 / 144 (the subtree builder's share is 120); rings,
+// from 256 up the same but for noise: 0.34 at 300,000, 2.74, 2.77, 2.77 at 10 M
+// (0.357 at 300,000 with 64), and at 100 M 31.6, 30.6 and, with 256, 28.4.
+#ifndef KD_PAIR_TILES
+#define KD_PAIR_TILES 256
+#endif
+constexpr uint32_t PAIR_TILES = KD_PAIR_TILES;
 constexpr uint32_t TILE_WORDS = LVL_TILE / 64;
 static_assert(TILE_WORDS == 16, "a tile's words are scanned within a row of 16 lanes");
 
 // FOREST: the system in blockIdx.y (a single system's table entry is not read:
-// it would be one more wait).
-template <bool FOREST>
+// it would be one more wait).  DECIDED: k_level_split has run.
+template <bool FOREST, bool DECIDED>
 __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
     ListBufs LB, Coords P, TreeDev t, const SysDesc *__restrict__ sys,
     const uint32_t *__restrict__ oid, uint32_t level, uint32_t T, const unsigned long long *range,
@@ -1064,19 +1104,32 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
     for (int i = 0; i < LVL_ITEMS; ++i)
       id[d][i] = ld[min(base + i * LVL_THREADS + threadIdx.x, e - 1)];
   }
-  if (threadIdx.x == 0) {
-    bool tie;
-    double kv;
-    sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, q == 0, kv);
-    kv_s = ordered(kv);
-    tie_s = tie;
+  int sd;
+  double kv;
+  uint32_t thr = 0;  // 0: no run at the median
+  if (DECIDED) {
+    sd = t.split_dim[h];
+    kv = ordered(t.split_val[h]);
+    thr = *level_thr(cnt, nseg, k, T, sd);
+  } else {
+    if (threadIdx.x == 0) {
+      bool tie;
+      sd_s = split_decide(LB, P, t, h, s, c, m, range, lazy, viol, tie, q == 0, kv);
+      kv_s = ordered(kv);
+      tie_s = tie;
+    }
+    __syncthreads();
+    sd = sd_s;
+    kv = kv_s;
+    if (tie_s) {
+      uint32_t r0, r1;
+      const uint32_t *ls = LB.in(m, sd);
+      tie_run(ls, P.c[sd], s, c, r0, r1);
+      thr = tie_threshold<LVL_THREADS>(ls, oid, r0, r1, s + c / 2 - r0);
+    }
+    if (q == 0 && threadIdx.x == 0) *level_thr(cnt, nseg, k, T, sd) = thr;
   }
-  __syncthreads();
-  const int sd = sd_s;
-  const double kv = kv_s;
   const double *key = P.c[sd];
-  uint32_t thr = 0, r0, r1;
-  if (tie_s) thr = tie_threshold<LVL_THREADS>(LB.in(m, sd), key, oid, s, c, r0, r1);
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (d == sd || d == lazy) continue;  // not partitioned, or not kept
@@ -1087,7 +1140,7 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
 #pragma unroll
     for (int i = 0; i < LVL_ITEMS; ++i) {
       bool left = x[i] < kv;
-      if (tie_s) left = left || (x[i] == kv && oid[id[d][i]] < thr);
+      if (thr != 0) left = left || (x[i] == kv && oid[id[d][i]] < thr);
       const uint64_t b =
           __builtin_amdgcn_ballot_w64(left && base + i * LVL_THREADS + threadIdx.x < e);
       sum += (uint32_t)__builtin_popcountll(b);
@@ -1105,11 +1158,12 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_mark(
   }
 }
 
-template <bool FOREST>
+// DECIDED: the counts are scanned, the run is in order.
+template <bool FOREST, bool DECIDED>
 __global__ __launch_bounds__(LVL_THREADS) void k_level_move(
     ListBufs LB, Coords P, TreeDev t, const SysDesc *__restrict__ sys,
     const uint32_t *__restrict__ oid, uint32_t level, uint32_t T, int lazy,
-    const uint64_t *__restrict__ words, const uint32_t *__restrict__ cnt) {
+    const uint64_t *__restrict__ words, uint32_t *cnt) {
   __shared__ uint32_t sh[3][LVL_THREADS / 64];
   const uint32_t nseg = 1u << level, k = blockIdx.x / T, q = blockIdx.x % T;
   const uint32_t h = nseg - 1 + k;
@@ -1138,19 +1192,24 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_move(
     for (int i = 0; i < LVL_ITEMS; ++i)
       id[d][i] = ld[min(base + i * LVL_THREADS + threadIdx.x, e - 1)];
     word[d] = words[(row + q) * TILE_WORDS + (lane & (TILE_WORDS - 1u))];
-    uint32_t sum = 0;  // lefts in the tiles before this one
+    // lefts in the tiles before this one
+    if (DECIDED) {
+      pre[d] = cnt[row + q];
+      continue;
+    }
+    uint32_t sum = 0;
     for (uint32_t i = threadIdx.x; i < q; i += LVL_THREADS) sum += cnt[row + i];
     const uint32_t inc = lane_scan<true>(sum);
     if (lane == 63) sh[d][w] = inc;
   }
-  __syncthreads();
+  if (!DECIDED) __syncthreads();
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (d == sd || d == lazy) continue;
     uint32_t *od = LB.out(m, d);
-    uint32_t before = 0;
+    uint32_t before = DECIDED ? pre[d] : 0u;
 #pragma unroll
-    for (int v = 0; v < LVL_THREADS / 64; ++v) before += sh[d][v];
+    for (int v = 0; v < LVL_THREADS / 64 && !DECIDED; ++v) before += sh[d][v];
     // lefts before each of the tile's words (every row of 16 lanes alike)
     const uint32_t p = (uint32_t)__builtin_popcountll(word[d]);
     uint32_t inc = p;
@@ -1175,13 +1234,14 @@ __global__ __launch_bounds__(LVL_THREADS) void k_level_move(
       if (j < e) od[(b >> lane) & 1u ? s + l : mid + (j - s - l)] = id[d][i];
     }
   }
-  if (q != 0) return;
+  if (DECIDED || q != 0) return;
   // the run of equal keys at the median, if there is one
+  const uint32_t thr = *level_thr(cnt, nseg, k, T, sd);
+  if (thr == 0) return;
+  uint32_t r0, r1;
   uint32_t *ls = LB.in(m, sd);
-  const double *key = P.c[sd];
-  // (uniform: read by every thread before the run moves)
-  if (ordered(key[ls[mid - 1]]) == ordered(key[ls[mid]]))
-    tie_fix<LVL_THREADS>(ls, LB.out(m, sd), key, oid, s, c);
+  tie_run(ls, P.c[sd], s, c, r0, r1);
+  tie_order<LVL_THREADS>(ls, LB.out(m, sd), oid, r0, r1, mid - r0, thr);
 }
 
 // Device-wide levels [mid_level, sub_level) of each system, one workgroup per
@@ -2410,6 +2470,15 @@ void set_mid_levels(std::vector<SysDesc> &sys, std::vector<uint2> &tasks) {
   });
 }
 
+static void scan_level(uint32_t *cnt, uint32_t T, const SysDesc *sys, int lev, unsigned ny,
+                       hipStream_t s) {
+  const dim3 rows(3u << lev, ny);
+  if (T > SCAN_SMALL_T)
+    k_level_scan<1024><<<rows, 1024, 0, s>>>(cnt, T, sys, lev);
+  else
+    k_level_scan<64><<<rows, 64, 0, s>>>(cnt, T, sys, lev);
+}
+
 hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const StateDev &out,
                         const TreeDev &t, BuildBufs &b, double4 *pos64, float4 *pos32,
                         double theta, hipStream_t s, bool range_ready, int lazy, bool report,
@@ -2502,32 +2571,35 @@ hipError_t launch_build(const Forest &f, int leaf, const StateDev &in, const Sta
     const uint32_t nseg = 1u << lev, T = level_tiles(f, lev);
     const dim3 grid(nseg * T, ny);
     uint32_t *viol = report ? b.viol : nullptr;
-    if (f.nsys == 1) {
-      k_level_mark<false><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, b.range,
-                                                       lazy, viol, b.words, b.cnt);
-      k_level_move<false><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, lazy,
-                                                       b.words, b.cnt);
-    } else {
-      k_level_mark<true><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, b.range,
+    auto level = [&](auto forest, auto decided) {
+      constexpr bool F = decltype(forest)::value, D = decltype(decided)::value;
+      if (D)
+        k_level_split<<<dim3(nseg, ny), SPLIT_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev,
+                                                               b.range, lazy, viol, b.cnt, T);
+      k_level_mark<F, D><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, b.range,
                                                       lazy, viol, b.words, b.cnt);
-      k_level_move<true><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, lazy,
+      if (D) scan_level(b.cnt, T, lsys, lev, ny, s);
+      k_level_move<F, D><<<grid, LVL_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev, T, lazy,
                                                       b.words, b.cnt);
-    }
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (T > PAIR_TILES)
+      f.nsys > 1 ? level(yes, yes) : level(no, yes);
+    else
+      f.nsys > 1 ? level(yes, no) : level(no, no);
   }
   for (int lev = 0; lev < lev_end && !pair; ++lev) {
     const uint32_t nseg = 1u << lev;
     const uint32_t T = level_tiles(f, lev);
     k_level_split<<<dim3(nseg, ny), SPLIT_THREADS, 0, s>>>(LB, P, t, lsys, in.oid, lev,
                                                            b.range, lazy,
-                                                           report ? b.viol : nullptr);
+                                                           report ? b.viol : nullptr, nullptr, T);
     k_level_flags<<<dim3(nseg * T, ny), LVL_THREADS, 0, s>>>(LB, t, lsys, lev, T, b.flags);
     k_level_pack<<<(b.flag_words + 255) / 256, 256, 0, s>>>(b.flags, b.bits, b.flag_words);
     k_level_count<<<dim3(nseg * T, ny), LVL_THREADS, 0, s>>>(LB, t, lsys, lev, T, b.bits,
                                                              b.cnt, lazy);
-    if (T > SCAN_SMALL_T)
-      k_level_scan<1024><<<dim3(3 * nseg, ny), 1024, 0, s>>>(b.cnt, T, lsys, lev);
-    else
-      k_level_scan<64><<<dim3(3 * nseg, ny), 64, 0, s>>>(b.cnt, T, lsys, lev);
+    scan_level(b.cnt, T, lsys, lev, ny, s);
     k_level_scatter<<<dim3(nseg * T, ny), LVL_THREADS, 0, s>>>(LB, t, lsys, lev, T, b.bits,
                                                                b.cnt, lazy);
   }
