@@ -253,13 +253,11 @@ __global__ __launch_bounds__(SEL_THREADS) void k_sel_scatter(const uint64_t *__r
 // the rate of a copy), 4 M (in random order) 244 us against 375, 1,000 60 us
 // against 178; 100 M equal values 1.13 ms against 8.18.
 // The order is that of (value, index) throughout, so equal values are no
-// special case.  A bracket that misses the rank (rare) sends the call to the
-// radix passes.
+// special case.  A bracket that misses the rank (rare, see sample_at) sends the
+// call to the radix passes.
 
 // A sample is 8 keys a thread of one workgroup (16 took 30 us longer a sample
-// and saved half the candidates); the last candidates may be 16 a thread.  A
-// bracket of 4 standard deviations of a rank in the sample, and 8, holds the
-// rank but for about one call in 10^4.
+// and saved half the candidates); the last candidates may be 16 a thread.
 constexpr int SMP_THREADS = 1024, SMP_ITEMS = 8, PIVOT_ITEMS = 16;
 constexpr uint32_t SAMPLE = SMP_THREADS * SMP_ITEMS, PIVOT_MAX = SMP_THREADS * PIVOT_ITEMS;
 
@@ -412,7 +410,24 @@ __device__ void block_select_pair(const uint64_t (&k)[ITEMS], const uint64_t (&x
   __syncthreads();
 }
 
-// Brackets the wanted rank from a sample at evenly spaced positions.  FIRST:
+// Position of sample i of S among `count` elements: one from every S-th part of
+// them, at a place in it that a hash of i picks.  At the parts' starts the
+// sample would alias with data of a period: of a 128^3 lattice by its fastest
+// coordinate it saw one value, and 99 % of the ranks missed the bracket.  With
+// places that have nothing to do with the data, a rank in the sample varies no
+// more than in independent draws, so a bracket of 4 standard deviations and 8
+// misses about once in 10^4 calls.
+__device__ __forceinline__ uint64_t sample_at(uint32_t i, uint64_t count, uint32_t S) {
+  constexpr uint32_t C = 0x9E3779B1u;  // 2^32 / golden ratio, odd
+  uint32_t x = (i + 1u) * C;
+  x = (x ^ (x >> 15)) * C;
+  x = (x ^ (x >> 13)) * C;
+  x ^= x >> 16;
+  const uint64_t first = i * count / S, len = (i + 1u) * count / S - first;
+  return first + ((x * len) >> 32);  // len is at most 2^32 / S, or 1
+}
+
+// Brackets the wanted rank from a sample (sample_at).  FIRST:
 // of the elements themselves; otherwise of the candidates that the last pass
 // wrote, whose rank and count are settled first.
 template <bool FIRST>
@@ -445,7 +460,7 @@ __global__ __launch_bounds__(SMP_THREADS) void k_sel_sample(const int64_t *__res
   for (int i = 0; i < SMP_ITEMS; ++i) {
     k[i] = x[i] = 0;
     if ((uint32_t)i >= have) continue;
-    const uint64_t j = (uint64_t)(i * SMP_THREADS + threadIdx.x) * count / S;
+    const uint64_t j = sample_at(i * SMP_THREADS + threadIdx.x, count, S);
     if (FIRST) {
       const int64_t v = idx[j];
       x[i] = (uint64_t)v;
