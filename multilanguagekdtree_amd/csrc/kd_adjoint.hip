@@ -8,7 +8,9 @@
 //   f(d, m) = -m d / |d|^3,  M_n = sum m_j,  c_n = sum m_j p_j / M_n.
 // Backward through v' = v + dt a(p), p' = p + dt v' (array_kd_tree.rs:649-662):
 //   lv += dt lp;  u = dt lv;  lp += (da/dp)^T u;  lm += (da/dm)^T u.
-// k_adj_walk replays the forward walk (same decisions) and adds, per term,
+// k_adj_walk replays the forward walk (FP64: the same decisions; mixed: but
+// for nodes within an ulp or two of the opening threshold, whose |d|^2 is
+// rounded after every operation here and fused there) and adds, per term,
 //   d/dp_i (u_i . f) = -m (u_i / r^3 - 3 (d.u_i) d / r^5)  to body i,
 // its negative to the partner body (P2P) or to the node's centre of mass
 // (M2P), and -(u_i . d) / r^3 to the partner's mass or the node's mass.
@@ -249,7 +251,11 @@ __global__ __launch_bounds__(64 * S) void k_adj_walk(AdjWalk a, int lzd) {
     const auto d2 = dx * dx + dy * dy + dz * dz;
     bool ok;
     if constexpr (MIXED)
-      ok = r.size2 < d2;  // size^2 / theta^2 < d2, as the forward walk
+      // size^2 / theta^2 < d2.  (The forward walk fuses its d2, so a node that
+      // lies that close to the threshold may be taken by one and opened by the
+      // other: some of a step's 1e8 tests at 100,000 bodies, 4e-8 of a gradient
+      // whose FP32 terms are 5e-4 off.)
+      ok = r.size2 < d2;
     else
       ok = r.size2 < a.theta2 * d2;
     const uint64_t tm = actm & __builtin_amdgcn_ballot_w64(ok);
