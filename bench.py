@@ -82,12 +82,18 @@ def force_error(bodies, n, theta, leaf, precision, k=4096, seed=2024):
     return float(np.median(rel)), float(np.percentile(rel, 99)), float(rel.max())
 
 
+# body-steps that the oracle's port takes in about ten seconds
+PORT_BODY_STEPS = 100_000
+
+
 def cpu_baseline(bodies, n, steps, threads, dt):
     """The reference's own C simple_sim (Parallel/CVersion/src/kdtree.c:221-260:
     build_tree on one thread, calc_accel of every body and the kick-drift as
     OpenMP parallel-for loops), run whole for `steps` steps on a copy of the
     bodies and timed around the call; without the reference build, the
-    oracle's single-thread port over the same steps."""
+    oracle's single-thread port over the same steps, or over as many bodies
+    (the first ones) and steps as PORT_BODY_STEPS allows: 10 M would take it
+    some twenty minutes a step."""
     import oracle
     r = oracle.ref_simple_sim_timed(bodies, dt=dt, steps=steps, threads=threads)
     if r is not None:
@@ -97,6 +103,9 @@ def cpu_baseline(bodies, n, steps, threads, dt):
                 f"{threads} threads, sequential build_tree), {steps} whole step(s) of all {n} "
                 f"bodies: {sec:.2f} s")
     else:
+        n = min(n, PORT_BODY_STEPS)
+        steps = max(1, min(steps, PORT_BODY_STEPS // n))
+        bodies = {k: v[:n] for k, v in bodies.items()}
         t0 = time.perf_counter()
         oracle.simple_sim(bodies, dt=dt, steps=steps)
         sec = time.perf_counter() - t0
@@ -571,8 +580,9 @@ def main():
                                          args.leaf, dt, precs=("fp64",), err=False)
         if c1 is not None:
             extra["config1_fp64"]["cpu_reference"] = c1
-            extra["config1_fp64"]["speedup_vs_cpu"] = (
-                extra["config1_fp64"]["fp64"]["value"] / c1["value"])
+            if c1["n"] == n1:  # (the port may have taken fewer bodies)
+                extra["config1_fp64"]["speedup_vs_cpu"] = (
+                    extra["config1_fp64"]["fp64"]["value"] / c1["value"])
             log(f"[bench] cpu n={n1}: {c1}")
         del b1
 
@@ -635,7 +645,7 @@ def main():
                            "phases_ms": {k: round(res["fp64"][k], 3)
                                          for k in ("build_ms", "traverse_ms", "kick_drift_ms")}}
         out["speedup_mixed_vs_fp64"] = res["mixed"]["rate"] / res["fp64"]["rate"]
-    if cpu is not None:
+    if cpu is not None and cpu["n"] == n:
         out["speedup_vs_cpu"] = r["rate"] / cpu["value"]
     out.update(extra)
     print(json.dumps(out), flush=True)
