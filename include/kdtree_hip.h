@@ -164,7 +164,8 @@ int kd_counters(kd_ctx *ctx, int64_t out[5]);
 
 /* Launch-shape knobs of the kernels (no counterpart in the reference):
  * "leaf_predicated" 0/1 -- compute whole leaf batches with predication
- * instead of branching per body; "fp64_batched_walk" 0/1 -- accepted
+ * instead of branching per body (mixed precisions; FP64 then runs the
+ * compiler's own square root and division, with the same sums); "fp64_batched_walk" 0/1 -- accepted
  * and read back, but without effect: FP64 has one walk; "lazy_dimension" 0/1 (default
  * 1) -- let the build skip the sort and the device-wide partitions of a
  * dimension that the previous full build found could not be split at those

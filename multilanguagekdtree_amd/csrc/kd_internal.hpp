@@ -386,7 +386,13 @@ hipError_t launch_select(int64_t *idx, const double *vals, int64_t n, int64_t nv
 // shorter chains, at the price of idle lanes.  Walks in us at 64, 32, 16, 8
 // bodies, ring: 140, 133, 119, 116 at 1,000, 298, 269, 232, 223 at 8,000, 366,
 // 301, 276, 278 at 16,000, 402, 370, 370, 435 at 30,000, 483, 450, 450, 544 at
-// 60,000, 538, 552, 550 (16), 757 at 100,000.  (Sums cut in parts for several
+// 60,000, 538, 552, 550 (16), 757 at 100,000.  A uniform cube: 481, 390, 374, 384
+// at 2,000, 714, 667, 632, 588 at 5,000, 1046, 990, 891, 905 at 10,000, 1507, 1377,
+// 1398, 1477 at 20,000, 1648, 1663, 1660, 2002 at 40,000, 2012, 2078, 2399, 3071 at
+// 70,000.  A concentrated ball, whose long chains of visits are few: 606, 541,
+// 496, 556 at 2,000, 1104, 1071, 1138, 1254 at 5,000, 2047, 2083, 2136, 2309 at
+// 10,000, 3630, 3631, 3851, 4820 at 20,000, 5140, 5413, 6172, 8089 at 40,000; there
+// the rule gives up 5 to 14 % of the walk between 5,000 and 70,000.  (Sums cut in parts for several
 // wavefronts took 53 at 1,000 and 429 at 100,000, but their rounding differs,
 // and a few steps with close pairs make that visible.)
 constexpr uint32_t WALK_FEW_WAVES = 2048;  // at most so many more than ceil(n / 64)
