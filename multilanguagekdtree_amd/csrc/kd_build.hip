@@ -1495,13 +1495,18 @@ __device__ void write_internal_rec(const TreeDev &t, uint32_t h, uint32_t start,
 }
 
 // A dimension's order inside a segment, for a dimension whose list the
-// device-wide steps did not keep.  The order of equal coordinates is free:
-// a split takes the key at the median, and a run of equal keys there is put
-// in order of the original indices first.  The values sorted are a 21-bit
-// fixed-point key of the coordinate over the segment's own range with the
-// 11-bit local index below it, by a radix sort in LDS; bodies whose keys
-// collide are put in exact order afterwards, and a segment with a run of more
-// than LZ_RUN colliding keys of unequal coordinates falls back to a bitonic
+// device-wide steps did not keep.  The order of equal coordinates is free: a
+// split takes the key at the median, and one thread's insertion sort puts a run
+// of equal keys there in order of the original indices first.  But a long run
+// takes it long unless it is in that order already, so a lazy dimension that
+// the segment will probably split gets its equal coordinates by original
+// index (a million bodies in four thin layers, built after an upload / from
+// tree order: 5.7 / 5.0 ms in any order, 1.4 / 0.9 so; the network below costs
+// two values in one dimension 40 us a build, hence the guess).  The values
+// sorted are a 21-bit fixed-point key of the coordinate over the segment's own
+// range with the 11-bit local index below it, by a radix sort in LDS; bodies
+// whose keys collide are put in exact order afterwards, and a segment with a
+// run of more than LZ_RUN colliding keys out of order falls back to a bitonic
 // network on 64-bit ordered keys.
 //
 // The network is in the form whose comparators all sort upward: the merge of
@@ -1511,9 +1516,11 @@ __device__ void write_internal_rec(const TreeDev &t, uint32_t h, uint32_t start,
 // and every comparator whose upper position is one of them is skipped.  A
 // pass runs 2 consecutive stages of one merge in registers, 4 positions a
 // thread.
+template <class Before>
 struct LzWide {
   uint64_t *k;
   uint16_t *l;
+  Before before;  // of equal coordinates
   struct V {
     uint64_t k;
     uint16_t l;
@@ -1524,7 +1531,7 @@ struct LzWide {
     l[p] = v.l;
   }
   __device__ void order(V &a, V &b) const {
-    if (a.k > b.k) {
+    if (a.k > b.k || (a.k == b.k && before(b.l, a.l))) {
       const V t = a;
       a = b;
       b = t;
@@ -1724,10 +1731,11 @@ __device__ void lz_sort(const Pol &pol, uint32_t n0, int tid) {
 // A dimension's order of a segment: local indices into iz (its 2 SUB_MAX
 // bytes also hold the sort's counts before that).  buf: 8 SUB_MAX bytes of
 // LDS; shd: 2 NT / 64 doubles; flagp: two words.  zc(i): local index i's
-// coordinate.
-template <int NT, class Coord>
-__device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint32_t n0, int tid,
-                         double *shd, uint32_t *flagp) {
+// coordinate.  ties(extent): whether equal coordinates shall be in order too,
+// which before(i, j) says (i's original index is below j's).
+template <int NT, class Coord, class Before, class Ties>
+__device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, const Before &before,
+                         const Ties &ties, uint32_t n0, int tid, double *shd, uint32_t *flagp) {
   constexpr int IT = SUB_MAX / NT;
   constexpr int NW = NT / 64;
   double z[IT];
@@ -1757,7 +1765,7 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint
     lo = fmin(lo, shd[w]);
     hi = fmax(hi, shd[NW + w]);
   }
-  if (!(hi > lo)) {  // all coordinates equal (a planar system): any order
+  if (!(hi > lo)) {  // all coordinates equal (a planar system): not split, any order
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       const uint32_t i = tid + q * NT;
@@ -1788,15 +1796,16 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint
     if (i < n0) iz[i] = (uint16_t)(kp[i] & IMASK);
   }
   __syncthreads();
-  // runs of equal keys with unequal coordinates, each ordered by the thread
-  // at its start (flagp[0]: such a pair exists, flagp[1]: a long run exists)
+  // runs of equal keys that may be out of order, each ordered by the thread at
+  // its start (flagp[0]: such a pair exists, flagp[1]: a long run exists)
 #pragma unroll
   for (int q = 0; q < IT; ++q) {
     const uint32_t i = tid + q * NT;
     if (i + 1 >= n0) continue;
     const uint32_t a = kp[i], b = kp[i + 1];
     if ((a ^ b) >> (32 - LZ_KEY_BITS)) continue;
-    if (zc(a & IMASK) != zc(b & IMASK)) flagp[0] = 1;
+    if (zc(a & IMASK) != zc(b & IMASK) || (before(b & IMASK, a & IMASK) && ties(hi - lo)))
+      flagp[0] = 1;
   }
   __syncthreads();
   if (!flagp[0]) return;
@@ -1819,7 +1828,8 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint
       uint32_t y = x;
       while (y > i) {
         const uint16_t u = iz[y - 1];
-        if (zc(u) <= zv) break;
+        const double zu = zc(u);
+        if (zu < zv || (zu == zv && before(u, v))) break;
         iz[y] = u;
         --y;
       }
@@ -1838,7 +1848,7 @@ __device__ void lz_order(unsigned char *buf, uint16_t *iz, const Coord &zc, uint
       }
     }
     __syncthreads();
-    lz_sort<NT, 2>(LzWide{kz, iz}, n0, tid);
+    lz_sort<NT, 2>(LzWide<Before>{kz, iz, before}, n0, tid);
   }
 }
 
@@ -1911,6 +1921,7 @@ __global__ __launch_bounds__(SUB_THREADS)
   if (tid < 2) splits[tid] = 0;
   for (uint32_t i = tid; i < SUB_MAX; i += NT) inner[i] = 0;
   auto coord = [&](int d, uint32_t i) { return FEW ? sc[d][i] : a.P.c[d][ids[i]]; };
+  auto before = [&](uint32_t i, uint32_t j) { return a.in.oid[ids[i]] < a.in.oid[ids[j]]; };
 
   if (FEW && a.sort_all) {
     for (uint32_t i = tid; i < n0; i += NT) {
@@ -1920,7 +1931,8 @@ __global__ __launch_bounds__(SUB_THREADS)
     }
     __syncthreads();
     for (int d = 0; d < 3; ++d)
-      lz_order<NT>(smem + 10 * SUB_MAX, lst[0][d], [&](uint32_t i) { return sc[d][i]; }, n0, tid,
+      lz_order<NT>(smem + 10 * SUB_MAX, lst[0][d], [&](uint32_t i) { return sc[d][i]; },
+                   [](uint32_t, uint32_t) { return false; }, [](double) { return false; }, n0, tid,
                    shd, lzflag);
   } else {
     for (uint32_t i = tid; i < n0; i += NT) {
@@ -1948,8 +1960,16 @@ __global__ __launch_bounds__(SUB_THREADS)
                     "the sort's keys need 8 SUB_MAX bytes");
       static_assert(2 * SUB_MAX >= NT / 64 * 128 * 4, "the sort's counts fit a list");
       const double *zc = a.P.c[lz];
+      // probably split: its extent above half of what the others shrink to in
+      // n0 / leaf nodes
+      auto split = [&](double ext) {
+        const double e0 = coord(g0, lst[0][g0][n0 - 1]) - coord(g0, lst[0][g0][0]);
+        const double e1 = coord(g1, lst[0][g1][n0 - 1]) - coord(g1, lst[0][g1][0]);
+        return ext * ext * (double)(n0 / (uint32_t)leaf) > 0.25 * e0 * e1;
+      };
       lz_order<NT>(smem + 10 * SUB_MAX, lst[0][lz],
-                   [&](uint32_t i) { return FEW ? sc[lz][i] : zc[ids[i]]; }, n0, tid, shd, lzflag);
+                   [&](uint32_t i) { return FEW ? sc[lz][i] : zc[ids[i]]; }, before, split, n0,
+                   tid, shd, lzflag);
     }
   }
   __syncthreads();
