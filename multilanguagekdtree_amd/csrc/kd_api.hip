@@ -1237,7 +1237,7 @@ static int batch_step_enqueue(kd_batch *b, int lazy) {
   const int nxt = c->cur ^ 1;
   c->tree.recs = records_for(c);
   // the workgroup levels only from tree order (a step after an upload runs
-  // eagerly with the kernel-by-kernel levels)
+  // eagerly, with the device-wide kernels to the last level)
   HIP_TRY(launch_build(c->forest, c->params.leaf_size, c->st[c->cur], c->st[nxt], c->tree, c->b,
                        c->pos64, c->pos32, c->params.theta, c->stream, true, lazy, b->lazy_on,
                        c->tree_order, c->mid_levels));

@@ -305,7 +305,8 @@ hipError_t launch_shape(const TreeDev &t, const Forest &f, int leaf, hipStream_t
 // lazy build could not have skipped).
 // Each system's mid_level (a single system's from level 8 on, so that its
 // segments fill the GPU; a forest's from the first level whose segments hold
-// at most MID_MAX bodies) and the (system, segment) table of the workgroup
+// at most as many bodies as give every CU two segments over all systems, a
+// quarter of MID_MAX at least and MID_MAX at most) and the (system, segment) table of the workgroup
 // levels.
 void set_mid_levels(std::vector<SysDesc> &sys, std::vector<uint2> &tasks);
 size_t mid_tasks_max(int64_t n, int nsys);  // bound on the table's entries
