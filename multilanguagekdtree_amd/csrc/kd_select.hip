@@ -410,21 +410,22 @@ __device__ void block_select_pair(const uint64_t (&k)[ITEMS], const uint64_t (&x
   __syncthreads();
 }
 
-// Position of sample i of S among `count` elements: one from every S-th part of
-// them, at a place in it that a hash of i picks.  At the parts' starts the
-// sample would alias with data of a period: of a 128^3 lattice by its fastest
+// Position of sample i of SAMPLE among `count` elements (i itself if there are
+// no more): one from every SAMPLE-th part of them, at a place in it that a hash
+// of i picks.  At the parts' starts the sample would alias with data of a period: of a 128^3 lattice by its fastest
 // coordinate it saw one value, and 99 % of the ranks missed the bracket.  With
 // places that have nothing to do with the data, a rank in the sample varies no
 // more than in independent draws, so a bracket of 4 standard deviations and 8
 // misses about once in 10^4 calls.
-__device__ __forceinline__ uint64_t sample_at(uint32_t i, uint64_t count, uint32_t S) {
+__device__ __forceinline__ uint64_t sample_at(uint32_t i, uint64_t count) {
+  if (count <= SAMPLE) return i;
   constexpr uint32_t C = 0x9E3779B1u;  // 2^32 / golden ratio, odd
   uint32_t x = (i + 1u) * C;
   x = (x ^ (x >> 15)) * C;
   x = (x ^ (x >> 13)) * C;
   x ^= x >> 16;
-  const uint64_t first = i * count / S, len = (i + 1u) * count / S - first;
-  return first + ((x * len) >> 32);  // len is at most 2^32 / S, or 1
+  const uint64_t first = i * count / SAMPLE, len = (i + 1u) * count / SAMPLE - first;
+  return first + ((x * len) >> 32);  // len is at most 2^32 / SAMPLE
 }
 
 // Brackets the wanted rank from a sample (sample_at).  FIRST:
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(SMP_THREADS) void k_sel_sample(const int64_t *__res
   for (int i = 0; i < SMP_ITEMS; ++i) {
     k[i] = x[i] = 0;
     if ((uint32_t)i >= have) continue;
-    const uint64_t j = sample_at(i * SMP_THREADS + threadIdx.x, count, S);
+    const uint64_t j = sample_at(i * SMP_THREADS + threadIdx.x, count);
     if (FIRST) {
       const int64_t v = idx[j];
       x[i] = (uint64_t)v;
